@@ -221,11 +221,12 @@ int mfg_operator_qp_data(mfg_operator op, void *out, int32_t *n_fields);
  * reference, whose storage is fixed; the operator is the same either way).
  * MFG_T2_FOLDED: Jinv_cur (9), JxW_ref s, JxW_ref tau (6), plus JxW_ref on
  * meshes with a cell that is not affine -- the layout mfg_operator_qp_data
- * documents.  MFG_T2_GRADIENT (meshes whose cells are all affine): the
- * reference-cell gradient of the linearisation point Grad_xi u[d][f] (9) and
- * s = mu - 2 lambda ln J, 10 words per point; vmult rebuilds Jinv_cur =
- * (J_ref + Grad_xi u)^{-1} and tau = mu F F^T - s I per point from the
- * per-cell J_ref.  Default: GRADIENT on meshes whose cells are all affine,
+ * documents.  MFG_T2_GRADIENT (meshes whose cells are all affine): 10 words per
+ * point, from which vmult forms the stress products on the reference cell with
+ * the per-cell metric J_ref^{-1} J_ref^{-T}.  It holds Jinv_cur (9) and
+ * s = mu - 2 lambda ln J; mfg_operator_qp_data gives the reference-cell
+ * gradient of the linearisation point Grad_xi u[d][f] (9) and s, computed from
+ * the displacement, of which the operator keeps a copy.  Default: GRADIENT on meshes whose cells are all affine,
  * FOLDED otherwise.  Changing the storage discards the cache: call
  * mfg_operator_cache (and compute_diagonal) again. */
 #define MFG_T2_FOLDED 0

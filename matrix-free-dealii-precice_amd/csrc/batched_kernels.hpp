@@ -50,7 +50,7 @@ struct BatchInst {
   Number prm[3];  // F1: 2 lambda, rho alpha_1 (and mu for F1G); F0: kappa, c_1, rho alpha_1; heat: dt
   const Number *cell_jxw, *wq;  // F1: per-cell reference JxW (or null) and tensor weights
   const Number *cell_geo;       // heat: per-cell Jinv and det J (or null)
-  const Number *cell_jac;       // F1G: per-cell J_ref and J_ref^{-1}
+  const Number *cell_met;       // F1G: per-cell J_ref^{-1} J_ref^{-T}
 };
 
 struct BatchTask {
@@ -107,7 +107,7 @@ __device__ inline void batch_task_degree(int kind, const BatchInst<Number> &in, 
   }
   if constexpr ((KINDS & kind_bit(kSolidF1G)) != 0) {
     if (kind == kSolidF1G) {
-      QSolidT2F1G<Number> q{in.qd, in.nqp, in.prm[2], in.prm[0], in.prm[1], in.cell_jac, in.cell_jxw, in.wq};
+      QSolidT2F1G<Number> q{in.qd, in.nqp, in.prm[2], in.prm[0], in.prm[1], in.cell_met, in.cell_jxw, in.wq};
       batch_task_cells<P>(q, in, v, tk, assign, s_tab, s_tile);
     }
   }
@@ -216,7 +216,7 @@ __device__ inline auto batch_qop(const BatchInst<Number> &in) {
     return QSolidT2F1<Number>{in.qd, in.nqp, in.prm[0], in.prm[1], in.cell_jxw, in.wq};
   } else if constexpr (KIND == kSolidF1G) {
     return QSolidT2F1G<Number, kEarlyCell>{in.qd,       in.nqp,      in.prm[2], in.prm[0],
-                                           in.prm[1],   in.cell_jac, in.cell_jxw, in.wq};
+                                           in.prm[1],   in.cell_met, in.cell_jxw, in.wq};
   } else if constexpr (KIND == kSolidF0) {
     return QSolidT2F0<Number>{in.qd, in.nqp, in.prm[0], in.prm[1], in.prm[2]};
   } else {

@@ -312,25 +312,32 @@ struct QSolidT2F1 {
   }
 };
 
-// Solid, tensor2 caching, formulation 1, rebuilt per point from the
-// displacement gradient: the operator of QSolidT2F1 from 10 words per point.
-// On affine meshes J_ref and J_ref^{-1} are constant per cell, so what the
-// folded layout stores follows from Grad_xi u (the reference-cell gradient of
-// the linearisation point, 9 words) and s = mu - 2 lambda ln J (1 word) with
-// the arithmetic of the cache kernel:
-//   J_cur = J_ref + Grad_xi u,   Jinv_cur = J_cur^{-1},
-//   F = I + Grad_xi u J_ref^{-1},   tau = mu F F^T - s I,
-// and JxW_ref = det J_ref w_q.  Fields: Grad_xi u [d][f] (9), s; stored in
-// pairs of fields (below).
+// Solid, tensor2 caching, formulation 1, from 10 words per point on affine
+// meshes: the operator of QSolidT2F1 with the stress products pulled back to
+// the reference cell.  With g = Grad_xi v Jinv_cur the spatial gradient,
+// s = mu - 2 lambda ln J and tau = mu F F^T - s I,
+//   s (g + g^T) + 2 lambda tr(g) I + g tau = s g^T + 2 lambda tr(g) I + mu g F F^T,
+// and with Jinv_cur = J_ref^{-1} F^{-1} the last term, multiplied by
+// Jinv_cur^T, is mu Grad_xi v (J_ref^{-1} J_ref^{-T}): it needs neither F nor
+// tau, only the metric G = J_ref^{-1} J_ref^{-T}, constant per cell.  With
+// M = Jinv_cur Grad_xi v the submitted gradient is
+//   w [ mu Grad_xi v G + ((s M + 2 lambda tr(M) I) Jinv_cur)^T ],
+// w = JxW_ref = det J_ref w_q.  Fields: Jinv_cur[f][e] (9), s; stored in pairs
+// of fields (below).
 // kEarlyCell (the cell index is the same on every lane: one cell per
-// workgroup): the cell's J_ref, J_ref^{-1} and det J_ref are loaded into
-// SGPRs with the point data, so that their latency overlaps the gather's
-// instead of following the evaluate sweeps.
+// workgroup): the cell's G and det J_ref are loaded into SGPRs with the point
+// data, so that their latency overlaps the gather's instead of following the
+// evaluate sweeps.
 // kCartesian (with kEarlyCell; every cell's J_ref is diagonal, as on
-// axis-aligned boxes): only the 3 + 3 diagonal entries are loaded, and the
+// axis-aligned boxes): only the 3 diagonal entries of G are loaded, and the
 // products with the exact zeros off the diagonal are left out.  Every
 // rounding step of the general form survives, so the two agree bit for bit
 // (up to the sign of a zero).
+// Measured against rebuilding Jinv_cur, F and tau per point from Grad_xi u
+// (about 90 instead of 200 FP64 operations per point and no division; the
+// same 10 words): Q4 beam of 128x32x32 cells FP64 0.647 -> 0.605 ms per vmult
+// (2.76 -> 2.95 TB/s of the data held), 96x24x24 cells FP32 0.167 -> 0.161 ms,
+// Q2 37x29x23 cells FP64 44.5 -> 41.3 us.
 template <typename Number, bool kEarlyCell = false, bool kCartesian = false>
 struct QSolidT2F1G {
   static_assert(kEarlyCell || !kCartesian, "the Cartesian form loads the cell's diagonal into SGPRs");
@@ -340,14 +347,13 @@ struct QSolidT2F1G {
   const Number *qd;
   int64_t nqp;
   Number mu, two_lambda, rho_alpha;
-  const Number *cell_jac;  // per stored cell: J_ref (9), J_ref^{-1} (9)
+  const Number *cell_met;  // per stored cell: G (xx, yy, zz, xy, xz, yz)
   const Number *cell_jxw;  // det J_ref per stored cell
   const Number *wq;        // N^3 tensor-product quadrature weights
   struct Data {
-    Number gu[9], s, w;
-    const Number *jac;
-    // kCartesian: diag J_ref (3), diag J_ref^{-1} (3); else J_ref (9), J_ref^{-1} (9)
-    Number jr[kEarlyCell ? (kCartesian ? 6 : 18) : 1];
+    Number ji[9], s, w;
+    const Number *met;
+    Number g[kEarlyCell ? (kCartesian ? 3 : 6) : 1];  // the cell's G, or its diagonal
   };
   // fields are stored in pairs, qd[((f / 2) nqp + q) 2 + f % 2]: one 16-byte
   // (FP64) load brings two fields of a point
@@ -358,122 +364,65 @@ struct QSolidT2F1G {
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       const Pair x = __builtin_nontemporal_load(qp + k * nqp + q);
-      if (k < 4) {
-        d.gu[2 * k] = x.x;
-        d.gu[2 * k + 1] = x.y;
-      } else {
-        d.gu[8] = x.x;
-        d.s = x.y;
-      }
+      d.ji[2 * k] = x.x;
+      if (k < 4) d.ji[2 * k + 1] = x.y;
+      else d.s = x.y;
     }
     load_cell(d, cell, pt);
     return d;
   }
-  // the per-cell part of load(): J_ref, J_ref^{-1} and JxW_ref at point pt
+  // the per-cell part of load(): G and JxW_ref at point pt
   __device__ void load_cell(Data &d, int cell, int pt) const {
-    d.jac = cell_jac + (int64_t)cell * 18;
-    if constexpr (kCartesian) {
+    d.met = cell_met + (int64_t)cell * 6;
+    if constexpr (kEarlyCell) {
       Number jxw = as_constant(cell_jxw)[cell];
 #pragma unroll
-      for (int e = 0; e < 3; ++e) {
-        d.jr[e] = as_constant(d.jac)[4 * e];
-        d.jr[3 + e] = as_constant(d.jac)[9 + 4 * e];
-      }
-      asm volatile("" : "+s"(jxw), "+s"(d.jr[0]), "+s"(d.jr[1]), "+s"(d.jr[2]), "+s"(d.jr[3]), "+s"(d.jr[4]),
-                   "+s"(d.jr[5]));
-      d.w = jxw * wq[pt];
-    } else if constexpr (kEarlyCell) {
-      Number jxw = as_constant(cell_jxw)[cell];
-#pragma unroll
-      for (int f = 0; f < 18; ++f) d.jr[f] = as_constant(d.jac)[f];
-      // all 19 values in SGPRs here: one wait, before the first barrier
-      asm volatile(""
-                   : "+s"(jxw), "+s"(d.jr[0]), "+s"(d.jr[1]), "+s"(d.jr[2]), "+s"(d.jr[3]), "+s"(d.jr[4]),
-                     "+s"(d.jr[5]), "+s"(d.jr[6]), "+s"(d.jr[7]), "+s"(d.jr[8]), "+s"(d.jr[9]), "+s"(d.jr[10]),
-                     "+s"(d.jr[11]), "+s"(d.jr[12]), "+s"(d.jr[13]), "+s"(d.jr[14]), "+s"(d.jr[15]), "+s"(d.jr[16]),
-                     "+s"(d.jr[17]));
+      for (int f = 0; f < (kCartesian ? 3 : 6); ++f) d.g[f] = as_constant(d.met)[f];
+      // all values in SGPRs here: one wait, before the first barrier
+      if constexpr (kCartesian)
+        asm volatile("" : "+s"(jxw), "+s"(d.g[0]), "+s"(d.g[1]), "+s"(d.g[2]));
+      else
+        asm volatile("" : "+s"(jxw), "+s"(d.g[0]), "+s"(d.g[1]), "+s"(d.g[2]), "+s"(d.g[3]), "+s"(d.g[4]), "+s"(d.g[5]));
       d.w = jxw * wq[pt];
     } else {
       d.w = as_constant(cell_jxw)[cell] * wq[pt];
     }
   }
   __device__ void apply(const Data &d, Number (&val)[3], Number (&grad)[3][3]) const {
-    // J_ref (f < 9) and J_ref^{-1} (9 + f) of the cell
-    auto jr = [&](int f) -> Number {
-      if constexpr (kEarlyCell) return d.jr[f];
-      else return as_constant(d.jac)[f];
-    };
-    Number ji[9];
-    {
-      Number Jc[3][3];
-      if constexpr (kCartesian) {
+    const Number *ji = d.ji;
+    Number M[3][3];
 #pragma unroll
-        for (int f = 0; f < 9; ++f) Jc[f / 3][f % 3] = f % 4 == 0 ? d.jr[f / 4] + d.gu[f] : d.gu[f];
-      } else {
+    for (int f = 0; f < 3; ++f)
 #pragma unroll
-        for (int f = 0; f < 9; ++f) Jc[f / 3][f % 3] = jr(f) + d.gu[f];
-      }
-      const Number id =
-          Number(1) / (Jc[0][0] * (Jc[1][1] * Jc[2][2] - Jc[1][2] * Jc[2][1]) -
-                       Jc[0][1] * (Jc[1][0] * Jc[2][2] - Jc[1][2] * Jc[2][0]) + Jc[0][2] * (Jc[1][0] * Jc[2][1] - Jc[1][1] * Jc[2][0]));
-      ji[0] = (Jc[1][1] * Jc[2][2] - Jc[1][2] * Jc[2][1]) * id;
-      ji[1] = (Jc[0][2] * Jc[2][1] - Jc[0][1] * Jc[2][2]) * id;
-      ji[2] = (Jc[0][1] * Jc[1][2] - Jc[0][2] * Jc[1][1]) * id;
-      ji[3] = (Jc[1][2] * Jc[2][0] - Jc[1][0] * Jc[2][2]) * id;
-      ji[4] = (Jc[0][0] * Jc[2][2] - Jc[0][2] * Jc[2][0]) * id;
-      ji[5] = (Jc[0][2] * Jc[1][0] - Jc[0][0] * Jc[1][2]) * id;
-      ji[6] = (Jc[1][0] * Jc[2][1] - Jc[1][1] * Jc[2][0]) * id;
-      ji[7] = (Jc[0][1] * Jc[2][0] - Jc[0][0] * Jc[2][1]) * id;
-      ji[8] = (Jc[0][0] * Jc[1][1] - Jc[0][1] * Jc[1][0]) * id;
-    }
-    Number T[6];
-    {
-      Number F[3][3];
+      for (int h = 0; h < 3; ++h) M[f][h] = ji[f * 3 + 0] * grad[0][h] + ji[f * 3 + 1] * grad[1][h] + ji[f * 3 + 2] * grad[2][h];
+    const Number sw = d.w * d.s, wm = d.w * mu;
+    const Number diag = two_lambda * d.w * (M[0][0] + M[1][1] + M[2][2]);
+#pragma unroll
+    for (int f = 0; f < 3; ++f)
+#pragma unroll
+      for (int h = 0; h < 3; ++h) M[f][h] = f == h ? sw * M[f][h] + diag : sw * M[f][h];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      Number t[3];  // row c of Grad_xi v G
       if constexpr (kCartesian) {
         // the general form's sum of three products, two of them exact zeros,
         // rounds as this one product does
 #pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-          for (int e = 0; e < 3; ++e) {
-            const Number t = d.gu[a * 3 + e] * d.jr[3 + e];
-            F[a][e] = a == e ? t + Number(1) : t;
-          }
+        for (int f = 0; f < 3; ++f) t[f] = grad[c][f] * d.g[f];
       } else {
-#pragma unroll
-        for (int a = 0; a < 3; ++a)
-#pragma unroll
-          for (int e = 0; e < 3; ++e)
-            F[a][e] = d.gu[a * 3 + 0] * jr(9 + 0 * 3 + e) + d.gu[a * 3 + 1] * jr(9 + 1 * 3 + e) +
-                      d.gu[a * 3 + 2] * jr(9 + 2 * 3 + e) + (a == e ? Number(1) : Number(0));
+        auto G = [&](int f) -> Number {
+          if constexpr (kEarlyCell) return d.g[f];
+          else return as_constant(d.met)[f];
+        };
+        t[0] = grad[c][0] * G(0) + grad[c][1] * G(3) + grad[c][2] * G(4);
+        t[1] = grad[c][0] * G(3) + grad[c][1] * G(1) + grad[c][2] * G(5);
+        t[2] = grad[c][0] * G(4) + grad[c][1] * G(5) + grad[c][2] * G(2);
       }
 #pragma unroll
-      for (int s6 = 0; s6 < 6; ++s6) {
-        const int x = kSymI[s6], y = kSymJ[s6];
-        const Number b = F[x][0] * F[y][0] + F[x][1] * F[y][1] + F[x][2] * F[y][2];
-        T[s6] = d.w * (mu * b - (x == y ? d.s : Number(0)));
+      for (int f = 0; f < 3; ++f) {
+        const Number r = M[f][0] * ji[0 * 3 + c] + M[f][1] * ji[1 * 3 + c] + M[f][2] * ji[2 * 3 + c];
+        grad[c][f] = wm * t[f] + r;
       }
-    }
-    const Number sw = d.w * d.s;
-    Number g[3][3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int e = 0; e < 3; ++e) g[c][e] = grad[c][0] * ji[0 * 3 + e] + grad[c][1] * ji[1 * 3 + e] + grad[c][2] * ji[2 * 3 + e];
-    const Number tr = g[0][0] + g[1][1] + g[2][2];
-    const Number diag = two_lambda * d.w * tr;
-    const Number Tm[3][3] = {{T[0], T[3], T[4]}, {T[3], T[1], T[5]}, {T[4], T[5], T[2]}};
-    Number Pm[3][3];
-#pragma unroll
-    for (int a = 0; a < 3; ++a)
-#pragma unroll
-      for (int b = 0; b < 3; ++b)
-        Pm[a][b] = sw * (g[a][b] + g[b][a]) + (a == b ? diag : Number(0)) + g[a][0] * Tm[0][b] + g[a][1] * Tm[1][b] +
-                   g[a][2] * Tm[2][b];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-#pragma unroll
-      for (int f = 0; f < 3; ++f) grad[c][f] = Pm[c][0] * ji[f * 3 + 0] + Pm[c][1] * ji[f * 3 + 1] + Pm[c][2] * ji[f * 3 + 2];
       val[c] = rho_alpha * d.w * val[c];
     }
   }

@@ -30,7 +30,7 @@ QSolidT2F1G<Number, kEarlyCell, kCartesian> t2_gradient_op(const OperatorData &o
   const OperatorData::MaterialConstants &M = op.mats[m];
   return QSolidT2F1G<Number, kEarlyCell, kCartesian>{op.qd.as<Number>(),       op.nqp,
                                                      Number(M.mu),             Number(2.0 * M.lambda),
-                                                     Number(M.rho_alpha),      op.cell_jac.as<Number>(),
+                                                     Number(M.rho_alpha),      op.cell_met.as<Number>(),
                                                      op.cell_jxw.as<Number>(), op.wq3.as<Number>()};
 }
 
@@ -140,7 +140,7 @@ static void launch_apply(const OperatorData &op, const void *src, void *dst, int
 }
 
 template <int P, typename Number>
-static void launch_cache(OperatorData &op, const void *u, int u_fp32) {
+static void launch_cache(OperatorData &op, const void *u, int u_fp32, void *export_gradient) {
   constexpr int CPB = DefaultCPB<P, Number>::value;
   CacheArgs<Number> a;
   a.cell_nodes = op.cell_nodes.as<uint32_t>();
@@ -151,12 +151,14 @@ static void launch_cache(OperatorData &op, const void *u, int u_fp32) {
   a.colloc = op.tab_colloc.as<Number>();
   a.points = op.tab_points.as<double>();
   a.weights = op.tab_weights.as<double>();
-  a.qd = op.qd.as<Number>();
+  a.qd = export_gradient ? (Number *)export_gradient : op.qd.as<Number>();
   a.nqp = op.nqp;
   a.formulation = op.sp.formulation;
   a.caching = op.sp.caching;
+  a.affine = op.affine_ref ? 1 : 0;
   a.jxw_ref_field = op.affine_ref ? 0 : 1;
-  a.t2_gradient = op.t2_gradient() ? 1 : 0;
+  a.t2_gradient = export_gradient ? 2 : op.t2_gradient() ? 1 : 0;
+  a.u_copy = a.t2_gradient == 1 ? op.u_nodal.as<Number>() : nullptr;
   a.error = op.flag.as<int>();
   auto cells = [&](int b, int e, int m) {
     a.cell_begin = b;
@@ -205,8 +207,8 @@ static void apply_t(const OperatorData &op, const void *src, void *dst, int fix_
   MFG_DISPATCH_DEGREE(op.p, launch_apply, op, src, dst, fix_mode, stream);
 }
 template <typename Number>
-static void cache_t(OperatorData &op, const void *u, int u_fp32) {
-  MFG_DISPATCH_DEGREE(op.p, launch_cache, op, u, u_fp32);
+static void cache_t(OperatorData &op, const void *u, int u_fp32, void *export_gradient = nullptr) {
+  MFG_DISPATCH_DEGREE(op.p, launch_cache, op, u, u_fp32, export_gradient);
 }
 template <typename Number>
 static void diagonal_t(OperatorData &op) {
@@ -306,12 +308,15 @@ void OperatorData::cache(const void *u, int u_precision) {
   MFG_REQUIRE(kind == 0, MFG_ERR_ARGUMENT, "cache() applies to the solid operator");
   MFG_REQUIRE(u, MFG_ERR_ARGUMENT, "null displacement");
   fill<int>(flag.as<int>(), 1, 0, stream);
-  if (sp.caching == MFG_CACHING_SCALAR_REFERENTIAL) {  // keeps the displacement itself (mf_nh_operator.h:442-455)
+  const bool scalar_referential = sp.caching == MFG_CACHING_SCALAR_REFERENTIAL;
+  // scalar_referential keeps the displacement itself (mf_nh_operator.h:442-455),
+  // the 10-word storage for export_qp_gradient
+  if ((scalar_referential || t2_gradient()) && u_nodal.bytes != (size_t)n_dofs * elem_size()) {
+    u_nodal.allocate((size_t)n_dofs * elem_size());
+    ++buffers_version;
+  }
+  if (scalar_referential) {
     const int threads = 256, blocks = std::min(blocks_for(n_dofs, threads), 65536);
-    if (u_nodal.bytes != (size_t)n_dofs * elem_size()) {
-      u_nodal.allocate((size_t)n_dofs * elem_size());
-      ++buffers_version;
-    }
     if (precision == MFG_FP64 && u_precision == MFG_FP64)
       convert_kernel<double, double><<<blocks, threads, 0, stream>>>(u_nodal.as<double>(), (const double *)u, n_dofs);
     else if (precision == MFG_FP64)
@@ -330,6 +335,16 @@ void OperatorData::cache(const void *u, int u_precision) {
   MFG_REQUIRE(h == 0, MFG_ERR_NUMERIC, "det_F is not positive");
   ready = true;
   has_diagonal = false;
+}
+
+// Grad_xi u and s of the linearisation point (field-major pairs as the cache
+// stores its fields) from the kept displacement: the operator itself stores
+// Jinv_cur, whose inverse less J_ref would give Grad_xi u to the precision of
+// J_cur only.
+void OperatorData::export_qp_gradient(DeviceBuffer &out) {
+  out.allocate((size_t)n_fields * nqp * elem_size());
+  if (precision == MFG_FP64) cache_t<double>(*this, u_nodal.ptr, 0, out.ptr);
+  else cache_t<float>(*this, u_nodal.ptr, 1, out.ptr);
 }
 
 template <typename Number>
@@ -477,8 +492,8 @@ void OperatorData::setup_layout(const mfg_level_desc &d) {
     MFG_REQUIRE(touched[node], MFG_ERR_ARGUMENT, "node referenced by no cell");
   // affine cells: the mixed terms of the trilinear map vanish (vertex v at
   // (v & 1, v >> 1 & 1, v >> 2 & 1)); then det J_ref is one number per cell
-  std::vector<double> det_ref((size_t)n_cells), jac((size_t)n_cells * 18);
-  affine_ref = true;
+  std::vector<double> det_ref((size_t)n_cells), met((size_t)n_cells * 6);
+  affine_ref = cartesian_ref = true;
   for (int c = 0; c < n_cells; ++c) {
     const double *X = &vert[(size_t)c * 24];
     auto V = [&](int v, int e) { return X[v * 3 + e]; };
@@ -497,24 +512,25 @@ void OperatorData::setup_layout(const mfg_level_desc &d) {
     const double det = J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1]) -
                        J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) + J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0]);
     det_ref[c] = std::fabs(det);
-    // J_ref and J_ref^{-1} of an affine cell (the tensor2 gradient storage)
-    double *G = &jac[(size_t)c * 18];
-    for (int f = 0; f < 9; ++f) G[f] = J[f / 3][f % 3];
+    // the metric G = J_ref^{-1} J_ref^{-T} of an affine cell (the 10-word
+    // tensor2 storage)
     const double id = det != 0 ? 1.0 / det : 0.0;
-    G[9] = (J[1][1] * J[2][2] - J[1][2] * J[2][1]) * id;
-    G[10] = (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id;
-    G[11] = (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id;
-    G[12] = (J[1][2] * J[2][0] - J[1][0] * J[2][2]) * id;
-    G[13] = (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id;
-    G[14] = (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id;
-    G[15] = (J[1][0] * J[2][1] - J[1][1] * J[2][0]) * id;
-    G[16] = (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id;
-    G[17] = (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id;
+    const double R[3][3] = {
+        {(J[1][1] * J[2][2] - J[1][2] * J[2][1]) * id, (J[0][2] * J[2][1] - J[0][1] * J[2][2]) * id,
+         (J[0][1] * J[1][2] - J[0][2] * J[1][1]) * id},
+        {(J[1][2] * J[2][0] - J[1][0] * J[2][2]) * id, (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id,
+         (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id},
+        {(J[1][0] * J[2][1] - J[1][1] * J[2][0]) * id, (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id,
+         (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id}};
+    for (int s6 = 0; s6 < 6; ++s6) {
+      const double *a = R[kSymI[s6]], *b = R[kSymJ[s6]];
+      met[(size_t)c * 6 + s6] = a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
+    }
+    // axis-aligned cells: J_ref exactly zero off the diagonal (so J_ref^{-1} and G)
+    for (int x = 0; x < 9; ++x)
+      if (x % 4 != 0 && J[x / 3][x % 3] != 0.0) cartesian_ref = false;
   }
-  // axis-aligned cells: J_ref and J_ref^{-1} exactly zero off the diagonal
-  cartesian_ref = affine_ref;
-  for (size_t x = 0; x < jac.size() && cartesian_ref; ++x)
-    if ((x % 9) % 4 != 0 && jac[x] != 0.0) cartesian_ref = false;
+  cartesian_ref = cartesian_ref && affine_ref;
   upload(cell_nodes, map.data(), map.size(), stream);
   upload(constrained, d.constrained_dofs, (size_t)n_constrained, stream);
   host_constrained.assign(d.constrained_dofs, d.constrained_dofs + n_constrained);
@@ -540,14 +556,14 @@ void OperatorData::setup_layout(const mfg_level_desc &d) {
     if (precision == MFG_FP64) {
       upload(cell_jxw, det_ref.data(), det_ref.size(), stream);
       upload(wq3, w3.data(), w3.size(), stream);
-      if (kind == 0) upload(cell_jac, jac.data(), jac.size(), stream);
+      if (kind == 0) upload(cell_met, met.data(), met.size(), stream);
     } else {
       std::vector<float> a(det_ref.begin(), det_ref.end()), b(w3.begin(), w3.end());
       upload(cell_jxw, a.data(), a.size(), stream);
       upload(wq3, b.data(), b.size(), stream);
       if (kind == 0) {
-        std::vector<float> g(jac.begin(), jac.end());
-        upload(cell_jac, g.data(), g.size(), stream);
+        std::vector<float> g(met.begin(), met.end());
+        upload(cell_met, g.data(), g.size(), stream);
       }
     }
   }
@@ -664,7 +680,7 @@ void OperatorData::setup_solid() {
 }
 
 size_t OperatorData::memory_consumption() const {
-  return qd.bytes + cell_nodes.bytes + constrained.bytes + u_nodal.bytes + cell_jxw.bytes + wq3.bytes + cell_geo.bytes + cell_jac.bytes +
+  return qd.bytes + cell_nodes.bytes + constrained.bytes + u_nodal.bytes + cell_jxw.bytes + wq3.bytes + cell_geo.bytes + cell_met.bytes +
          gather_offsets.bytes + gather_points.bytes + gather_cmask.bytes + contrib.bytes;
 }
 
@@ -844,15 +860,19 @@ int mfg_operator_qp_data(mfg_operator op, void *out, int32_t *n_fields) {
       const int n3 = (op->p + 1) * (op->p + 1) * (op->p + 1);
       const int threads = 256;
       const int blocks = std::min(blocks_for(op->nqp * op->n_fields, threads), 65536);
+      DeviceBuffer gradient;
+      if (op->t2_gradient()) op->export_qp_gradient(gradient);
+      const DeviceBuffer &qd = gradient.ptr ? gradient : op->qd;
       if (op->precision == MFG_FP64)
         unpermute_fields_kernel<double><<<blocks, threads, 0, op->stream>>>(
-            op->qd.as<double>(), (double *)out, op->perm_dev.as<int32_t>(), op->n_cells, n3, op->n_fields,
+            qd.as<double>(), (double *)out, op->perm_dev.as<int32_t>(), op->n_cells, n3, op->n_fields,
             op->kind == 0 && op->sp.caching == MFG_CACHING_TENSOR2 && op->sp.formulation == 1 ? 1 : 0);
       else
         unpermute_fields_kernel<float><<<blocks, threads, 0, op->stream>>>(
-            op->qd.as<float>(), (float *)out, op->perm_dev.as<int32_t>(), op->n_cells, n3, op->n_fields,
+            qd.as<float>(), (float *)out, op->perm_dev.as<int32_t>(), op->n_cells, n3, op->n_fields,
             op->kind == 0 && op->sp.caching == MFG_CACHING_TENSOR2 && op->sp.formulation == 1 ? 1 : 0);
       MFG_HIP(hipGetLastError());
+      if (gradient.ptr) MFG_HIP(hipStreamSynchronize(op->stream));  // before its memory is freed
     }
   });
 }

@@ -36,14 +36,14 @@ struct OperatorData {
   DeviceBuffer tab_shape, tab_colloc, tab_sq, tab_points, tab_weights;
   DeviceBuffer qd;           // quadrature cache, field-major SoA
   DeviceBuffer diag, inv_diag;
-  DeviceBuffer u_nodal;      // scalar_referential caching: the linearisation point
+  DeviceBuffer u_nodal;      // the linearisation point (scalar_referential caching and the 10-word storage)
   // reference-frame JxW per cell: when every cell's trilinear map is affine,
   // JxW_ref = cell_jxw[stored cell] * wq3[point] (tensor2, formulation 1)
   bool affine_ref = false;
   DeviceBuffer cell_jxw, wq3;
   DeviceBuffer cell_geo;  // heat on affine cells: Jinv (9), det J per stored cell
-  DeviceBuffer cell_jac;  // solid on affine cells: J_ref (9), J_ref^{-1} (9) per stored cell
-  bool cartesian_ref = false;  // affine, and every cell's J_ref (so J_ref^{-1}) is diagonal
+  DeviceBuffer cell_met;  // solid on affine cells: J_ref^{-1} J_ref^{-T} (6, symmetric) per stored cell
+  bool cartesian_ref = false;  // affine, and every cell's J_ref is diagonal
   int t2_storage = MFG_T2_FOLDED;  // tensor2 formulation-1 point storage (MFG_T2_*)
   bool t2_gradient() const { return kind == 0 && sp.caching == MFG_CACHING_TENSOR2 && sp.formulation == 1 && t2_storage == MFG_T2_GRADIENT; }
   DeviceBuffer flag;         // int error flag
@@ -91,6 +91,7 @@ struct OperatorData {
   void setup_solid();
   void setup_heat(const mfg_level_desc &d, const double *coef);
   void cache(const void *u, int u_precision);
+  void export_qp_gradient(DeviceBuffer &out);
   // dst (+)= A src on `on` (the operator's stream when null)
   void apply(const void *src, void *dst, bool add, hipStream_t on = nullptr) const;
   void compute_diagonal();

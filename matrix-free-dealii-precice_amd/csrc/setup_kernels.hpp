@@ -21,8 +21,13 @@ struct CacheArgs {
   Number mu, lambda;
   int formulation;
   int caching;  // MFG_CACHING_*
+  int affine;          // every cell's trilinear map is affine
   int jxw_ref_field;  // tensor2 formulation 1: store JxW_ref as field 16 (not supplied per cell)
-  int t2_gradient;    // tensor2 formulation 1: store Grad_xi u and s (10 fields) instead
+  // tensor2 formulation 1, MFG_T2_GRADIENT: 1 stores the operator's 10 fields
+  // (Jinv_cur, s), and the displacement itself to u_copy; 2 stores Grad_xi u
+  // and s (what mfg_operator_qp_data exports)
+  int t2_gradient;
+  Number *u_copy;  // 3 per node, with t2_gradient 1
   int *error;   // set to 1 if det F <= 0 anywhere
 };
 
@@ -67,6 +72,19 @@ __device__ inline void trilinear_jacobian(const double *v, double x0, double x1,
   }
 }
 
+// The same on an affine cell, where it is constant: the edge differences, as
+// the host forms the per-cell tables from them.  The general sum over the
+// vertices cancels from the size of the coordinates down to that of the cell
+// (1e-14 of the Jacobian on the 32-cell beam, 4 long); the differences do not.
+__device__ inline void affine_jacobian(const double *v, double (&J)[3][3]) {
+#pragma unroll
+  for (int e = 0; e < 3; ++e) {
+    J[e][0] = v[3 + e] - v[e];
+    J[e][1] = v[6 + e] - v[e];
+    J[e][2] = v[12 + e] - v[e];
+  }
+}
+
 template <int P, int CPB, typename Number>
 __global__ void __launch_bounds__((block_threads<P, CPB>())) cache_solid(CacheArgs<Number> a) {
   constexpr int N = P + 1, N3 = N * N * N;
@@ -91,7 +109,8 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) cache_solid(CacheAr
   const int cell = a.cell_begin + blockIdx.x * CPB + lc;
   const bool active = !pad && cell < a.cell_end;
   const int64_t qidx = active ? (int64_t)cell * N3 + pt : 0;
-  const int64_t node = active ? (int64_t)(a.cell_nodes[qidx] & kNodeMaskDev) : 0;
+  const uint32_t entry = active ? a.cell_nodes[qidx] : 0u;
+  const int64_t node = (int64_t)(entry & kNodeMaskDev);
   Number u[3];
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
@@ -100,13 +119,16 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) cache_solid(CacheAr
     else if (a.u_fp32) u[c] = (Number)((const float *)a.u)[node * 3 + c];
     else u[c] = (Number)((const double *)a.u)[node * 3 + c];
   }
+  // one (cell, point) of every node carries the first-touch bit
+  if (a.u_copy && active && (entry >> 31)) store_node<Number, 3>(a.u_copy + node * 3, u);
   __syncthreads();
   Number gr[3][3];
   evaluate_g<N, 3, Number>(T, s_shape, s_colloc, u, gr);
   if (!active) return;
 
   double Jr[3][3], Jri[3][3];
-  trilinear_jacobian(a.vertices + (int64_t)cell * 24, a.points[T.i], a.points[T.j], a.points[T.k], Jr);
+  if (a.affine) affine_jacobian(a.vertices + (int64_t)cell * 24, Jr);
+  else trilinear_jacobian(a.vertices + (int64_t)cell * 24, a.points[T.i], a.points[T.j], a.points[T.k], Jr);
   {
     const double id = 1.0 / (Jr[0][0] * (Jr[1][1] * Jr[2][2] - Jr[1][2] * Jr[2][1]) -
                              Jr[0][1] * (Jr[1][0] * Jr[2][2] - Jr[1][2] * Jr[2][0]) +
@@ -139,10 +161,21 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) cache_solid(CacheAr
   const int64_t n = a.nqp;
   const double wq = a.weights[T.i] * a.weights[T.j] * a.weights[T.k];
   const Number scalar = a.mu - Number(2) * a.lambda * log(J);
-  if (a.t2_gradient) {  // the 10-word tensor2 storage: Grad_xi u [d][f], s, in pairs of fields
+  if (a.t2_gradient) {  // 9 words and s, in pairs of fields
+    Number f10[10];
+    if (a.t2_gradient == 1) {
+      inv3(Jc, Jci);
 #pragma unroll
-    for (int f = 0; f < 9; ++f) a.qd[((f >> 1) * n + qidx) * 2 + (f & 1)] = gr[f / 3][f % 3];
-    a.qd[(4 * n + qidx) * 2 + 1] = scalar;
+      for (int f = 0; f < 9; ++f) f10[f] = Jci[f / 3][f % 3];
+    } else {
+#pragma unroll
+      for (int f = 0; f < 9; ++f) f10[f] = gr[f / 3][f % 3];
+    }
+    f10[9] = scalar;
+    typedef Number Pair __attribute__((ext_vector_type(2)));
+    Pair *qp = reinterpret_cast<Pair *>(a.qd);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) qp[k * n + qidx] = Pair{f10[2 * k], f10[2 * k + 1]};
     return;
   }
   if (a.caching == MFG_CACHING_SCALAR_REFERENTIAL || a.caching == MFG_CACHING_TENSOR4_NS) {

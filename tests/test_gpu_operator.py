@@ -522,3 +522,27 @@ def test_gradient_point_storage_errors(cuda):
             mfgpu.NeoHookOperator(gm, O.MU, O.NU, O.RHO, O.ALPHA1, **kw).set_point_storage(mfgpu.T2_GRADIENT)
     with pytest.raises(mfgpu.MfgError):
         mfgpu.LaplaceOperator(mfgpu.BoxMesh(lo, hi, n, p, 1, 63, 1), 0.1).set_point_storage(mfgpu.T2_GRADIENT)
+
+
+@pytest.mark.parametrize("precision,amp", [(mfgpu.FP64, 1e-9), (mfgpu.FP64, 1e-2), (mfgpu.FP32, 1e-5)])
+@pytest.mark.parametrize("p", [1, 4])
+def test_gradient_point_storage_export(cuda, p, precision, amp):
+    """qp_data of the 10-word storage is Grad_xi u to the precision of u itself
+    (not of J_ref + Grad_xi u): for a linear displacement u = A X it is A J_ref
+    at every point, and s = mu - 2 lambda ln det(I + A)."""
+    print(f"10-word export p={p} precision={precision} amp={amp}", flush=True)
+    gm = mfgpu.BoxMesh([0, 0, 0], [1.0, 0.6, 0.4], [3, 2, 2], p, 3, 1, 7)
+    A = amp * np.array([[1.0, 0.3, -0.2], [0.4, -0.7, 0.1], [0.2, 0.5, 0.6]])
+    u = (gm.node_coords() @ A.T).ravel()
+    go = mfgpu.NeoHookOperator(gm, O.MU, O.NU, O.RHO, O.ALPHA1, precision=precision)
+    go.cache(dev(u, go.dtype))
+    g = go.qp_data().double().cpu().numpy()
+    eps = np.finfo(np.float64 if precision == mfgpu.FP64 else np.float32).eps
+    ref = (A @ np.diag([1.0 / 3, 0.3, 0.2])).reshape(9, 1)
+    # three sweeps of p + 1 terms and a derivative whose rows sum to 2 p^2 at most, on values up to |u|
+    tol = 4 * (p + 1) * 2 * p * p * eps * np.abs(u).max()
+    assert np.abs(g[:9] - ref).max() <= tol
+    lam = 2 * O.MU * O.NU / (1 - 2 * O.NU)
+    s = O.MU - 2 * lam * np.log(np.linalg.det(np.eye(3) + A))
+    # ln det F to the rounding of F and of the gradient over a cell
+    assert np.abs(g[9] - s).max() <= 2 * lam * (16 * eps + 9 * tol / 0.2) + 4 * eps * O.MU
