@@ -49,7 +49,7 @@ struct BatchInst {
   int id;  // batch-wide instance number (active mask)
   Number prm[3];  // F1: 2 lambda, rho alpha_1 (and mu for F1G); F0: kappa, c_1, rho alpha_1; heat: dt
   const Number *cell_jxw, *wq;  // F1: per-cell reference JxW (or null) and tensor weights
-  const Number *cell_geo;       // heat: per-cell Jinv and det J (or null)
+  const Number *cell_geo;       // heat: per-cell Jinv Jinv^T and det J (or null)
   const Number *cell_met;       // F1G: per-cell J_ref^{-1} J_ref^{-T}
 };
 
@@ -119,8 +119,13 @@ __device__ inline void batch_task_degree(int kind, const BatchInst<Number> &in, 
   }
   if constexpr ((KINDS & kind_bit(kHeat)) != 0) {
     if (kind == kHeat) {
-      QHeat<Number> q{in.qd, in.nqp, in.prm[0], in.cell_geo, in.wq};
-      batch_task_cells<P>(q, in, v, tk, assign, s_tab, s_tile);
+      if (in.cell_geo) {
+        QHeat<Number, true> q{in.qd, in.nqp, in.prm[0], in.cell_geo, in.wq};
+        batch_task_cells<P>(q, in, v, tk, assign, s_tab, s_tile);
+      } else {
+        QHeat<Number, false> q{in.qd, in.nqp, in.prm[0], nullptr, nullptr};
+        batch_task_cells<P>(q, in, v, tk, assign, s_tab, s_tile);
+      }
     }
   }
 }
@@ -210,7 +215,7 @@ __global__ void __launch_bounds__(kBatchThreads, WAVES) batched_apply_kernel(Bat
 // batched_gather_kernel sums every node's contributions in colour order, the
 // order in which the colour launches add them, so the result is the
 // per-instance result bit for bit.
-template <int KIND, bool kEarlyCell, typename Number>
+template <int KIND, bool kEarlyCell, bool kAffineHeat, typename Number>
 __device__ inline auto batch_qop(const BatchInst<Number> &in) {
   if constexpr (KIND == kSolidF1) {
     return QSolidT2F1<Number>{in.qd, in.nqp, in.prm[0], in.prm[1], in.cell_jxw, in.wq};
@@ -220,7 +225,7 @@ __device__ inline auto batch_qop(const BatchInst<Number> &in) {
   } else if constexpr (KIND == kSolidF0) {
     return QSolidT2F0<Number>{in.qd, in.nqp, in.prm[0], in.prm[1], in.prm[2]};
   } else {
-    return QHeat<Number>{in.qd, in.nqp, in.prm[0], in.cell_geo, in.wq};
+    return QHeat<Number, kAffineHeat>{in.qd, in.nqp, in.prm[0], in.cell_geo, in.wq};
   }
 }
 
@@ -240,9 +245,12 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) batched_cells_kerne
   const BatchTask tk = a.tasks[xcd_remap(blockIdx.x, gridDim.x)];
   const BatchInst<Number> in = a.inst[tk.inst];
   const BatchVecs<Number> v = a.vecs[tk.inst];
-  const auto q = batch_qop<KIND, CPB == 1>(in);
-  cell_group<P, Number, decltype(q), true, kSpare>(q, in.cell_nodes, v.src, v.dst, tk.cell_begin, tk.cell_end, CPB,
-                                                   1, in.shape, in.colloc, s_shape, s_colloc, s_tile);
+  auto group = [&](auto q) {
+    cell_group<P, Number, decltype(q), true, kSpare>(q, in.cell_nodes, v.src, v.dst, tk.cell_begin, tk.cell_end, CPB,
+                                                     1, in.shape, in.colloc, s_shape, s_colloc, s_tile);
+  };
+  if (KIND == kHeat && !in.cell_geo) group(batch_qop<KIND, CPB == 1, false>(in));
+  else group(batch_qop<KIND, CPB == 1, true>(in));
 }
 
 template <typename Number>

@@ -228,10 +228,24 @@ __device__ inline ConstantPtr<Number> as_constant(const Number *p) {
 }
 
 // ------------------------------------------------------ quadrature ops ---
-// Each op provides load(qidx, cell, pt) -> Data (point qidx = cell N^3 + pt
-// of the stored cell order) and apply(Data, val, grad), turning values and
-// reference gradients at a point into submitted value and reference gradient
-// already multiplied by JxW.
+// Each op provides
+//   load_cell(cell) -> Cell          what is constant on a stored cell,
+//   load(qb, lo, pt) -> Data         the fields of point qb + lo = cell N^3 + pt
+//                                    (qb the same on every lane: the loads take
+//                                    a scalar base and a 32-bit lane offset),
+//   apply_grad(Cell, Data, grad)     reference gradients at the point -> the
+//                                    submitted reference gradients, with JxW,
+//   value_scale(Cell, Data)          the factor of the submitted values
+// (apply: both).
+struct NoCell {};
+template <class QOp, typename Number, int NC>
+__device__ inline void apply_qop(const QOp &qop, const typename QOp::Cell &cd, const typename QOp::Data &d,
+                                 Number (&val)[NC], Number (&grad)[NC][3]) {
+  qop.apply_grad(cd, d, grad);
+  const Number s = qop.value_scale(cd, d);
+#pragma unroll
+  for (int c = 0; c < NC; ++c) val[c] = s * val[c];
+}
 
 // symmetric index pairs xx, yy, zz, xy, xz, yz
 constexpr int kSymI[6] = {0, 1, 2, 0, 0, 1}, kSymJ[6] = {0, 1, 2, 1, 2, 2};
@@ -261,19 +275,24 @@ struct QSolidT2F1 {
   Number two_lambda, rho_alpha;
   const Number *cell_jxw;  // det J_ref per stored cell, or null: field 16 holds JxW_ref
   const Number *wq;        // N^3 tensor-product quadrature weights (with cell_jxw)
-  struct Data {
-    Number ji[9], s, T[6], w;
+  struct Cell {
+    Number jxw;
   };
+  struct Data {
+    Number ji[9], s, T[6], w;  // w: the point's quadrature weight (with cell_jxw) or JxW_ref
+  };
+  __device__ Cell load_cell(int cell) const { return Cell{cell_jxw ? as_constant(cell_jxw)[cell] : Number(1)}; }
+  __device__ Number jxw(const Cell &cd, const Data &d) const { return cd.jxw * d.w; }
   // fields 0..15 are stored in pairs, qd[((f / 2) nqp + q) 2 + f % 2], field
   // 16 plainly after them: 8 16-byte (FP64) loads bring a point's 16 words
   typedef Number Pair __attribute__((ext_vector_type(2)));
-  __device__ Data load(int64_t q, int cell, int pt) const {
+  __device__ Data load(int64_t qb, uint32_t lo, int pt) const {
     Data d;
     Number f16[16];
     const Pair *qp = reinterpret_cast<const Pair *>(qd);
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
-      const Pair x = __builtin_nontemporal_load(qp + k * nqp + q);
+      const Pair x = __builtin_nontemporal_load(qp + k * nqp + qb + lo);
       f16[2 * k] = x.x;
       f16[2 * k + 1] = x.y;
     }
@@ -282,17 +301,19 @@ struct QSolidT2F1 {
     d.s = f16[9];
 #pragma unroll
     for (int f = 0; f < 6; ++f) d.T[f] = f16[10 + f];
-    d.w = cell_jxw ? as_constant(cell_jxw)[cell] * wq[pt] : stream_load(qd + 16 * nqp + q);
+    d.w = cell_jxw ? wq[pt] : stream_load(qd + 16 * nqp + qb + lo);
     return d;
   }
-  __device__ void apply(const Data &d, Number (&val)[3], Number (&grad)[3][3]) const {
+  __device__ Number value_scale(const Cell &cd, const Data &d) const { return rho_alpha * jxw(cd, d); }
+  __device__ void apply_grad(const Cell &cd, const Data &d, Number (&grad)[3][3]) const {
+    const Number w = jxw(cd, d);
     Number g[3][3];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
       for (int e = 0; e < 3; ++e) g[c][e] = grad[c][0] * d.ji[0 * 3 + e] + grad[c][1] * d.ji[1 * 3 + e] + grad[c][2] * d.ji[2 * 3 + e];
     const Number tr = g[0][0] + g[1][1] + g[2][2];
-    const Number diag = two_lambda * d.w * tr;
+    const Number diag = two_lambda * w * tr;
     // T symmetric: T[0]=xx T[1]=yy T[2]=zz T[3]=xy T[4]=xz T[5]=yz
     const Number Tm[3][3] = {{d.T[0], d.T[3], d.T[4]}, {d.T[3], d.T[1], d.T[5]}, {d.T[4], d.T[5], d.T[2]}};
     Number Pm[3][3];
@@ -303,12 +324,10 @@ struct QSolidT2F1 {
         Pm[a][b] = d.s * (g[a][b] + g[b][a]) + (a == b ? diag : Number(0)) + g[a][0] * Tm[0][b] +
                    g[a][1] * Tm[1][b] + g[a][2] * Tm[2][b];
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
+    for (int c = 0; c < 3; ++c)
 #pragma unroll
       for (int f = 0; f < 3; ++f)
         grad[c][f] = Pm[c][0] * d.ji[f * 3 + 0] + Pm[c][1] * d.ji[f * 3 + 1] + Pm[c][2] * d.ji[f * 3 + 2];
-      val[c] = rho_alpha * d.w * val[c];
-    }
   }
 };
 
@@ -328,11 +347,10 @@ struct QSolidT2F1 {
 // workgroup): the cell's G and det J_ref are loaded into SGPRs with the point
 // data, so that their latency overlaps the gather's instead of following the
 // evaluate sweeps.
-// kCartesian (with kEarlyCell; every cell's J_ref is diagonal, as on
-// axis-aligned boxes): only the 3 diagonal entries of G are loaded, and the
-// products with the exact zeros off the diagonal are left out.  Every
-// rounding step of the general form survives, so the two agree bit for bit
-// (up to the sign of a zero).
+// kCartesian (every cell's J_ref is diagonal, as on axis-aligned boxes): only
+// the 3 diagonal entries of G are loaded, and the products with the exact
+// zeros off the diagonal are left out.  Every rounding step of the general
+// form survives, so the two agree bit for bit (up to the sign of a zero).
 // Measured against rebuilding Jinv_cur, F and tau per point from Grad_xi u
 // (about 90 instead of 200 FP64 operations per point and no division; the
 // same 10 words): Q4 beam of 128x32x32 cells FP64 0.647 -> 0.605 ms per vmult
@@ -340,7 +358,6 @@ struct QSolidT2F1 {
 // Q2 37x29x23 cells FP64 44.5 -> 41.3 us.
 template <typename Number, bool kEarlyCell = false, bool kCartesian = false>
 struct QSolidT2F1G {
-  static_assert(kEarlyCell || !kCartesian, "the Cartesian form loads the cell's diagonal into SGPRs");
   static constexpr int NC = 3;
   static constexpr int kFields = 10;
   static constexpr bool kNodalField = false;
@@ -350,53 +367,56 @@ struct QSolidT2F1G {
   const Number *cell_met;  // per stored cell: G (xx, yy, zz, xy, xz, yz)
   const Number *cell_jxw;  // det J_ref per stored cell
   const Number *wq;        // N^3 tensor-product quadrature weights
-  struct Data {
-    Number ji[9], s, w;
-    const Number *met;
-    Number g[kEarlyCell ? (kCartesian ? 3 : 6) : 1];  // the cell's G, or its diagonal
+  struct Cell {
+    Number jxw, g[kCartesian ? 3 : 6];  // det J_ref; G or its diagonal
   };
+  struct Data {
+    Number ji[9], s, w;  // w: the point's quadrature weight
+  };
+  __device__ Cell load_cell(int cell) const {
+    Cell cd;
+    const ConstantPtr<Number> m = as_constant(cell_met) + (int64_t)cell * 6;
+    cd.jxw = as_constant(cell_jxw)[cell];
+#pragma unroll
+    for (int f = 0; f < (kCartesian ? 3 : 6); ++f) cd.g[f] = m[f];
+    if constexpr (kEarlyCell) {
+      // all values in SGPRs here: one wait, before the first barrier
+      if constexpr (kCartesian)
+        asm volatile("" : "+s"(cd.jxw), "+s"(cd.g[0]), "+s"(cd.g[1]), "+s"(cd.g[2]));
+      else
+        asm volatile(""
+                     : "+s"(cd.jxw), "+s"(cd.g[0]), "+s"(cd.g[1]), "+s"(cd.g[2]), "+s"(cd.g[3]), "+s"(cd.g[4]),
+                       "+s"(cd.g[5]));
+    }
+    return cd;
+  }
   // fields are stored in pairs, qd[((f / 2) nqp + q) 2 + f % 2]: one 16-byte
   // (FP64) load brings two fields of a point
   typedef Number Pair __attribute__((ext_vector_type(2)));
-  __device__ Data load(int64_t q, int cell, int pt) const {
+  __device__ Data load(int64_t qb, uint32_t lo, int pt) const {
     Data d;
     const Pair *qp = reinterpret_cast<const Pair *>(qd);
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
-      const Pair x = __builtin_nontemporal_load(qp + k * nqp + q);
+      const Pair x = __builtin_nontemporal_load(qp + k * nqp + qb + lo);
       d.ji[2 * k] = x.x;
       if (k < 4) d.ji[2 * k + 1] = x.y;
       else d.s = x.y;
     }
-    load_cell(d, cell, pt);
+    d.w = wq[pt];
     return d;
   }
-  // the per-cell part of load(): G and JxW_ref at point pt
-  __device__ void load_cell(Data &d, int cell, int pt) const {
-    d.met = cell_met + (int64_t)cell * 6;
-    if constexpr (kEarlyCell) {
-      Number jxw = as_constant(cell_jxw)[cell];
-#pragma unroll
-      for (int f = 0; f < (kCartesian ? 3 : 6); ++f) d.g[f] = as_constant(d.met)[f];
-      // all values in SGPRs here: one wait, before the first barrier
-      if constexpr (kCartesian)
-        asm volatile("" : "+s"(jxw), "+s"(d.g[0]), "+s"(d.g[1]), "+s"(d.g[2]));
-      else
-        asm volatile("" : "+s"(jxw), "+s"(d.g[0]), "+s"(d.g[1]), "+s"(d.g[2]), "+s"(d.g[3]), "+s"(d.g[4]), "+s"(d.g[5]));
-      d.w = jxw * wq[pt];
-    } else {
-      d.w = as_constant(cell_jxw)[cell] * wq[pt];
-    }
-  }
-  __device__ void apply(const Data &d, Number (&val)[3], Number (&grad)[3][3]) const {
+  __device__ Number value_scale(const Cell &cd, const Data &d) const { return rho_alpha * (cd.jxw * d.w); }
+  __device__ void apply_grad(const Cell &cd, const Data &d, Number (&grad)[3][3]) const {
+    const Number w = cd.jxw * d.w;
     const Number *ji = d.ji;
     Number M[3][3];
 #pragma unroll
     for (int f = 0; f < 3; ++f)
 #pragma unroll
       for (int h = 0; h < 3; ++h) M[f][h] = ji[f * 3 + 0] * grad[0][h] + ji[f * 3 + 1] * grad[1][h] + ji[f * 3 + 2] * grad[2][h];
-    const Number sw = d.w * d.s, wm = d.w * mu;
-    const Number diag = two_lambda * d.w * (M[0][0] + M[1][1] + M[2][2]);
+    const Number sw = w * d.s, wm = w * mu;
+    const Number diag = two_lambda * w * (M[0][0] + M[1][1] + M[2][2]);
 #pragma unroll
     for (int f = 0; f < 3; ++f)
 #pragma unroll
@@ -408,22 +428,17 @@ struct QSolidT2F1G {
         // the general form's sum of three products, two of them exact zeros,
         // rounds as this one product does
 #pragma unroll
-        for (int f = 0; f < 3; ++f) t[f] = grad[c][f] * d.g[f];
+        for (int f = 0; f < 3; ++f) t[f] = grad[c][f] * cd.g[f];
       } else {
-        auto G = [&](int f) -> Number {
-          if constexpr (kEarlyCell) return d.g[f];
-          else return as_constant(d.met)[f];
-        };
-        t[0] = grad[c][0] * G(0) + grad[c][1] * G(3) + grad[c][2] * G(4);
-        t[1] = grad[c][0] * G(3) + grad[c][1] * G(1) + grad[c][2] * G(5);
-        t[2] = grad[c][0] * G(4) + grad[c][1] * G(5) + grad[c][2] * G(2);
+        t[0] = grad[c][0] * cd.g[0] + grad[c][1] * cd.g[3] + grad[c][2] * cd.g[4];
+        t[1] = grad[c][0] * cd.g[3] + grad[c][1] * cd.g[1] + grad[c][2] * cd.g[5];
+        t[2] = grad[c][0] * cd.g[4] + grad[c][1] * cd.g[5] + grad[c][2] * cd.g[2];
       }
 #pragma unroll
       for (int f = 0; f < 3; ++f) {
         const Number r = M[f][0] * ji[0 * 3 + c] + M[f][1] * ji[1 * 3 + c] + M[f][2] * ji[2 * 3 + c];
         grad[c][f] = wm * t[f] + r;
       }
-      val[c] = rho_alpha * d.w * val[c];
     }
   }
 };
@@ -438,28 +453,36 @@ struct QSolidT2F0 {
   const Number *qd;
   int64_t nqp;
   Number kappa, c_1, rho_alpha;
+  using Cell = NoCell;
+  __device__ Cell load_cell(int) const { return Cell{}; }
   struct Data {
     Number ji[9], jxw, jm13, F[9];
   };
-  __device__ Data load(int64_t q, int cell, int pt) const {
+  __device__ Data load(int64_t qb, uint32_t lo, int) const {
     Data d;
 #pragma unroll
-    for (int f = 0; f < 9; ++f) d.ji[f] = stream_load(qd + f * nqp + q);
-    d.jxw = stream_load(qd + 9 * nqp + q);
-    d.jm13 = stream_load(qd + 10 * nqp + q);
+    for (int f = 0; f < 9; ++f) d.ji[f] = stream_load(qd + f * nqp + qb + lo);
+    d.jxw = stream_load(qd + 9 * nqp + qb + lo);
+    d.jm13 = stream_load(qd + 10 * nqp + qb + lo);
 #pragma unroll
-    for (int f = 0; f < 9; ++f) d.F[f] = stream_load(qd + (11 + f) * nqp + q);
+    for (int f = 0; f < 9; ++f) d.F[f] = stream_load(qd + (11 + f) * nqp + qb + lo);
     return d;
   }
-  __device__ void apply(const Data &d, Number (&val)[3], Number (&grad)[3][3]) const {
+  __device__ static Number det(const Number *F) {
+    return F[0] * (F[4] * F[8] - F[5] * F[7]) - F[1] * (F[3] * F[8] - F[5] * F[6]) + F[2] * (F[3] * F[7] - F[4] * F[6]);
+  }
+  __device__ Number value_scale(const Cell &, const Data &d) const {
+    const Number inv_det = Number(1) / det(d.F);
+    return d.jxw * rho_alpha * inv_det;
+  }
+  __device__ void apply_grad(const Cell &, const Data &d, Number (&grad)[3][3]) const {
     Number g[3][3];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
 #pragma unroll
       for (int e = 0; e < 3; ++e) g[c][e] = grad[c][0] * d.ji[0 * 3 + e] + grad[c][1] * d.ji[1 * 3 + e] + grad[c][2] * d.ji[2 * 3 + e];
     const Number *F = d.F;
-    const Number det_F = F[0] * (F[4] * F[8] - F[5] * F[7]) - F[1] * (F[3] * F[8] - F[5] * F[6]) +
-                         F[2] * (F[3] * F[7] - F[4] * F[6]);
+    const Number det_F = det(F);
     Number Fb[9];
 #pragma unroll
     for (int a = 0; a < 9; ++a) Fb[a] = F[a] * d.jm13;
@@ -506,56 +529,74 @@ struct QSolidT2F0 {
         Pm[a][b] = (jc + geo) * inv_det;
       }
 #pragma unroll
-    for (int c = 0; c < 3; ++c) {
+    for (int c = 0; c < 3; ++c)
 #pragma unroll
       for (int f = 0; f < 3; ++f)
         grad[c][f] = d.jxw * (Pm[c][0] * d.ji[f * 3 + 0] + Pm[c][1] * d.ji[f * 3 + 1] + Pm[c][2] * d.ji[f * 3 + 2]);
-      val[c] = d.jxw * rho_alpha * inv_det * val[c];
-    }
   }
 };
 
-// Heat: value v, gradient c*dt*grad v (heat_transfer.h:242-248).
-// Fields: Jinv (9), JxW, c per point; or, when every cell is affine (the
-// affine-cell geometry of MatrixFree), Jinv and det J once per cell
-// (cell_geo, 10 words), JxW = det J * wq[point], and c the only field.
-template <typename Number>
+// Heat: value v, gradient c*dt*grad v (heat_transfer.h:242-248).  On the
+// reference cell the gradient term is c dt JxW G Grad_xi v with the metric
+// G = Jinv Jinv^T (symmetric).  Fields: Jinv (9), JxW, c per point; or, when
+// every cell is affine (the affine-cell geometry of MatrixFree), G and det J
+// once per cell (cell_geo, 7 words), JxW = det J * wq[point], and c the only
+// field.
+template <typename Number, bool kAffine>
 struct QHeat {
   static constexpr int NC = 1;
-  static constexpr int kFields = 11;  // 1 with cell_geo
+  static constexpr int kFields = kAffine ? 1 : 11;
   static constexpr bool kNodalField = false;
   const Number *qd;
   int64_t nqp;
   Number dt;
-  const Number *cell_geo;  // per stored cell: Jinv (9), det J; or null
-  const Number *wq;        // N^3 tensor-product quadrature weights (with cell_geo)
-  struct Data {
-    Number ji[9], jxw, c;
+  const Number *cell_geo;  // kAffine, per stored cell: G (xx, yy, zz, xy, xz, yz), det J
+  const Number *wq;        // N^3 tensor-product quadrature weights (kAffine)
+  struct Cell {
+    Number g[6], det;
   };
-  __device__ Data load(int64_t q, int cell, int pt) const {
-    Data d;
-    if (cell_geo) {
-      const ConstantPtr<Number> g = as_constant(cell_geo) + (int64_t)cell * 10;
+  struct Data {
+    Number ji[kAffine ? 1 : 9], w, c;  // w: the point's quadrature weight (kAffine) or JxW
+  };
+  __device__ Cell load_cell(int cell) const {
+    Cell cd{};
+    if constexpr (kAffine) {
+      const ConstantPtr<Number> g = as_constant(cell_geo) + (int64_t)cell * 7;
 #pragma unroll
-      for (int f = 0; f < 9; ++f) d.ji[f] = g[f];
-      d.jxw = g[9] * wq[pt];
-      d.c = stream_load(qd + q);
-      return d;
+      for (int f = 0; f < 6; ++f) cd.g[f] = g[f];
+      cd.det = g[6];
     }
+    return cd;
+  }
+  __device__ Data load(int64_t qb, uint32_t lo, int pt) const {
+    Data d;
+    if constexpr (kAffine) {
+      d.w = wq[pt];
+      d.c = stream_load(qd + qb + lo);
+    } else {
 #pragma unroll
-    for (int f = 0; f < 9; ++f) d.ji[f] = stream_load(qd + f * nqp + q);
-    d.jxw = stream_load(qd + 9 * nqp + q);
-    d.c = stream_load(qd + 10 * nqp + q);
+      for (int f = 0; f < 9; ++f) d.ji[f] = stream_load(qd + f * nqp + qb + lo);
+      d.w = stream_load(qd + 9 * nqp + qb + lo);
+      d.c = stream_load(qd + 10 * nqp + qb + lo);
+    }
     return d;
   }
-  __device__ void apply(const Data &d, Number (&val)[1], Number (&grad)[1][3]) const {
-    Number gx[3];
+  __device__ Number value_scale(const Cell &cd, const Data &d) const { return kAffine ? cd.det * d.w : d.w; }
+  __device__ void apply_grad(const Cell &cd, const Data &d, Number (&grad)[1][3]) const {
+    const Number s = d.c * dt * value_scale(cd, d);
+    const Number g0 = grad[0][0], g1 = grad[0][1], g2 = grad[0][2];
+    if constexpr (kAffine) {
+      grad[0][0] = s * (cd.g[0] * g0 + cd.g[3] * g1 + cd.g[4] * g2);
+      grad[0][1] = s * (cd.g[3] * g0 + cd.g[1] * g1 + cd.g[5] * g2);
+      grad[0][2] = s * (cd.g[4] * g0 + cd.g[5] * g1 + cd.g[2] * g2);
+    } else {
+      Number gx[3];
 #pragma unroll
-    for (int e = 0; e < 3; ++e) gx[e] = grad[0][0] * d.ji[e] + grad[0][1] * d.ji[3 + e] + grad[0][2] * d.ji[6 + e];
-    const Number s = d.c * dt * d.jxw;
+      for (int e = 0; e < 3; ++e) gx[e] = g0 * d.ji[e] + g1 * d.ji[3 + e] + g2 * d.ji[6 + e];
 #pragma unroll
-    for (int f = 0; f < 3; ++f) grad[0][f] = s * (gx[0] * d.ji[f * 3] + gx[1] * d.ji[f * 3 + 1] + gx[2] * d.ji[f * 3 + 2]);
-    val[0] = d.jxw * val[0];
+      for (int f = 0; f < 3; ++f)
+        grad[0][f] = s * (gx[0] * d.ji[f * 3] + gx[1] * d.ji[f * 3 + 1] + gx[2] * d.ji[f * 3 + 2]);
+    }
   }
 };
 
@@ -575,22 +616,25 @@ struct QSolidSR {
   int64_t nqp;
   const Number *u;  // nodal linearisation point, 3 per node
   Number mu, two_lambda, rho_alpha;
+  using Cell = NoCell;
+  __device__ Cell load_cell(int) const { return Cell{}; }
   struct Data {
     Number ji[9], jxw, sc, ug[9];
   };
-  __device__ Data load(int64_t q, int cell, int pt) const {
+  __device__ Data load(int64_t qb, uint32_t lo, int) const {
     Data d;
 #pragma unroll
-    for (int f = 0; f < 9; ++f) d.ji[f] = stream_load(qd + f * nqp + q);
-    d.jxw = stream_load(qd + 9 * nqp + q);
-    d.sc = stream_load(qd + 10 * nqp + q);
+    for (int f = 0; f < 9; ++f) d.ji[f] = stream_load(qd + f * nqp + qb + lo);
+    d.jxw = stream_load(qd + 9 * nqp + qb + lo);
+    d.sc = stream_load(qd + 10 * nqp + qb + lo);
     return d;
   }
   __device__ void attach(Data &d, const Number (&ug)[3][3]) const {
 #pragma unroll
     for (int f = 0; f < 9; ++f) d.ug[f] = ug[f / 3][f % 3];
   }
-  __device__ void apply(const Data &d, Number (&val)[3], Number (&grad)[3][3]) const {
+  __device__ Number value_scale(const Cell &, const Data &d) const { return d.jxw * rho_alpha; }
+  __device__ void apply_grad(const Cell &, const Data &d, Number (&grad)[3][3]) const {
     Number g[3][3], F[3][3];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
@@ -642,7 +686,6 @@ struct QSolidSR {
       for (int b = 0; b < 3; ++b) Pm[b] = Q[c][0] * Fi[b][0] + Q[c][1] * Fi[b][1] + Q[c][2] * Fi[b][2];
 #pragma unroll
       for (int f = 0; f < 3; ++f) grad[c][f] = d.jxw * (Pm[0] * d.ji[f * 3 + 0] + Pm[1] * d.ji[f * 3 + 1] + Pm[2] * d.ji[f * 3 + 2]);
-      val[c] = d.jxw * rho_alpha * val[c];
     }
   }
 };
@@ -660,22 +703,25 @@ struct QSolidT4 {
   const Number *qd;
   int64_t nqp;
   Number rho_alpha;
+  using Cell = NoCell;
+  __device__ Cell load_cell(int) const { return Cell{}; }
   struct Data {
     Number ji[9], jxw, c1, T[6];
     int64_t q;
   };
-  __device__ Data load(int64_t q, int cell, int pt) const {
+  __device__ Data load(int64_t qb, uint32_t lo, int) const {
     Data d;
 #pragma unroll
-    for (int f = 0; f < 9; ++f) d.ji[f] = stream_load(qd + f * nqp + q);
-    d.jxw = stream_load(qd + 9 * nqp + q);
-    d.c1 = stream_load(qd + 10 * nqp + q);
+    for (int f = 0; f < 9; ++f) d.ji[f] = stream_load(qd + f * nqp + qb + lo);
+    d.jxw = stream_load(qd + 9 * nqp + qb + lo);
+    d.c1 = stream_load(qd + 10 * nqp + qb + lo);
 #pragma unroll
-    for (int f = 0; f < 6; ++f) d.T[f] = stream_load(qd + (11 + f) * nqp + q);
-    d.q = q;
+    for (int f = 0; f < 6; ++f) d.T[f] = stream_load(qd + (11 + f) * nqp + qb + lo);
+    d.q = qb + lo;
     return d;
   }
-  __device__ void apply(const Data &d, Number (&val)[3], Number (&grad)[3][3]) const {
+  __device__ Number value_scale(const Cell &, const Data &d) const { return d.jxw * rho_alpha * d.c1; }
+  __device__ void apply_grad(const Cell &, const Data &d, Number (&grad)[3][3]) const {
     Number g[3][3];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
@@ -706,7 +752,6 @@ struct QSolidT4 {
 #pragma unroll
       for (int f = 0; f < 3; ++f)
         grad[c][f] = d.jxw * (Pm[c][0] * d.ji[f * 3 + 0] + Pm[c][1] * d.ji[f * 3 + 1] + Pm[c][2] * d.ji[f * 3 + 2]);
-      val[c] = d.jxw * rho_alpha * d.c1 * val[c];
     }
   }
 };
@@ -722,19 +767,22 @@ struct QSolidT4NS {
   const Number *qd;
   int64_t nqp;
   Number rho_alpha;
+  using Cell = NoCell;
+  __device__ Cell load_cell(int) const { return Cell{}; }
   struct Data {
     Number ji[9], jxw;
     int64_t q;
   };
-  __device__ Data load(int64_t q, int cell, int pt) const {
+  __device__ Data load(int64_t qb, uint32_t lo, int) const {
     Data d;
 #pragma unroll
-    for (int f = 0; f < 9; ++f) d.ji[f] = stream_load(qd + f * nqp + q);
-    d.jxw = stream_load(qd + 9 * nqp + q);
-    d.q = q;
+    for (int f = 0; f < 9; ++f) d.ji[f] = stream_load(qd + f * nqp + qb + lo);
+    d.jxw = stream_load(qd + 9 * nqp + qb + lo);
+    d.q = qb + lo;
     return d;
   }
-  __device__ void apply(const Data &d, Number (&val)[3], Number (&grad)[3][3]) const {
+  __device__ Number value_scale(const Cell &, const Data &d) const { return d.jxw * rho_alpha; }
+  __device__ void apply_grad(const Cell &, const Data &d, Number (&grad)[3][3]) const {
     Number g[3][3];
 #pragma unroll
     for (int c = 0; c < 3; ++c)
@@ -757,7 +805,6 @@ struct QSolidT4NS {
 #pragma unroll
       for (int f = 0; f < 3; ++f)
         grad[c][f] = d.jxw * (Pm[c][0] * d.ji[f * 3 + 0] + Pm[c][1] * d.ji[f * 3 + 1] + Pm[c][2] * d.ji[f * 3 + 2]);
-      val[c] = d.jxw * rho_alpha * val[c];
     }
   }
 };
@@ -830,9 +877,12 @@ __device__ inline void cell_group(const QOp &qop, const uint32_t *__restrict__ c
   T.writer = !pad;
   const int cell = cell_begin + lc;
   const bool active = !pad && cell < cell_end;
-  const int64_t qidx = active ? (int64_t)cell * N3 + pt : 0;
+  // this thread's point: a base that is the same on every lane and a 32-bit
+  // lane offset (threads without a point stay on the group's first)
+  const int64_t qb = (int64_t)__builtin_amdgcn_readfirstlane(cell_begin) * N3;
+  const uint32_t lo = active ? (uint32_t)t : 0u;
 
-  uint32_t entry = active ? cell_nodes[qidx] : 0u;
+  uint32_t entry = active ? (cell_nodes + qb)[lo] : 0u;
   // the 1D matrices are loaded with the map and written to LDS just before
   // the first barrier of the sweeps, which publishes them: no wait on these
   // loads stands before the gather
@@ -860,7 +910,7 @@ __device__ inline void cell_group(const QOp &qop, const uint32_t *__restrict__ c
   // late read gives the kernel one more wave per SIMD and is the faster of the
   // two (measured); for the heat op and the 10-word tensor2 op, whose wave
   // count it does not change, and elsewhere the early read is.
-  constexpr bool kLateDst = sizeof(Number) == 8 && P <= 4 && !std::is_same<QOp, QHeat<Number>>::value &&
+  constexpr bool kLateDst = sizeof(Number) == 8 && P <= 4 && NC == 3 &&
                             !std::is_same<QOp, QSolidT2F1G<Number>>::value &&
                             !std::is_same<QOp, QSolidT2F1G<Number, true>>::value &&
                             !std::is_same<QOp, QSolidT2F1G<Number, true, true>>::value;
@@ -881,7 +931,8 @@ __device__ inline void cell_group(const QOp &qop, const uint32_t *__restrict__ c
   // one cell per workgroup: the cell index is the same on every lane (padding
   // lanes included), which lets the per-cell tables come in as scalar loads
   const int qcell = cpb == 1 ? __builtin_amdgcn_readfirstlane(cell < cell_end ? cell : 0) : (active ? cell : 0);
-  typename QOp::Data qd = qop.load(qidx, qcell, pt);
+  typename QOp::Data qd = qop.load(qb, lo, pt);
+  const typename QOp::Cell cd = qop.load_cell(qcell);
   // read only after the barrier that follows the first puts of the sweeps
   if (table_lane) {
     s_shape[t] = sh;
@@ -897,11 +948,11 @@ __device__ inline void cell_group(const QOp &qop, const uint32_t *__restrict__ c
 
   Number val[NC], grad[NC][3];
   evaluate_vg<N, NC, Number>(T, s_shape, s_colloc, u, val, grad);
-  qop.apply(qd, val, grad);
+  apply_qop(qop, cd, qd, val, grad);
   Number out[NC];
   integrate_vg<N, NC, Number, kSpareSlots>(T, s_shape, s_colloc, val, grad, out);
   if constexpr (kToCells) {
-    if (active) store_node<Number, NC>(dst + qidx * NC, out);
+    if (active) store_node<Number, NC>(dst + (qb + lo) * NC, out);
     return;
   }
   if constexpr (kLateDst) {

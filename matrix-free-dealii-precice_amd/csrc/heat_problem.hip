@@ -49,8 +49,8 @@ struct HeatRhsArgs {
 // value JxW (u_old + dt f - u_D) and the gradient of -dt c grad u_D, i.e.
 // int (u_old + dt f) phi - A u_D.  Scatter as the operator does (the first
 // colour touching a node stores).
-template <int P, int CPB>
-__global__ void __launch_bounds__((block_threads<P, CPB>())) heat_rhs_cells(HeatRhsArgs a, QHeat<double> qop) {
+template <int P, int CPB, class QOp>
+__global__ void __launch_bounds__((block_threads<P, CPB>())) heat_rhs_cells(HeatRhsArgs a, QOp qop) {
   constexpr int N = P + 1, N3 = N * N * N;
   __shared__ double s_shape[N * N], s_colloc[N * N];
   __shared__ double s_tile[CPB * 6 * N3];
@@ -76,14 +76,15 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) heat_rhs_cells(Heat
   const uint32_t entry = active ? a.cell_nodes[qidx] : 0u;
   const int64_t node = entry & kNodeMaskDev;
   const double u2[2] = {active ? a.u_dir[node] : 0.0, active ? a.u_old[node] : 0.0};
-  const typename QHeat<double>::Data qd = qop.load(qidx, active ? cell : 0, pt);
+  const typename QOp::Data qd = qop.load(qidx, 0, pt);
+  const typename QOp::Cell cd = qop.load_cell(active ? cell : 0);
   const double f = (active && a.f) ? a.f[(int64_t)a.perm[cell] * N3 + pt] : 0.0;
   __syncthreads();
   double val[2], grad[2][3];
   evaluate_vg<N, 2, double>(T, s_shape, s_colloc, u2, val, grad);
   double v1[1] = {val[0]}, g1[1][3] = {{grad[0][0], grad[0][1], grad[0][2]}};
-  qop.apply(qd, v1, g1);  // A u_D at the point: JxW u_D and dt c JxW J^-T J^-1 grad u_D
-  double vs[1] = {qd.jxw * (val[1] + a.dt * f) - v1[0]};
+  apply_qop(qop, cd, qd, v1, g1);  // A u_D at the point: JxW u_D and dt c JxW J^-T J^-1 grad u_D
+  double vs[1] = {qop.value_scale(cd, qd) * (val[1] + a.dt * f) - v1[0]};
   double gs[1][3] = {{-g1[0][0], -g1[0][1], -g1[0][2]}};
   double out[1];
   integrate_vg<N, 1, double>(T, s_shape, s_colloc, vs, gs, out);
@@ -105,8 +106,8 @@ struct HeatErrorArgs {
 };
 
 // sum over the group's points of (exact - u_h)^2 JxW, u_h read as stored
-template <int P, int CPB>
-__global__ void __launch_bounds__((block_threads<P, CPB>())) heat_error_cells(HeatErrorArgs a, QHeat<double> qop) {
+template <int P, int CPB, class QOp>
+__global__ void __launch_bounds__((block_threads<P, CPB>())) heat_error_cells(HeatErrorArgs a, QOp qop) {
   constexpr int N = P + 1, N3 = N * N * N, NT = block_threads<P, CPB>();
   __shared__ double s_shape[N * N], s_colloc[N * N];
   __shared__ double s_tile[CPB * 3 * N3];
@@ -132,13 +133,14 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) heat_error_cells(He
   const int64_t qidx = active ? (int64_t)cell * N3 + pt : 0;
   const int64_t node = active ? (int64_t)(a.cell_nodes[qidx] & kNodeMaskDev) : 0;
   const double u1[1] = {active ? a.u[node] : 0.0};
-  const typename QHeat<double>::Data qd = qop.load(qidx, active ? cell : 0, pt);
+  const typename QOp::Data qd = qop.load(qidx, 0, pt);
+  const typename QOp::Cell cd = qop.load_cell(active ? cell : 0);
   const double ex = active ? a.exact[(int64_t)a.perm[cell] * N3 + pt] : 0.0;
   __syncthreads();
   double val[1], grad[1][3];
   evaluate_vg<N, 1, double>(T, s_shape, s_colloc, u1, val, grad);
   const double e = ex - val[0];
-  s_red[t] = active ? e * e * qd.jxw : 0.0;
+  s_red[t] = active ? e * e * qop.value_scale(cd, qd) : 0.0;
   __syncthreads();
   // fold the block (any size) into 64 values, then a tree; fixed order
   __shared__ double s_fold[64];
@@ -170,9 +172,12 @@ static void quadrature_points_t(const OperatorData &op, double *xyz) {
   MFG_HIP(hipGetLastError());
 }
 
-static QHeat<double> heat_qop(const OperatorData &op) {
-  return QHeat<double>{op.qd.as<double>(), op.nqp, op.dt, op.affine_ref ? op.cell_geo.as<double>() : nullptr,
-                       op.wq3.as<double>()};
+template <class F>
+static void with_heat_qop(const OperatorData &op, F fn) {
+  if (op.affine_ref)
+    fn(QHeat<double, true>{op.qd.as<double>(), op.nqp, op.dt, op.cell_geo.as<double>(), op.wq3.as<double>()});
+  else
+    fn(QHeat<double, false>{op.qd.as<double>(), op.nqp, op.dt, nullptr, nullptr});
 }
 
 template <int P>
@@ -189,13 +194,14 @@ static void heat_rhs_t(const OperatorData &op, double *rhs, const double *u_old,
   a.colloc = op.tab_colloc.as<double>();
   a.dt = op.dt;
   a.rhs = rhs;
-  const QHeat<double> q = heat_qop(op);
   for (size_t col = 0; col + 1 < op.colour_start.size(); ++col) {
     a.cell_begin = op.colour_start[col];
     a.cell_end = op.colour_start[col + 1];
     const int groups = (a.cell_end - a.cell_begin + CPB - 1) / CPB;
     if (groups == 0) continue;
-    heat_rhs_cells<P, CPB><<<groups, block_threads<P, CPB>(), 0, op.stream>>>(a, q);
+    with_heat_qop(op, [&](auto q) {
+      heat_rhs_cells<P, CPB, decltype(q)><<<groups, block_threads<P, CPB>(), 0, op.stream>>>(a, q);
+    });
     MFG_HIP(hipGetLastError());
   }
   if (op.n_constrained > 0) {
@@ -219,7 +225,9 @@ static double heat_error_t(const OperatorData &op, const double *u, const double
   a.shape = op.tab_shape.as<double>();
   a.colloc = op.tab_colloc.as<double>();
   a.partials = partials.as<double>();
-  heat_error_cells<P, CPB><<<groups, block_threads<P, CPB>(), 0, op.stream>>>(a, heat_qop(op));
+  with_heat_qop(op, [&](auto q) {
+    heat_error_cells<P, CPB, decltype(q)><<<groups, block_threads<P, CPB>(), 0, op.stream>>>(a, q);
+  });
   MFG_HIP(hipGetLastError());
   std::vector<double> h((size_t)groups);
   MFG_HIP(hipMemcpyAsync(h.data(), partials.ptr, h.size() * sizeof(double), hipMemcpyDeviceToHost, op.stream));

@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "column_kernels.hpp"
 #include "common.hpp"
 #include "operator.hpp"
 #include "setup_kernels.hpp"
@@ -34,10 +35,13 @@ QSolidT2F1G<Number, kEarlyCell, kCartesian> t2_gradient_op(const OperatorData &o
                                                      op.cell_jxw.as<Number>(), op.wq3.as<Number>()};
 }
 
-// per-cell geometry of the heat op on affine meshes, or null (per-point fields)
-template <typename Number>
-const Number *heat_cell_geo(const OperatorData &op) {
-  return op.affine_ref ? op.cell_geo.as<Number>() : nullptr;
+// fn(q) with the heat op
+template <typename Number, class F>
+static void with_heat_qop(const OperatorData &op, F fn) {
+  if (op.affine_ref)
+    fn(QHeat<Number, true>{op.qd.as<Number>(), op.nqp, Number(op.dt), op.cell_geo.as<Number>(), op.wq3.as<Number>()});
+  else
+    fn(QHeat<Number, false>{op.qd.as<Number>(), op.nqp, Number(op.dt), nullptr, nullptr});
 }
 
 // fn(q) with the quadrature op of this operator for the cells of material m
@@ -47,7 +51,7 @@ const Number *heat_cell_geo(const OperatorData &op) {
 template <typename Number, bool kEarlyCell, class F>
 static void with_qop(const OperatorData &op, int m, F fn) {
   if (op.kind == 1) {
-    fn(QHeat<Number>{op.qd.as<Number>(), op.nqp, Number(op.dt), heat_cell_geo<Number>(op), op.wq3.as<Number>()});
+    with_heat_qop<Number>(op, fn);
     return;
   }
   const OperatorData::MaterialConstants &M = op.mats[m];
@@ -72,6 +76,65 @@ static void with_qop(const OperatorData &op, int m, F fn) {
   } else {
     fn(QSolidT2F0<Number>{op.qd.as<Number>(), op.nqp, Number(M.kappa), Number(M.c_1), ra});
   }
+}
+
+// Whether a launch over n_cells cells takes the column kernels (the results
+// are the same bit for bit).  They hold 64 / (p+1)^2 cells per wave at 1 to 4
+// waves per SIMD, so they need that many waves to fill the 1024 SIMDs; with
+// fewer, the point-per-thread kernels spread the same cells over more waves.
+// Measured over cubes of 2e4 to 2e7 unknowns, in one launch (GATHER) and in 8
+// colours, times as point -> column in us:
+//  - heat on affine cells: equal at about 600 waves (Q4 7.8 -> 9.2 at 172, Q2
+//    8.4 -> 8.4 at 392), 7 to 50 % faster from 1000 (Q4 16.6 -> 14.8 at 1688,
+//    Q6 16.8 -> 15.0 at 1000).  FP64 Q1 to Q3 is bound by its vector traffic
+//    once that leaves the caches: Q2 151 -> 143 at 46,656 cells a launch but
+//    906 -> 943 at 314,432, Q3 108 -> 103 at 13,824 but 583 -> 608 at 91,125;
+//    Q1 gains nothing at any size.
+//  - solid Q6 FP64: 175 -> 146 at 614 waves, 881 -> 577 at 3724 (formulation 0
+//    213 -> 176 and 1027 -> 743).
+//  - solid Q5 and Q6 FP32, Q5 FP64, formulation 1: slower at 614 to 1000 waves
+//    (Q6 FP32 91 -> 118, Q5 FP64 113.6 -> 114), faster at 1728 and above (Q6
+//    FP32 36.6 -> 30.7, Q5 FP64 48.5 -> 45.9 at 2744).
+//  - solid up to Q4: not faster at the large sizes.
+template <int P, typename Number>
+constexpr bool has_heat_columns() {
+  return P >= 2 || sizeof(Number) == 4;
+}
+template <int P, typename Number>
+static bool use_columns(const OperatorData &op, int n_cells) {
+  constexpr bool fp64 = sizeof(Number) == 8;
+  const int waves = blocks_for(n_cells, column_cells<P>());
+  if (op.kind == 1)
+    return has_heat_columns<P, Number>() && op.affine_ref && waves >= 768 && !(fp64 && P <= 3 && n_cells > 65536);
+  if (P < 5 || op.sp.caching != MFG_CACHING_TENSOR2) return false;
+  if (fp64 && P == 6) return waves >= 512;
+  return op.sp.formulation == 1 && waves >= 1536;
+}
+// fn(q) with the quadrature op of the column kernels, where use_columns holds
+template <int P, typename Number, class F>
+static void with_column_qop(const OperatorData &op, int m, F fn) {
+  const OperatorData::MaterialConstants &M = op.mats[m];
+  if constexpr (has_heat_columns<P, Number>()) {
+    if (op.kind == 1) {
+      fn(QHeat<Number, true>{op.qd.as<Number>(), op.nqp, Number(op.dt), op.cell_geo.as<Number>(),
+                             op.wq3.as<Number>()});
+      return;
+    }
+  }
+  if constexpr (P >= 5) {
+    if (op.t2_gradient()) {
+      if (op.cartesian_ref) fn(t2_gradient_op<Number, false, true>(op, m));
+      else fn(t2_gradient_op<Number>(op, m));
+      return;
+    }
+    if (op.sp.formulation == 1) {
+      fn(QSolidT2F1<Number>{op.qd.as<Number>(), op.nqp, Number(2.0 * M.lambda), Number(M.rho_alpha),
+                            t2_cell_jxw<Number>(op), op.wq3.as<Number>()});
+      return;
+    }
+  }
+  if constexpr (P == 6 && sizeof(Number) == 8)
+    fn(QSolidT2F0<Number>{op.qd.as<Number>(), op.nqp, Number(M.kappa), Number(M.c_1), Number(M.rho_alpha)});
 }
 
 template <typename Number>
@@ -102,6 +165,17 @@ static void launch_apply(const OperatorData &op, const void *src, void *dst, int
     // material); the first launch also writes the identity rows
     bool fix_pending = true;
     op.for_each_range([&](int, int b, int e, int m) {
+      if (use_columns<P, Number>(op, e - b)) {
+        with_column_qop<P, Number>(op, m, [&](auto q) {
+          a.cell_begin = b;
+          a.cell_end = e;
+          a.fix_mode = fix_pending ? fix_mode : 0;
+          fix_pending = false;
+          apply_columns<P, Number, decltype(q)><<<blocks_for(e - b, column_cells<P>()), 64, 0, stream>>>(a, q, assign);
+          MFG_HIP(hipGetLastError());
+        });
+        return;
+      }
       with_qop<Number, CPB == 1>(op, m, [&](auto q) {
         a.cell_begin = b;
         a.cell_end = e;
@@ -117,9 +191,17 @@ static void launch_apply(const OperatorData &op, const void *src, void *dst, int
   // buffer, then the ordered per-node sums
   a.fix_mode = 0;
   auto cells = [&](int b, int e, int m) {
+    a.cell_begin = b;
+    a.cell_end = e;
+    if (use_columns<P, Number>(op, e - b)) {
+      with_column_qop<P, Number>(op, m, [&](auto q) {
+        apply_columns_to_cells<P, Number, decltype(q)>
+            <<<blocks_for(e - b, column_cells<P>()), 64, 0, stream>>>(a, q, op.contrib.as<Number>());
+        MFG_HIP(hipGetLastError());
+      });
+      return;
+    }
     with_qop<Number, CPB == 1>(op, m, [&](auto q) {
-      a.cell_begin = b;
-      a.cell_end = e;
       apply_cells_to_cells<P, CPB, Number, decltype(q)><<<blocks_for(e - b, CPB), NT, 0, stream>>>(
           a, q, op.contrib.as<Number>());
       MFG_HIP(hipGetLastError());
@@ -577,7 +659,7 @@ static void heat_geometry(OperatorData &op, const mfg_level_desc &d, const doubl
   const int64_t n = op.nqp;
   if (op.affine_ref) {
     // affine cells: the geometry once per cell, the coefficient per point
-    std::vector<Number> geo((size_t)op.n_cells * 10), cq((size_t)n);
+    std::vector<Number> geo((size_t)op.n_cells * 7), cq((size_t)n);
     for (int c = 0; c < op.n_cells; ++c) {
       const int64_t orig = op.perm[c];
       const double *X = d.cell_vertices + orig * 24;
@@ -597,8 +679,11 @@ static void heat_geometry(OperatorData &op, const mfg_level_desc &d, const doubl
                            (J[0][0] * J[2][2] - J[0][2] * J[2][0]) * id, (J[0][2] * J[1][0] - J[0][0] * J[1][2]) * id,
                            (J[1][0] * J[2][1] - J[1][1] * J[2][0]) * id, (J[0][1] * J[2][0] - J[0][0] * J[2][1]) * id,
                            (J[0][0] * J[1][1] - J[0][1] * J[1][0]) * id};
-      for (int f = 0; f < 9; ++f) geo[(size_t)c * 10 + f] = (Number)R[f];
-      geo[(size_t)c * 10 + 9] = (Number)det;
+      for (int s6 = 0; s6 < 6; ++s6) {
+        const double *a = R + 3 * kSymI[s6], *b = R + 3 * kSymJ[s6];
+        geo[(size_t)c * 7 + s6] = (Number)(a[0] * b[0] + a[1] * b[1] + a[2] * b[2]);
+      }
+      geo[(size_t)c * 7 + 6] = (Number)det;
       for (int q = 0; q < N3; ++q) cq[(size_t)c * N3 + q] = (Number)(coef ? coef[orig * N3 + q] : 1.0);
     }
     upload(op.cell_geo, geo.data(), geo.size(), op.stream);
@@ -643,7 +728,7 @@ static void heat_geometry(OperatorData &op, const mfg_level_desc &d, const doubl
 void OperatorData::setup_heat(const mfg_level_desc &d, const double *coef) {
   if (precision == MFG_FP64) heat_geometry<double>(*this, d, coef);
   else heat_geometry<float>(*this, d, coef);
-  n_fields = affine_ref ? 1 : QHeat<double>::kFields;
+  n_fields = affine_ref ? QHeat<double, true>::kFields : QHeat<double, false>::kFields;
   ready = true;
 }
 

@@ -41,7 +41,7 @@ struct OperatorData {
   // JxW_ref = cell_jxw[stored cell] * wq3[point] (tensor2, formulation 1)
   bool affine_ref = false;
   DeviceBuffer cell_jxw, wq3;
-  DeviceBuffer cell_geo;  // heat on affine cells: Jinv (9), det J per stored cell
+  DeviceBuffer cell_geo;  // heat on affine cells: Jinv Jinv^T (6, symmetric), det J per stored cell
   DeviceBuffer cell_met;  // solid on affine cells: J_ref^{-1} J_ref^{-T} (6, symmetric) per stored cell
   bool cartesian_ref = false;  // affine, and every cell's J_ref is diagonal
   int t2_storage = MFG_T2_FOLDED;  // tensor2 formulation-1 point storage (MFG_T2_*)

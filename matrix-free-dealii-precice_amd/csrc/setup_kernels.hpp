@@ -300,7 +300,8 @@ __global__ void __launch_bounds__(((P + 1) * (P + 1) * (P + 1) + 63) / 64 * 64) 
   const int64_t qidx = active ? (int64_t)cell * N3 + pt : 0;
   Number coef[NTERM];
   {
-    typename QOp::Data qd = qop.load(qidx, active ? cell : 0, pt);
+    typename QOp::Data qd = qop.load((int64_t)(a.cell_begin + blockIdx.x) * N3, (uint32_t)pt, pt);
+    const typename QOp::Cell cd = qop.load_cell(active ? cell : 0);
     if constexpr (QOp::kNodalField) {
       __shared__ Number s_shape[N * N], s_colloc[N * N];
       if (t < N * N) {
@@ -320,7 +321,7 @@ __global__ void __launch_bounds__(((P + 1) * (P + 1) * (P + 1) + 63) / 64 * 64) 
       v[c] = 1;
       g[c][0] = g[c][1] = g[c][2] = 0;
     }
-    qop.apply(qd, v, g);
+    apply_qop(qop, cd, qd, v, g);
 #pragma unroll
     for (int c = 0; c < NC; ++c) coef[c * 7] = v[c];
     Number G[NC][3][3];
@@ -334,7 +335,7 @@ __global__ void __launch_bounds__(((P + 1) * (P + 1) * (P + 1) + 63) / 64 * 64) 
           g[c][0] = g[c][1] = g[c][2] = 0;
         }
         g[d][gg] = 1;
-        qop.apply(qd, v, g);
+        apply_qop(qop, cd, qd, v, g);
 #pragma unroll
         for (int f = 0; f < 3; ++f) G[d][f][gg] = g[d][f];
       }

@@ -546,3 +546,63 @@ def test_gradient_point_storage_export(cuda, p, precision, amp):
     s = O.MU - 2 * lam * np.log(np.linalg.det(np.eye(3) + A))
     # ln det F to the rounding of F and of the gradient over a cell
     assert np.abs(g[9] - s).max() <= 2 * lam * (16 * eps + 9 * tol / 0.2) + 4 * eps * O.MU
+
+
+# (kind, degree, precision, cells): one launch over all cells (GATHER) takes the
+# column-per-thread kernels, the eighth of them in a colour launch the
+# point-per-thread ones.  Cell counts: the first the column kernels serve (768
+# waves of 64 // (p+1)^2 heat cells, 1536 or 512 solid cells) and others whose
+# last wave is not full.
+COLUMN_CASES = [
+    ("heat", 1, mfgpu.FP32, (24, 32, 16)), ("heat", 2, mfgpu.FP64, (21, 16, 16)), ("heat", 2, mfgpu.FP32, (19, 17, 18)),
+    ("heat", 3, mfgpu.FP64, (15, 15, 14)), ("heat", 3, mfgpu.FP32, (16, 16, 12)), ("heat", 4, mfgpu.FP64, (13, 13, 13)),
+    ("heat", 4, mfgpu.FP32, (12, 16, 8)), ("heat", 5, mfgpu.FP64, (11, 10, 9)), ("heat", 6, mfgpu.FP64, (8, 8, 12)),
+    ("heat", 6, mfgpu.FP32, (9, 10, 9)), ("solid", 5, mfgpu.FP64, (12, 16, 8)), ("solid", 5, mfgpu.FP32, (13, 11, 11)),
+    ("solid", 6, mfgpu.FP64, (8, 8, 8)), ("solid", 6, mfgpu.FP32, (12, 16, 8)), ("solid_f0", 6, mfgpu.FP64, (9, 8, 8)),
+    ("solid_folded", 5, mfgpu.FP64, (12, 16, 8)), ("solid_sheared", 5, mfgpu.FP64, (12, 16, 8)),
+    ("solid_distorted", 6, mfgpu.FP64, (8, 8, 8)),
+]
+
+
+@pytest.mark.parametrize("kind,p,precision,n", COLUMN_CASES)
+def test_column_kernels(cuda, kind, p, precision, n):
+    """vmult and vmult_add of the column kernels against the oracle, and bit for
+    bit against the point-per-thread kernels."""
+    print(f"columns {kind} p={p} precision={precision} n={n}", flush=True)
+    lo, hi = [0, 0, 0], [1.0, 0.6, 0.4]
+    nc, fm, cm = (1, 63, 1) if kind == "heat" else (3, 1, 7)
+    om = O.Mesh(lo, hi, list(n), p, nc, fm, cm)
+    gm = mfgpu.BoxMesh(lo, hi, list(n), p, nc, fm, cm)
+    if kind in ("solid_sheared", "solid_distorted"):
+        A = np.array([[1.0, 0.3, 0.1], [0.05, 1.0, 0.2], [0.1, -0.15, 1.0]])
+        v = om.cell_vertices()
+        v = (v.reshape(-1, 3) @ A.T).ravel() if kind == "solid_sheared" else distort(v)
+        om.set_cell_vertices(v)
+        gm = DistortedMesh(gm, v)
+    if kind == "heat":
+        coef = np.random.default_rng(p).uniform(0.5, 2.0, om.n_cells * (p + 1) ** 3)
+        oo = O.Heat(om, dt=0.1, coef=coef)
+        go = mfgpu.LaplaceOperator(gm, 0.1, coef, precision=precision)
+    else:
+        form = 0 if kind == "solid_f0" else 1
+        u = om.u0(amp=1e-2, noise=1e-5)
+        oo = O.Solid(om, formulation=form, caching=1)
+        oo.cache(u)
+        go = mfgpu.NeoHookOperator(gm, O.MU, O.NU, O.RHO, O.ALPHA1, formulation=form, precision=precision)
+        if kind == "solid_folded":
+            go.set_point_storage(mfgpu.T2_FOLDED)
+        go.cache(dev(u, go.dtype))
+    x = dev(O.fill_uniform(5, om.n_dofs), go.dtype)
+    y0 = dev(O.fill_uniform(6, om.n_dofs), go.dtype)
+    ref = oo.vmult(x.double().cpu().numpy())
+    tol = TOL64 if precision == mfgpu.FP64 else TOL32
+    out = []
+    for sched in (mfgpu.CELLS_GATHER, mfgpu.CELLS_COLOURS):
+        go.set_cell_schedule(sched)
+        y = torch.full((om.n_dofs,), float("nan"), dtype=go.dtype, device="cuda")
+        go.vmult(y, x)
+        assert rel(y.double(), ref) < tol, sched
+        z = y0.clone()
+        go.vmult_add(z, x)
+        out.append((y, z))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
