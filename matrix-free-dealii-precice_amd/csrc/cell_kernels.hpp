@@ -107,19 +107,24 @@ struct Tile {
 
 // The gradient phase of evaluate_vg and the first phase of integrate_vg read
 // 3 NC lines of N LDS values each.  Unrolled over the components, the
-// compiler issues all of them at once: for N >= 5 that peak (about 120 VGPRs
-// in FP64) holds the cell kernel at 2 waves per SIMD.  A rolled component
-// loop frees those registers (3 to 4 waves); for N <= 4 the unrolled form is
-// faster.
-template <int N>
+// compiler issues all of them at once; rolled, each line's reads wait for the
+// one before, since the register-indexed result keeps them in order.  For
+// N >= 6 the unrolled form's registers cost more than that (Q5 FP64 192 VGPRs
+// against 124, 20M unknowns: 658 against 560 us).  For N = 5 the kernel with
+// the 10-word point operation takes 106 VGPRs unrolled, 126 rolled: 487 -> 480
+// us at 20M unknowns FP64, 39.7 -> 37.5 us at 0.2M (FP32 266 -> 264, 35.4 ->
+// 33.1); the other point operations gain as well (formulation 0 649 -> 624,
+// the folded words 544 -> 526).  scalar_referential evaluates two fields (194
+// VGPRs unrolled) and stays rolled.
+template <int N, bool kTwoFields = false>
 constexpr bool rolled_components() {
-  return N >= 5;
+  return N >= (kTwoFields ? 5 : 6);
 }
 
 // Evaluate values and reference-coordinate gradients at the quadrature points
 // of NC components; slots 0..2NC-1 are used.  On return the B slots hold the
 // point values (still read by later lines until the next barrier).
-template <int N, int NC, typename Number>
+template <int N, int NC, typename Number, bool kRolled = rolled_components<N>()>
 __device__ inline void evaluate_vg(const Tile<N, Number> &T, const Number *S, const Number *D, const Number (&u)[NC],
                                    Number (&val)[NC], Number (&grad)[NC][3]) {
 #pragma unroll
@@ -146,7 +151,7 @@ __device__ inline void evaluate_vg(const Tile<N, Number> &T, const Number *S, co
     grad[c][1] = T.template line<1>(D, T.j, NC + c);
     grad[c][2] = T.template line<2>(D, T.k, NC + c);
   };
-  if constexpr (rolled_components<N>()) {
+  if constexpr (kRolled) {
 #pragma unroll 1
     for (int c = 0; c < NC; ++c) gradient(c);
   } else {
@@ -160,7 +165,7 @@ __device__ inline void evaluate_vg(const Tile<N, Number> &T, const Number *S, co
 // has 5NC slots and the gradients go to slots 2NC.. that evaluate_vg does not
 // use, which makes the two barriers that only guard slot reuse (after
 // evaluate_vg's last reads and after the gradient lines) unnecessary.
-template <int N, int NC, typename Number, bool kSpareSlots = false>
+template <int N, int NC, typename Number, bool kSpareSlots = false, bool kRolled = rolled_components<N>()>
 __device__ inline void integrate_vg(const Tile<N, Number> &T, const Number *S, const Number *D,
                                     const Number (&val)[NC], const Number (&grad)[NC][3], Number (&out)[NC]) {
   constexpr int G0 = kSpareSlots ? 2 * NC : 0;  // first gradient slot
@@ -175,7 +180,7 @@ __device__ inline void integrate_vg(const Tile<N, Number> &T, const Number *S, c
     r[c] = val[c] + T.template line_t<0>(D, T.i, G0 + 3 * c + 0) + T.template line_t<1>(D, T.j, G0 + 3 * c + 1) +
            T.template line_t<2>(D, T.k, G0 + 3 * c + 2);
   };
-  if constexpr (rolled_components<N>()) {
+  if constexpr (kRolled) {
 #pragma unroll 1
     for (int c = 0; c < NC; ++c) gradient_t(c);
   } else {
@@ -201,11 +206,11 @@ __device__ inline void integrate_vg(const Tile<N, Number> &T, const Number *S, c
 }
 
 // Evaluate only reference gradients (cache()); same slot usage as evaluate_vg.
-template <int N, int NC, typename Number>
+template <int N, int NC, typename Number, bool kRolled = rolled_components<N>()>
 __device__ inline void evaluate_g(const Tile<N, Number> &T, const Number *S, const Number *D, const Number (&u)[NC],
                                   Number (&grad)[NC][3]) {
   Number val[NC];
-  evaluate_vg<N, NC, Number>(T, S, D, u, val, grad);
+  evaluate_vg<N, NC, Number, kRolled>(T, S, D, u, val, grad);
 }
 
 // The quadrature data is read once per operator application: load it
@@ -657,33 +662,27 @@ struct QSolidSR {
     Fi[2][0] = (F[1][0] * F[2][1] - F[1][1] * F[2][0]) * id;
     Fi[2][1] = (F[0][1] * F[2][0] - F[0][0] * F[2][1]) * id;
     Fi[2][2] = (F[0][0] * F[1][1] - F[0][1] * F[1][0]) * id;
-    // spatial gradient of the test direction: grad_X v F^{-1}
-    Number gx[3][3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int e = 0; e < 3; ++e) gx[c][e] = Fi[0][e] * g[c][0] + Fi[1][e] * g[c][1] + Fi[2][e] * g[c][2];
-    const Number trg = gx[0][0] + gx[1][1] + gx[2][2];
-    // tau = mu F F^T - (mu - 2 lambda ln J) I
-    Number tau[3][3];
+    // the stress products on the reference configuration (as in
+    // QSolidT2F1G): mu Grad v + ((s A + 2 lambda tr(A) I) F^{-1})^T with
+    // A = F^{-1} Grad v, then to reference-cell gradients
+    Number A[3][3];
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
-      for (int b = 0; b < 3; ++b)
-        tau[a][b] = mu * (F[a][0] * F[b][0] + F[a][1] * F[b][1] + F[a][2] * F[b][2]) - (a == b ? d.sc : Number(0));
-    Number Q[3][3];
+      for (int b = 0; b < 3; ++b) A[a][b] = Fi[a][0] * g[0][b] + Fi[a][1] * g[1][b] + Fi[a][2] * g[2][b];
+    const Number diag = two_lambda * (A[0][0] + A[1][1] + A[2][2]);
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
-      for (int b = 0; b < 3; ++b)
-        Q[a][b] = d.sc * (gx[a][b] + gx[b][a]) + (a == b ? two_lambda * trg : Number(0)) + gx[a][0] * tau[0][b] +
-                  gx[a][1] * tau[1][b] + gx[a][2] * tau[2][b];
-    // first Piola form: (jc + gx tau) F^{-T}, then to reference gradients
+      for (int b = 0; b < 3; ++b) A[a][b] = a == b ? d.sc * A[a][b] + diag : d.sc * A[a][b];
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       Number Pm[3];
 #pragma unroll
-      for (int b = 0; b < 3; ++b) Pm[b] = Q[c][0] * Fi[b][0] + Q[c][1] * Fi[b][1] + Q[c][2] * Fi[b][2];
+      for (int b = 0; b < 3; ++b) {
+        const Number r = A[b][0] * Fi[0][c] + A[b][1] * Fi[1][c] + A[b][2] * Fi[2][c];
+        Pm[b] = mu * g[c][b] + r;
+      }
 #pragma unroll
       for (int f = 0; f < 3; ++f) grad[c][f] = d.jxw * (Pm[0] * d.ji[f * 3 + 0] + Pm[1] * d.ji[f * 3 + 1] + Pm[2] * d.ji[f * 3 + 2]);
     }
@@ -863,6 +862,7 @@ __device__ inline void cell_group(const QOp &qop, const uint32_t *__restrict__ c
                                   const Number *__restrict__ g_colloc, Number *s_shape, Number *s_colloc,
                                   Number *s_tile) {
   constexpr int N = P + 1, N3 = N * N * N, NC = QOp::NC;
+  constexpr bool kRolled = rolled_components<N, QOp::kNodalField>();
   const int t = threadIdx.x;
   const int lc_raw = t / N3;
   const bool pad = lc_raw >= cpb;
@@ -942,15 +942,15 @@ __device__ inline void cell_group(const QOp &qop, const uint32_t *__restrict__ c
     // reference gradient of the cached nodal field (read plain: constrained
     // entries as stored), mf_nh_operator.h:873-877
     Number wg[3][3];
-    evaluate_g<N, 3, Number>(T, s_shape, s_colloc, w.v, wg);
+    evaluate_g<N, 3, Number, kRolled>(T, s_shape, s_colloc, w.v, wg);
     qop.attach(qd, wg);
   }
 
   Number val[NC], grad[NC][3];
-  evaluate_vg<N, NC, Number>(T, s_shape, s_colloc, u, val, grad);
+  evaluate_vg<N, NC, Number, kRolled>(T, s_shape, s_colloc, u, val, grad);
   apply_qop(qop, cd, qd, val, grad);
   Number out[NC];
-  integrate_vg<N, NC, Number, kSpareSlots>(T, s_shape, s_colloc, val, grad, out);
+  integrate_vg<N, NC, Number, kSpareSlots, kRolled>(T, s_shape, s_colloc, val, grad, out);
   if constexpr (kToCells) {
     if (active) store_node<Number, NC>(dst + (qb + lo) * NC, out);
     return;
