@@ -276,7 +276,9 @@ int32_t mfg_operator_n_colours(mfg_operator op);
  * summing every node's contributions in colour order -- bitwise the COLOURS
  * result, in two launches instead of one per colour (the default up to 2^20
  * quadrature points, where colour launches are latency bound); it holds
- * N_qp * n_components extra values. */
+ * N_qp * n_components extra values.  A multigrid hierarchy applies its level
+ * operators with GATHER up to 3 * 2^20 points (degrees 2, 3) or 5 * 2^20
+ * (above), unless a schedule was set here. */
 #define MFG_CELLS_COLOURS 0
 #define MFG_CELLS_GATHER 3
 int mfg_operator_set_cell_schedule(mfg_operator op, int32_t schedule);

@@ -617,7 +617,7 @@ struct BatchGather {
   struct Unit {
     int code = 0;  // kind * 8 + degree
     std::vector<int> inst;
-    DeviceBuffer tasks, segs, block_begin;
+    DeviceBuffer tasks, segs, gather_blocks;
     int n_tasks = 0;
     int64_t blocks = 0;
     double work = 0;
@@ -637,7 +637,10 @@ struct BatchGather {
     std::map<int, std::vector<int>> by_code;
     for (int i = 0; i < n; ++i) {
       OperatorData &op = *ops[i];
-      if (!op.contrib.ptr) op.build_gather();
+      if (!op.contrib.ptr) {
+        op.build_gather();
+        ++op.buffers_version;
+      }
       by_code[code_of(op)].push_back(i);
       total += apply_work(op);
     }
@@ -678,6 +681,13 @@ struct BatchGather {
       }
       u.n_tasks = (int)tv.size();
       upload_vec(u.tasks, tv, s);
+      std::vector<GatherBlock> gb;
+      for (size_t k = 0; k < u.inst.size(); ++k)
+        for (int64_t v = 0; v < ops[u.inst[k]]->n_nodes; v += kGatherThreads)
+          gb.push_back(GatherBlock{(int32_t)k, (int32_t)v});
+      MFG_REQUIRE(gb.size() < (size_t)INT32_MAX, MFG_ERR_ARGUMENT, "batch unit too large for one gather launch");
+      u.blocks = (int64_t)gb.size();
+      upload_vec(u.gather_blocks, gb, s);
       work.push_back(u.work);
     }
     pool.build(work, kBatchStreams);
@@ -695,34 +705,27 @@ struct BatchGather {
     std::vector<const void *> sv(src, src + n);
     std::vector<void *> dv(dst, dst + n);
     if (sv == last_src && dv == last_dst && vecs.ptr) return;
-    std::vector<BatchVecs<Number>> v(n);
+    std::vector<GatherVecs<Number>> v(n);
     for (size_t i = 0; i < n; ++i) {
       MFG_REQUIRE(src[i] && dst[i], MFG_ERR_ARGUMENT, "null vector");
       MFG_REQUIRE(src[i] != dst[i], MFG_ERR_ARGUMENT, "vmult needs distinct source and destination");
       v[i].src = (const Number *)src[i];
-      v[i].dst = ops[i]->contrib.as<Number>();
+      v[i].contrib = ops[i]->contrib.as<Number>();
+      v[i].slots = ops[i]->gather_slots();
     }
     upload_vec(vecs, v, s);
     for (Unit &u : units) {
       std::vector<GatherSeg<Number>> g;
-      std::vector<int64_t> bb(1, 0);  // first workgroup of every segment, and the grid size
       for (int i : u.inst) {
         const OperatorData &op = *ops[i];
         GatherSeg<Number> e;
-        e.contrib = op.contrib.as<Number>();
-        e.offsets = op.gather_offsets.as<int32_t>();
-        e.points = op.gather_points.as<int32_t>();
-        e.cmask = op.gather_cmask.as<uint8_t>();
+        e.tables = gather_tables<Number>(op);
         e.src = (const Number *)src[i];
         e.dst = (Number *)dst[i];
         e.n_nodes = op.n_nodes;
         g.push_back(e);
-        bb.push_back(bb.back() + (op.n_nodes + kGatherThreads - 1) / kGatherThreads);
       }
-      MFG_REQUIRE(bb.back() < INT32_MAX, MFG_ERR_ARGUMENT, "batch unit too large for one gather launch");
       upload_vec(u.segs, g, s);
-      upload_vec(u.block_begin, bb, s);
-      u.blocks = bb.back();
     }
     last_src = sv;
     last_dst = dv;
@@ -734,7 +737,7 @@ struct BatchGather {
     BatchCellsArgs<Number> a;
     a.inst = (const BatchInst<Number> *)inst_table;
     a.tasks = u.tasks.as<BatchTask>();
-    a.vecs = vecs.as<BatchVecs<Number>>();
+    a.vecs = vecs.as<GatherVecs<Number>>();
     batched_cells_kernel<P, CPB, KIND, Number><<<u.n_tasks, block_threads<P, CPB>(), 0, s>>>(a);
     MFG_HIP(hipGetLastError());
   }
@@ -765,13 +768,12 @@ struct BatchGather {
         case kSolidF0: launch_kind<kSolidF0, Number>(u, inst_table, us); break;
         default: launch_kind<kHeat, Number>(u, inst_table, us); break;
       }
-      const int n_segs = (int)u.inst.size();
       if (kind == kHeat)
         batched_gather_kernel<Number, 1><<<(unsigned)u.blocks, kGatherThreads, 0, us>>>(
-            u.segs.as<GatherSeg<Number>>(), u.block_begin.as<int64_t>(), n_segs, fix);
+            u.segs.as<GatherSeg<Number>>(), u.gather_blocks.as<GatherBlock>(), fix);
       else
         batched_gather_kernel<Number, 3><<<(unsigned)u.blocks, kGatherThreads, 0, us>>>(
-            u.segs.as<GatherSeg<Number>>(), u.block_begin.as<int64_t>(), n_segs, fix);
+            u.segs.as<GatherSeg<Number>>(), u.gather_blocks.as<GatherBlock>(), fix);
       MFG_HIP(hipGetLastError());
     });
   }

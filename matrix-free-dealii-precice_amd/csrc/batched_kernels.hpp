@@ -229,11 +229,19 @@ __device__ inline auto batch_qop(const BatchInst<Number> &in) {
   }
 }
 
+// per instance: src, the instance's contribution buffer and its slots there
+template <typename Number>
+struct GatherVecs {
+  const Number *src;
+  Number *contrib;
+  const uint32_t *slots;
+};
+
 template <typename Number>
 struct BatchCellsArgs {
   const BatchInst<Number> *inst;
-  const BatchTask *tasks;         // this launch's tasks: inst, cell_begin, cell_end
-  const BatchVecs<Number> *vecs;  // per instance: src and the instance's contribution buffer
+  const BatchTask *tasks;  // this launch's tasks: inst, cell_begin, cell_end
+  const GatherVecs<Number> *vecs;
 };
 
 template <int P, int CPB, int KIND, typename Number>
@@ -244,10 +252,10 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) batched_cells_kerne
   __shared__ Number s_tile[CPB * (kSpare ? 5 : 3) * NC * N3];
   const BatchTask tk = a.tasks[xcd_remap(blockIdx.x, gridDim.x)];
   const BatchInst<Number> in = a.inst[tk.inst];
-  const BatchVecs<Number> v = a.vecs[tk.inst];
+  const GatherVecs<Number> v = a.vecs[tk.inst];
   auto group = [&](auto q) {
-    cell_group<P, Number, decltype(q), true, kSpare>(q, in.cell_nodes, v.src, v.dst, tk.cell_begin, tk.cell_end, CPB,
-                                                     1, in.shape, in.colloc, s_shape, s_colloc, s_tile);
+    cell_group<P, Number, decltype(q), true, kSpare>(q, in.cell_nodes, v.src, v.contrib, tk.cell_begin, tk.cell_end, CPB,
+                                                     1, in.shape, in.colloc, s_shape, s_colloc, s_tile, v.slots);
   };
   if (KIND == kHeat && !in.cell_geo) group(batch_qop<KIND, CPB == 1, false>(in));
   else group(batch_qop<KIND, CPB == 1, true>(in));
@@ -255,34 +263,29 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) batched_cells_kerne
 
 template <typename Number>
 struct GatherSeg {
-  const Number *contrib;
-  const int32_t *offsets, *points;
-  const uint8_t *cmask;
+  GatherTables<Number> tables;
   const Number *src;
   Number *dst;
   int64_t n_nodes;
 };
 
-constexpr int kGatherThreads = 256;
+// One workgroup per kGatherThreads nodes of one instance (segment), taken from
+// a table: a binary search over the segments' first workgroups cost five
+// dependent loads before the first useful one.
+struct GatherBlock {
+  int32_t seg;
+  int32_t first_node;
+};
 
-// One workgroup per kGatherThreads nodes of one instance (segment);
-// block_begin[s] is segment s's first workgroup (n_segs + 1 entries, the last
-// one the grid size).
 template <typename Number, int NC>
 __global__ void __launch_bounds__(kGatherThreads)
-    batched_gather_kernel(const GatherSeg<Number> *__restrict__ segs, const int64_t *__restrict__ block_begin,
-                          int n_segs, int fix_mode) {
-  const int64_t blk = blockIdx.x;
-  int lo = 0, hi = n_segs - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (block_begin[mid] <= blk) lo = mid;
-    else hi = mid - 1;
-  }
-  const GatherSeg<Number> g = segs[lo];
-  const int64_t node = (blk - block_begin[lo]) * kGatherThreads + threadIdx.x;
+    batched_gather_kernel(const GatherSeg<Number> *__restrict__ segs, const GatherBlock *__restrict__ blocks,
+                          int fix_mode) {
+  const GatherBlock bl = blocks[blockIdx.x];
+  const GatherSeg<Number> g = segs[bl.seg];
+  const int64_t node = bl.first_node + (int64_t)threadIdx.x;
   if (node >= g.n_nodes) return;
-  gather_node<Number, NC>(g.contrib, g.offsets, g.points, g.cmask, g.src, g.dst, node, fix_mode);
+  gather_node<Number, NC>(g.tables, g.src, g.dst, node, fix_mode);
 }
 
 // --------------------------------------------------- segmented vectors ---

@@ -66,7 +66,8 @@ template <int P, typename Number, class QOp, bool kToCells>
 __device__ inline void cell_columns(const QOp &qop, const uint32_t *__restrict__ cell_nodes,
                                     const Number *__restrict__ src, Number *__restrict__ dst, int cell_begin,
                                     int cell_end, int assign, const Number *__restrict__ g_shape,
-                                    const Number *__restrict__ g_colloc, Number *lds) {
+                                    const Number *__restrict__ g_colloc, Number *lds,
+                                    const uint32_t *__restrict__ slots = nullptr) {
   constexpr int N = P + 1, NL = N * N, N3 = NL * N, NC = QOp::NC;
   Number *s_shape = lds, *s_colloc = lds + NL;
   const int t = threadIdx.x;
@@ -234,10 +235,15 @@ __device__ inline void cell_columns(const QOp &qop, const uint32_t *__restrict__
     rj[a] = s_shape[a * N + j];
   }
   put(0);
-  // dst of the thread's nodes, read while the last two contractions run; the
-  // first colour touching a node stores without reading
+  // dst of the thread's nodes (or the slots of its contributions), read while
+  // the last two contractions run; the first colour touching a node stores
+  // without reading
   Number dold[kToCells ? 1 : N][NC];
-  if constexpr (!kToCells) {
+  uint32_t slot[kToCells ? N : 1];
+  if constexpr (kToCells) {
+#pragma unroll
+    for (int k = 0; k < N; ++k) slot[k] = slots ? (slots + qb)[lo + k * NL] : (uint32_t)(qb + lo + k * NL);
+  } else {
 #pragma unroll
     for (int k = 0; k < N; ++k) {
       const bool first = assign && (entry[k] >> 31);
@@ -268,7 +274,7 @@ __device__ inline void cell_columns(const QOp &qop, const uint32_t *__restrict__
       for (int a = 0; a < N; ++a) r[c] += ri[a] * xl[(c * N + k) * NL + a];
     }
     if constexpr (kToCells) {
-      store_node<Number, NC>(dst + (qb + lo + k * NL) * NC, r);
+      store_node<Number, NC>(dst + (int64_t)slot[k] * NC, r);
     } else {
       Number *out = dst + (int64_t)(entry[k] & kNodeMaskDev) * NC;
 #pragma unroll
@@ -308,7 +314,7 @@ __global__ void __launch_bounds__(64)
   __shared__ Number lds[column_lds<P, QOp::NC>()];
   const int first_cell = a.cell_begin + xcd_remap(blockIdx.x, gridDim.x) * column_cells<P>();
   cell_columns<P, Number, QOp, true>(qop, a.cell_nodes, a.src, contrib, first_cell, a.cell_end, 1, a.shape, a.colloc,
-                                     lds);
+                                     lds, a.slots);
 }
 
 }  // namespace mfg

@@ -288,6 +288,8 @@ void TransferData::build(OperatorData *c, OperatorData *f, const int32_t *childr
 
 // ---------------------------------------------------- operator helpers ---
 static void op_vmult(const OperatorData &op, void *dst, const void *src) { op.apply(src, dst, false); }
+// the same for a multigrid level's operator
+static void level_vmult(const OperatorData &op, void *dst, const void *src) { op.apply_ordered(src, dst); }
 
 // Eigenvalues of the Lanczos tridiagonal matrix (bisection).
 static void tridiag_eigs(const std::vector<double> &dg, const std::vector<double> &off, double &lmin, double &lmax) {
@@ -373,7 +375,7 @@ void MGLevel::estimate_eigenvalues(int n_it, Reducer &red) {
   red.dot_dev(pr, cg_r.ptr, cg_r.ptr, n, kRedRes0, 0, s, 0.0, 1e-15);
   double sc[kRedScalars];
   for (int it = 0; it < n_it; ++it) {
-    op_vmult(A, cg_h.ptr, cg_p.ptr);
+    level_vmult(A, cg_h.ptr, cg_p.ptr);
     red.dot_dev(pr, cg_p.ptr, cg_h.ptr, n, kRedAlpha, 0, s, 0, 0, true);
     red.cg_update_dev(pr, sol.ptr, cg_r.ptr, cg_p.ptr, cg_h.ptr, n, kRedRRStop, s);
     if (it + 1 == n_it) break;
@@ -423,7 +425,7 @@ void MGLevel::chebyshev(void *x, const void *b, bool zero_guess) {
       cheb_first_kernel<float><<<grid_for(n), 256, 0, s>>>((float *)x, d.as<float>(), (const float *)b,
                                                            A.inv_diag.as<float>(), inv_theta, n);
   } else {
-    op_vmult(A, t.ptr, x);
+    level_vmult(A, t.ptr, x);
     if (A.precision == MFG_FP64)
       cheb_first_step_kernel<double><<<grid_for(n), 256, 0, s>>>((double *)x, d.as<double>(), (const double *)b,
                                                                  t.as<double>(), A.inv_diag.as<double>(), inv_theta, n);
@@ -436,7 +438,7 @@ void MGLevel::chebyshev(void *x, const void *b, bool zero_guess) {
   double rhok = delta / theta;
   const double sigma = theta / delta;
   for (int k = 0; k < degree - 1; ++k) {
-    op_vmult(A, t.ptr, x);
+    level_vmult(A, t.ptr, x);
     const double rhokp = 1.0 / (2.0 * sigma - rhok);
     const double f1 = rhokp * rhok, f2 = 2.0 * rhokp / delta;
     rhok = rhokp;
@@ -454,6 +456,7 @@ void MGLevel::chebyshev(void *x, const void *b, bool zero_guess) {
 void MGData::setup() {
   drop_graphs();  // new smoother coefficients
   for (auto &L : levels) {
+    L.op->prepare_gather();
     if (!L.op->has_diagonal) L.op->compute_diagonal();
     if (L.sol.bytes != (size_t)L.op->n_dofs * L.op->elem_size()) L.allocate();
   }
@@ -507,7 +510,7 @@ void MGData::coarse_solve() {
         red.dot_dev(pr, L.cg_r.ptr, L.cg_z.ptr, n, kRedBeta, 0, s);
         red.xpby_dev(pr, L.cg_p.ptr, L.cg_z.ptr, n, s);
       }
-      op_vmult(A, L.cg_h.ptr, L.cg_p.ptr);
+      level_vmult(A, L.cg_h.ptr, L.cg_p.ptr);
       red.dot_dev(pr, L.cg_p.ptr, L.cg_h.ptr, n, kRedAlpha, 0, s, 0, 0, true);
       red.cg_update_dev(pr, L.sol.ptr, L.cg_r.ptr, L.cg_p.ptr, L.cg_h.ptr, n, kRedRRStop, s);
     }
@@ -525,7 +528,7 @@ void MGData::down_sweep() {
     MGLevel &C = levels[l - 1];
     const OperatorData &A = *L.op;
     L.chebyshev(L.sol.ptr, L.def.ptr, true);  // pre-smoothing from a zero guess
-    op_vmult(A, L.tmp.ptr, L.sol.ptr);
+    level_vmult(A, L.tmp.ptr, L.sol.ptr);
     vec_residual(A.precision, L.tmp.ptr, L.def.ptr, A.n_dofs, A.stream);
     vec_fill(C.op->precision, C.def.ptr, C.op->n_dofs, 0.0, A.stream);
     transfers[l - 1]->restrict_add(C.def.ptr, L.tmp.ptr);

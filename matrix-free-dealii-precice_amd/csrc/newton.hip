@@ -229,13 +229,13 @@ size_t estimate_solid_problem_bytes(int n_levels, const mfg_level_desc *levels, 
     const int64_t nqp = (int64_t)d.n_cells * n3, ndof = d.n_nodes * d.n_components;
     const size_t es = (l == 0 || level_precision == MFG_FP64) ? 8 : 4;
     b += nqp * (18 * es + 4) + (size_t)d.n_cells * 24 * 8 + 11 * ndof * es;  // caches, map, vertices, diag + MG vectors
-    if (nqp <= kGatherMaxPoints) b += gather_bytes(nqp, d.n_nodes, d.n_components, es);
+    if (nqp <= gather_max_points(d.degree)) b += gather_bytes(nqp, d.n_nodes, d.n_components, es);
     if (l > 0) b += (size_t)levels[l - 1].n_cells * (2 * d.degree + 1) * (2 * d.degree + 1) * (2 * d.degree + 1) * 4;
     if (l == n_levels - 1) {
       b += 12 * ndof * 8;  // state, residual, CG workspace
       if (level_precision == MFG_FP32 && n_levels > 1) {
         b += nqp * (18 * 8 + 4) + (size_t)d.n_cells * 24 * 8 + 2 * ndof * 4;  // + FP32 condition-estimate vectors
-        if (nqp <= kGatherMaxPoints) b += gather_bytes(nqp, d.n_nodes, d.n_components, 8);
+        if (nqp <= gather_max_points(d.degree)) b += gather_bytes(nqp, d.n_nodes, d.n_components, 8);
       }
     }
   }
@@ -292,6 +292,9 @@ std::unique_ptr<SolidProblem> make_solid_problem(int n_levels, const mfg_level_d
     // folded 16 words, in FP64 and FP32)
     if (sp.formulation == 1 && sp.caching == MFG_CACHING_TENSOR2 && op->affine_ref) op->t2_storage = MFG_T2_GRADIENT;
     op->setup_solid();
+    // the problem's work is ordered on one stream
+    op->prepare_gather();
+    if (op->gather_ready) op->cell_schedule = MFG_CELLS_GATHER;
     return op;
   };
   for (int l = 0; l < n_levels; ++l) p->levels.push_back(make_op(levels[l], l == 0 ? MFG_FP64 : level_precision));

@@ -148,7 +148,8 @@ static void fill(Number *x, int64_t n, Number v, hipStream_t s) {
 
 // --------------------------------------------------------- dispatchers ---
 template <int P, typename Number>
-static void launch_apply(const OperatorData &op, const void *src, void *dst, int fix_mode, hipStream_t stream) {
+static void launch_apply(const OperatorData &op, const void *src, void *dst, int fix_mode, bool gather,
+                         hipStream_t stream) {
   constexpr int CPB = DefaultCPB<P, Number>::value;
   ApplyArgs<Number> a;
   a.cell_nodes = op.cell_nodes.as<uint32_t>();
@@ -158,9 +159,10 @@ static void launch_apply(const OperatorData &op, const void *src, void *dst, int
   a.colloc = op.tab_colloc.as<Number>();
   a.constrained = op.constrained.as<int32_t>();
   a.n_constrained = op.n_constrained;
+  a.slots = nullptr;
   constexpr int NT = block_threads<P, CPB>();
   const int assign = fix_mode == 1 ? 1 : 0;  // vmult: first touch stores, no zero fill
-  if (op.cell_schedule != MFG_CELLS_GATHER) {
+  if (!gather) {
     // one workgroup per group of CPB cells, one launch per colour (and
     // material); the first launch also writes the identity rows
     bool fix_pending = true;
@@ -190,6 +192,7 @@ static void launch_apply(const OperatorData &op, const void *src, void *dst, int
   // GATHER: all cells (of one material per launch) into the contribution
   // buffer, then the ordered per-node sums
   a.fix_mode = 0;
+  a.slots = op.gather_slots();
   auto cells = [&](int b, int e, int m) {
     a.cell_begin = b;
     a.cell_end = e;
@@ -212,9 +215,8 @@ static void launch_apply(const OperatorData &op, const void *src, void *dst, int
   const int64_t nn = op.n_nodes;
   auto sums = [&](auto nc_tag) {
     constexpr int NCv = decltype(nc_tag)::value;
-    gather_contributions<Number, NCv><<<(int)((nn + 255) / 256), 256, 0, stream>>>(
-        op.contrib.as<Number>(), op.gather_offsets.as<int32_t>(), op.gather_points.as<int32_t>(),
-        op.gather_cmask.as<uint8_t>(), (const Number *)src, (Number *)dst, nn, fix_mode);
+    gather_contributions<Number, NCv><<<blocks_for(nn, kGatherThreads), kGatherThreads, 0, stream>>>(
+        gather_tables<Number>(op), (const Number *)src, (Number *)dst, nn, fix_mode);
     MFG_HIP(hipGetLastError());
   };
   if (op.nc == 3) sums(std::integral_constant<int, 3>());
@@ -285,8 +287,9 @@ static void launch_diagonal(OperatorData &op) {
   }
 
 template <typename Number>
-static void apply_t(const OperatorData &op, const void *src, void *dst, int fix_mode, hipStream_t stream) {
-  MFG_DISPATCH_DEGREE(op.p, launch_apply, op, src, dst, fix_mode, stream);
+static void apply_t(const OperatorData &op, const void *src, void *dst, int fix_mode, bool gather,
+                    hipStream_t stream) {
+  MFG_DISPATCH_DEGREE(op.p, launch_apply, op, src, dst, fix_mode, gather, stream);
 }
 template <typename Number>
 static void cache_t(OperatorData &op, const void *u, int u_fp32, void *export_gradient = nullptr) {
@@ -297,17 +300,30 @@ static void diagonal_t(OperatorData &op) {
   MFG_DISPATCH_DEGREE(op.p, launch_diagonal, op);
 }
 
-void OperatorData::apply(const void *src, void *dst, bool add, hipStream_t on) const {
-  MFG_REQUIRE(ready, MFG_ERR_STATE, "operator used before cache()");
+static void apply_checked(const OperatorData &op, const void *src, void *dst, bool add, bool gather, hipStream_t s) {
+  MFG_REQUIRE(op.ready, MFG_ERR_STATE, "operator used before cache()");
   MFG_REQUIRE(src && dst, MFG_ERR_ARGUMENT, "null vector");
   // the scatter reads dst while other workgroups still gather src
   MFG_REQUIRE(src != dst, MFG_ERR_ARGUMENT, "dst and src must be different vectors");
-  const hipStream_t s = on ? on : stream;
   // vmult needs no zero fill: the first colour touching a node stores
-  timing_begin(s);
-  if (precision == MFG_FP64) apply_t<double>(*this, src, dst, add ? 2 : 1, s);
-  else apply_t<float>(*this, src, dst, add ? 2 : 1, s);
-  timing_end(s);
+  op.timing_begin(s);
+  if (op.precision == MFG_FP64) apply_t<double>(op, src, dst, add ? 2 : 1, gather, s);
+  else apply_t<float>(op, src, dst, add ? 2 : 1, gather, s);
+  op.timing_end(s);
+}
+
+void OperatorData::apply(const void *src, void *dst, bool add, hipStream_t on) const {
+  apply_checked(*this, src, dst, add, cell_schedule == MFG_CELLS_GATHER, on ? on : stream);
+}
+
+void OperatorData::apply_ordered(const void *src, void *dst) const {
+  apply_checked(*this, src, dst, false, gather_ordered(), stream);
+}
+
+void OperatorData::prepare_gather() {
+  if (schedule_set || nqp > gather_max_points(p)) return;
+  if (!contrib.ptr) build_gather();
+  gather_ready = true;
 }
 
 // Event pairs are reused; at most kMaxEvents launches are kept between
@@ -507,21 +523,26 @@ void OperatorData::colour_cells(const mfg_level_desc &d, int N3) {
 void OperatorData::build_gather() {
   MFG_REQUIRE(nqp < ((int64_t)1 << 31), MFG_ERR_ARGUMENT, "too many quadrature points for the GATHER tables");
   const int N3 = (p + 1) * (p + 1) * (p + 1);
-  std::vector<int32_t> offsets((size_t)n_nodes + 1, 0), points((size_t)nqp);
+  std::vector<int32_t> offsets((size_t)n_nodes + 1, 0);
+  std::vector<uint32_t> places((size_t)nqp);
+  // heat Q1 and Q2: reading through an index is the faster form (1M unknowns
+  // FP64, Q1 91 against 160 us, Q2 64 against 68; Q3 42 against 40, Q4 48
+  // against 34)
+  gather_indexed = nc == 1 && p <= 2;
   for (int64_t x = 0; x < nqp; ++x) offsets[host_cell_nodes[x] + 1]++;
   for (int64_t v = 0; v < n_nodes; ++v) offsets[v + 1] += offsets[v];
   std::vector<int32_t> fill(offsets.begin(), offsets.end() - 1);
   // stored (colour-major) cell order is the order of the colour launches
   for (int c = 0; c < n_cells; ++c)
     for (int pt = 0; pt < N3; ++pt) {
-      const int32_t node = host_cell_nodes[(int64_t)perm[c] * N3 + pt];
-      points[fill[node]++] = c * N3 + pt;
+      const uint32_t q = (uint32_t)c * N3 + pt, at = (uint32_t)fill[host_cell_nodes[(int64_t)perm[c] * N3 + pt]]++;
+      if (gather_indexed) places[at] = q;
+      else places[q] = at;
     }
   upload(gather_offsets, offsets.data(), offsets.size(), stream);
-  upload(gather_points, points.data(), points.size(), stream);
+  upload(gather_places, places.data(), places.size(), stream);
   upload(gather_cmask, host_cmask.data(), host_cmask.size(), stream);
   contrib.allocate((size_t)nqp * nc * elem_size());
-  ++buffers_version;
 }
 
 void OperatorData::setup_layout(const mfg_level_desc &d) {
@@ -624,9 +645,6 @@ void OperatorData::setup_layout(const mfg_level_desc &d) {
   const Tables1D t = make_tables(p);
   if (precision == MFG_FP64) upload_tables<double>(*this, t);
   else upload_tables<float>(*this, t);
-  // small operators: their colour launches are bound by one workgroup's
-  // critical path each, so the two launches of GATHER are faster (measured on
-  // the beam's MG levels up to 256K points; equal at 2M, slower at 16M)
   if (nqp <= kGatherMaxPoints) {
     build_gather();
     cell_schedule = MFG_CELLS_GATHER;
@@ -766,7 +784,7 @@ void OperatorData::setup_solid() {
 
 size_t OperatorData::memory_consumption() const {
   return qd.bytes + cell_nodes.bytes + constrained.bytes + u_nodal.bytes + cell_jxw.bytes + wq3.bytes + cell_geo.bytes + cell_met.bytes +
-         gather_offsets.bytes + gather_points.bytes + gather_cmask.bytes + contrib.bytes;
+         gather_offsets.bytes + gather_places.bytes + gather_cmask.bytes + contrib.bytes;
 }
 
 }  // namespace mfg
@@ -970,6 +988,7 @@ int mfg_operator_set_cell_schedule(mfg_operator op, int32_t schedule) {
     MFG_REQUIRE(schedule == MFG_CELLS_COLOURS || schedule == MFG_CELLS_GATHER, MFG_ERR_ARGUMENT,
                 "unknown cell schedule");
     op->cell_schedule = MFG_CELLS_COLOURS;
+    op->schedule_set = true;
     if (schedule == MFG_CELLS_GATHER) {
       if (!op->contrib.ptr) op->build_gather();
       op->cell_schedule = schedule;

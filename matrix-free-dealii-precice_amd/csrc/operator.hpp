@@ -4,9 +4,24 @@
 
 namespace mfg {
 
-// operators with at most this many quadrature points use the GATHER cell
-// schedule unless another is set
+// Operators with at most this many quadrature points use the GATHER schedule by
+// default: two launches over all cells against 8 of one colour each, whose
+// cells alone do not fill the GPU.  The contribution buffer is one per
+// operator, so a larger default would add a buffer that two applications on
+// different streams (set_stream in between) share.
 constexpr int64_t kGatherMaxPoints = 1 << 20;
+// Where the operator's work is ordered on one stream (multigrid levels, the
+// operators of a SolidProblem), GATHER serves up to this many points.  Past it
+// the colours' plain read-modify-write moves less than the contributions'
+// store and load.  Measured, time of colours / gather on cubes: solid Q1 1.3
+// at 0.55M points, 0.77 at 2.6M; Q2 1.23 at 1.2M, 1.02 at 3.4M, 0.84 at 6.8M;
+// Q3 1.47 at 0.9M, 1.07 at 2.3M, 0.94 at 4.7M; Q4 1.55 at 0.6M, 1.07 at 3.7M,
+// 0.88 at 8M (FP32 1.00); Q5 1.10 at 3.4M; Q6 1.39 at 3.2M, 1.15 at 6M; heat
+// Q2 0.96 at 3.4M (FP32 1.40), Q3 1.22 at 2.3M, Q4 1.04 at 5.8M, Q6 1.31 at
+// 4.7M.
+constexpr int64_t gather_max_points(int p) {
+  return p == 1 ? kGatherMaxPoints : p <= 3 ? 3 * kGatherMaxPoints : 5 * kGatherMaxPoints;
+}
 
 // device bytes of the GATHER schedule's tables and contribution buffer
 inline size_t gather_bytes(int64_t nqp, int64_t n_nodes, int nc, size_t es) {
@@ -76,11 +91,24 @@ struct OperatorData {
   // bumped whenever a device buffer that apply() reads is reallocated (graphs
   // that captured the old addresses must be re-captured)
   uint64_t buffers_version = 0;
-  // GATHER schedule: per node, the points (stored cell * N3 + point) that
-  // touch it in colour order (CSR), its constrained components, and the
-  // per-point contribution buffer
-  DeviceBuffer gather_offsets, gather_points, gather_cmask, contrib;
+  // GATHER schedule: node v's contributions in colour order are entries
+  // gather_offsets[v] .. gather_offsets[v + 1] of contrib, or (gather_indexed)
+  // of the points listed in gather_places, contrib being in point order;
+  // otherwise gather_places holds the place of every (stored cell, point).
+  // cmask: the node's constrained components.
+  DeviceBuffer gather_offsets, gather_places, gather_cmask, contrib;
+  bool gather_indexed = false;
+  const uint32_t *gather_slots() const { return gather_indexed ? nullptr : gather_places.as<uint32_t>(); }
   void build_gather();
+  // The schedule was set through mfg_operator_set_cell_schedule: every
+  // application keeps it.
+  bool schedule_set = false;
+  // Up to gather_max_points() a multigrid hierarchy (whose work, like its level
+  // vectors, is ordered on one stream) applies its level operators with GATHER
+  // whatever their default: prepare_gather() in its setup, apply_ordered() then.
+  void prepare_gather();
+  bool gather_ordered() const { return cell_schedule == MFG_CELLS_GATHER || (!schedule_set && gather_ready); }
+  bool gather_ready = false;
   // optional cell-kernel timing
   bool timing = false;
   mutable std::vector<std::pair<hipEvent_t, hipEvent_t>> events;
@@ -94,6 +122,8 @@ struct OperatorData {
   void export_qp_gradient(DeviceBuffer &out);
   // dst (+)= A src on `on` (the operator's stream when null)
   void apply(const void *src, void *dst, bool add, hipStream_t on = nullptr) const;
+  // dst = A src for callers that order all of the operator's work on its stream
+  void apply_ordered(const void *src, void *dst) const;
   void compute_diagonal();
   size_t memory_consumption() const;
   size_t elem_size() const { return precision == MFG_FP64 ? 8 : 4; }
