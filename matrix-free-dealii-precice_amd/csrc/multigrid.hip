@@ -180,6 +180,8 @@ static void transfer_launch(TransferData &t, int kind, void *fine, const void *c
   a.coarse_out = (CN *)coarse_out;
   a.fine_in = (const FN *)fine_in;
   a.fine_out = (FN *)fine;
+  a.contrib = nullptr;
+  a.slots = nullptr;
   hipStream_t s = C.stream;
   if (kind == 0) {  // prolongate_add: every fine node written once by its owner
     a.E = t.E.as<double>();
@@ -194,6 +196,17 @@ static void transfer_launch(TransferData &t, int kind, void *fine, const void *c
       if (a.cell_end > a.cell_begin)
         restrict_add_kernel<P, NC, CN, FN><<<a.cell_end - a.cell_begin, 256, 0, s>>>(a);
     }
+  } else if (kind == 3) {  // restrict_set: all coarse cells, then the sums per node
+    a.E = t.E.as<double>();
+    a.cell_begin = 0;
+    a.cell_end = C.n_cells;
+    a.contrib = t.contrib.as<double>();
+    a.slots = C.gather_slots();
+    restrict_to_cells_kernel<P, NC, CN, FN><<<C.n_cells, 256, 0, s>>>(a);
+    GatherTables<double> g{t.contrib.as<double>(), C.gather_offsets.as<int32_t>(),
+                           C.gather_indexed ? C.gather_places.as<uint32_t>() : nullptr, C.gather_cmask.as<uint8_t>()};
+    restrict_sums_kernel<CN, NC>
+        <<<blocks_for(C.n_nodes, kGatherThreads), kGatherThreads, 0, s>>>(g, a.coarse_out, C.n_nodes);
   } else {
     a.E = t.I.as<double>();
     a.cell_begin = 0;
@@ -232,6 +245,18 @@ void TransferData::run(int kind, void *fine, const void *coarse_in, void *coarse
 void TransferData::prolongate_add(void *fine, const void *coarse) { run(0, fine, coarse, nullptr, nullptr); }
 void TransferData::restrict_add(void *coarse, const void *fine) { run(1, nullptr, nullptr, coarse, fine); }
 void TransferData::interpolate(void *coarse, const void *fine) { run(2, nullptr, nullptr, coarse, fine); }
+void TransferData::prepare_restrict() {
+  // where the coarse operator has the tables of its nodes' points
+  if (coarse->gather_places.ptr && !contrib.ptr) contrib.allocate((size_t)coarse->nqp * nc * sizeof(double));
+}
+void TransferData::restrict_set(void *out, const void *fine_in) {
+  if (contrib.ptr) {
+    run(3, nullptr, nullptr, out, fine_in);
+    return;
+  }
+  vec_fill(coarse->precision, out, coarse->n_dofs, 0.0, coarse->stream);
+  restrict_add(out, fine_in);
+}
 
 void TransferData::build(OperatorData *c, OperatorData *f, const int32_t *children) {
   MFG_REQUIRE(c && f && children, MFG_ERR_ARGUMENT, "null argument");
@@ -424,6 +449,8 @@ void MGLevel::chebyshev(void *x, const void *b, bool zero_guess) {
     else
       cheb_first_kernel<float><<<grid_for(n), 256, 0, s>>>((float *)x, d.as<float>(), (const float *)b,
                                                            A.inv_diag.as<float>(), inv_theta, n);
+  } else if (A.gather_ordered()) {
+    A.apply_epilogue(x, EpilogueArgs{kEpiChebFirstStep, b, nullptr, d.ptr, inv_theta, 0.0});
   } else {
     level_vmult(A, t.ptr, x);
     if (A.precision == MFG_FP64)
@@ -438,10 +465,14 @@ void MGLevel::chebyshev(void *x, const void *b, bool zero_guess) {
   double rhok = delta / theta;
   const double sigma = theta / delta;
   for (int k = 0; k < degree - 1; ++k) {
-    level_vmult(A, t.ptr, x);
     const double rhokp = 1.0 / (2.0 * sigma - rhok);
     const double f1 = rhokp * rhok, f2 = 2.0 * rhokp / delta;
     rhok = rhokp;
+    if (A.gather_ordered()) {
+      A.apply_epilogue(x, EpilogueArgs{kEpiChebUpdate, b, nullptr, d.ptr, f1, f2});
+      continue;
+    }
+    level_vmult(A, t.ptr, x);
     if (A.precision == MFG_FP64)
       cheb_update_kernel<double><<<grid_for(n), 256, 0, s>>>((double *)x, d.as<double>(), (const double *)b,
                                                              t.as<double>(), A.inv_diag.as<double>(), f1, f2, n);
@@ -473,6 +504,7 @@ void MGData::setup() {
       L.setup_chebyshev(prm.cheb_degree, prm.smoothing_range, prm.eig_cg_iterations, red);
     }
   }
+  for (TransferData *t : transfers) t->prepare_restrict();
   ready = true;
 }
 
@@ -481,15 +513,15 @@ void MGData::setup() {
 void MGData::coarse_solve() {
   MGLevel &L = levels[0];
   if (coarse_kind() == 0) {
-    L.chebyshev(L.sol.ptr, L.def.ptr, true);
+    L.chebyshev(L.x, L.b, true);
     return;
   }
   const OperatorData &A = *L.op;
   const int64_t n = A.n_dofs;
   const int pr = A.precision;
   hipStream_t s = A.stream;
-  vec_fill(pr, L.sol.ptr, n, 0.0, s);
-  vec_convert(pr, L.cg_r.ptr, pr, L.def.ptr, n, s);
+  vec_fill(pr, L.x, n, 0.0, s);
+  vec_convert(pr, L.cg_r.ptr, pr, L.b, n, s);
   // The step lengths and the stop test (||r|| <= max(1e-10, coarse_tolerance
   // ||r_0||), or a breakdown) stay on the device: once the stop flag is set,
   // the remaining iterations change neither sol nor r.  The host reads the
@@ -512,7 +544,7 @@ void MGData::coarse_solve() {
       }
       level_vmult(A, L.cg_h.ptr, L.cg_p.ptr);
       red.dot_dev(pr, L.cg_p.ptr, L.cg_h.ptr, n, kRedAlpha, 0, s, 0, 0, true);
-      red.cg_update_dev(pr, L.sol.ptr, L.cg_r.ptr, L.cg_p.ptr, L.cg_h.ptr, n, kRedRRStop, s);
+      red.cg_update_dev(pr, L.x, L.cg_r.ptr, L.cg_p.ptr, L.cg_h.ptr, n, kRedRRStop, s);
     }
     red.read(sc, s);
     if (sc[kSlotStop] != 0 || it >= maxit) break;
@@ -527,11 +559,14 @@ void MGData::down_sweep() {
     MGLevel &L = levels[l];
     MGLevel &C = levels[l - 1];
     const OperatorData &A = *L.op;
-    L.chebyshev(L.sol.ptr, L.def.ptr, true);  // pre-smoothing from a zero guess
-    level_vmult(A, L.tmp.ptr, L.sol.ptr);
-    vec_residual(A.precision, L.tmp.ptr, L.def.ptr, A.n_dofs, A.stream);
-    vec_fill(C.op->precision, C.def.ptr, C.op->n_dofs, 0.0, A.stream);
-    transfers[l - 1]->restrict_add(C.def.ptr, L.tmp.ptr);
+    L.chebyshev(L.x, L.b, true);  // pre-smoothing from a zero guess
+    if (A.gather_ordered()) {
+      A.apply_epilogue(L.x, EpilogueArgs{kEpiResidual, L.b, L.tmp.ptr, nullptr, 0.0, 0.0});
+    } else {
+      level_vmult(A, L.tmp.ptr, L.x);
+      vec_residual(A.precision, L.tmp.ptr, L.b, A.n_dofs, A.stream);
+    }
+    transfers[l - 1]->restrict_set(C.def.ptr, L.tmp.ptr);
   }
 }
 
@@ -539,9 +574,18 @@ void MGData::up_sweep() {
   for (int l = 1; l < (int)levels.size(); ++l) {
     MGLevel &L = levels[l];
     MGLevel &C = levels[l - 1];
-    transfers[l - 1]->prolongate_add(L.sol.ptr, C.sol.ptr);
-    L.chebyshev(L.sol.ptr, L.def.ptr, false);  // post-smoothing
+    transfers[l - 1]->prolongate_add(L.x, C.x);
+    L.chebyshev(L.x, L.b, false);  // post-smoothing
   }
+}
+
+void MGData::set_vectors(void *x, const void *b) {
+  for (MGLevel &L : levels) {
+    L.x = L.sol.ptr;
+    L.b = L.def.ptr;
+  }
+  levels.back().x = x;
+  levels.back().b = b;
 }
 
 bool MGData::graphs_allowed() const {
@@ -632,21 +676,33 @@ void MGData::run_graphed(hipStream_t caller) {
 
 // Multigrid::level_v_step from the finest level: the down sweep, the coarse
 // solve and the up sweep (the same launches the graphs replay)
-void MGData::v_cycle() {
+void MGData::v_cycle(void *x, const void *b) {
+  set_vectors(x, b);
   down_sweep();
   coarse_solve();
   up_sweep();
 }
 
-// PreconditionMG::vmult: copy_to_mg, V-cycle, copy_from_mg
+// PreconditionMG::vmult: copy_to_mg, V-cycle, copy_from_mg.  The copies are
+// left out where the caller's vectors can stand for the finest level's own: of
+// its precision, distinct, and not held by a captured graph.
 void MGData::vmult(void *dst, const void *src, int vec_prec) {
   MFG_REQUIRE(ready, MFG_ERR_STATE, "mfg_mg_setup() not called");
   MGLevel &F = levels.back();
   const int64_t n = F.op->n_dofs;
   hipStream_t caller = F.op->stream;
+  const bool graphed = graphs_allowed() && ++graph_calls >= 2;
+  if (!graphed && vec_prec == F.op->precision && dst != src) {
+    v_cycle(dst, src);
+    return;
+  }
   vec_convert(F.op->precision, F.def.ptr, vec_prec, src, n, caller);
-  if (graphs_allowed() && ++graph_calls >= 2) run_graphed(caller);
-  else v_cycle();
+  if (graphed) {
+    set_vectors(F.sol.ptr, F.def.ptr);
+    run_graphed(caller);
+  } else {
+    v_cycle(F.sol.ptr, F.def.ptr);
+  }
   vec_convert(vec_prec, dst, F.op->precision, F.sol.ptr, n, caller);
 }
 

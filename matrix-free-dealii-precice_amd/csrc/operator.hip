@@ -149,7 +149,7 @@ static void fill(Number *x, int64_t n, Number v, hipStream_t s) {
 // --------------------------------------------------------- dispatchers ---
 template <int P, typename Number>
 static void launch_apply(const OperatorData &op, const void *src, void *dst, int fix_mode, bool gather,
-                         hipStream_t stream) {
+                         const EpilogueArgs *epi, hipStream_t stream) {
   constexpr int CPB = DefaultCPB<P, Number>::value;
   ApplyArgs<Number> a;
   a.cell_nodes = op.cell_nodes.as<uint32_t>();
@@ -213,10 +213,23 @@ static void launch_apply(const OperatorData &op, const void *src, void *dst, int
   if (op.has_inclusion()) op.for_each_range([&](int, int b, int e, int m) { cells(b, e, m); });
   else cells(0, op.n_cells, 0);
   const int64_t nn = op.n_nodes;
+  const int blocks = blocks_for(nn, kGatherThreads);
   auto sums = [&](auto nc_tag) {
     constexpr int NCv = decltype(nc_tag)::value;
-    gather_contributions<Number, NCv><<<blocks_for(nn, kGatherThreads), kGatherThreads, 0, stream>>>(
-        gather_tables<Number>(op), (const Number *)src, (Number *)dst, nn, fix_mode);
+    const GatherTables<Number> g = gather_tables<Number>(op);
+    if (!epi) {
+      gather_contributions<Number, NCv>
+          <<<blocks, kGatherThreads, 0, stream>>>(g, (const Number *)src, (Number *)dst, nn, fix_mode);
+    } else {
+      auto fused = [&](auto kind_tag) {
+        gather_epilogue<Number, NCv, decltype(kind_tag)::value><<<blocks, kGatherThreads, 0, stream>>>(
+            g, (Number *)dst, (const Number *)epi->b, op.inv_diag.as<Number>(), (Number *)epi->d, (Number *)epi->out,
+            epi->s0, epi->s1, nn);
+      };
+      if (epi->kind == kEpiResidual) fused(std::integral_constant<int, kEpiResidual>());
+      else if (epi->kind == kEpiChebFirstStep) fused(std::integral_constant<int, kEpiChebFirstStep>());
+      else fused(std::integral_constant<int, kEpiChebUpdate>());
+    }
     MFG_HIP(hipGetLastError());
   };
   if (op.nc == 3) sums(std::integral_constant<int, 3>());
@@ -288,8 +301,8 @@ static void launch_diagonal(OperatorData &op) {
 
 template <typename Number>
 static void apply_t(const OperatorData &op, const void *src, void *dst, int fix_mode, bool gather,
-                    hipStream_t stream) {
-  MFG_DISPATCH_DEGREE(op.p, launch_apply, op, src, dst, fix_mode, gather, stream);
+                    const EpilogueArgs *epi, hipStream_t stream) {
+  MFG_DISPATCH_DEGREE(op.p, launch_apply, op, src, dst, fix_mode, gather, epi, stream);
 }
 template <typename Number>
 static void cache_t(OperatorData &op, const void *u, int u_fp32, void *export_gradient = nullptr) {
@@ -307,8 +320,8 @@ static void apply_checked(const OperatorData &op, const void *src, void *dst, bo
   MFG_REQUIRE(src != dst, MFG_ERR_ARGUMENT, "dst and src must be different vectors");
   // vmult needs no zero fill: the first colour touching a node stores
   op.timing_begin(s);
-  if (op.precision == MFG_FP64) apply_t<double>(op, src, dst, add ? 2 : 1, gather, s);
-  else apply_t<float>(op, src, dst, add ? 2 : 1, gather, s);
+  if (op.precision == MFG_FP64) apply_t<double>(op, src, dst, add ? 2 : 1, gather, nullptr, s);
+  else apply_t<float>(op, src, dst, add ? 2 : 1, gather, nullptr, s);
   op.timing_end(s);
 }
 
@@ -318,6 +331,14 @@ void OperatorData::apply(const void *src, void *dst, bool add, hipStream_t on) c
 
 void OperatorData::apply_ordered(const void *src, void *dst) const {
   apply_checked(*this, src, dst, false, gather_ordered(), stream);
+}
+
+void OperatorData::apply_epilogue(void *x, const EpilogueArgs &e) const {
+  MFG_REQUIRE(ready && gather_ordered(), MFG_ERR_STATE, "epilogue without the GATHER schedule");
+  timing_begin(stream);
+  if (precision == MFG_FP64) apply_t<double>(*this, x, x, 1, true, &e, stream);
+  else apply_t<float>(*this, x, x, 1, true, &e, stream);
+  timing_end(stream);
 }
 
 void OperatorData::prepare_gather() {

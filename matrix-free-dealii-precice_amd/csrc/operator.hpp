@@ -28,6 +28,21 @@ inline size_t gather_bytes(int64_t nqp, int64_t n_nodes, int nc, size_t es) {
   return (size_t)nqp * (nc * es + 4) + (size_t)(n_nodes + 1) * 4 + (size_t)n_nodes;
 }
 
+// What the per-node sums of a GATHER application do with a row t of A x
+// besides storing it: the pass that would follow over the same vectors.
+enum GatherEpilogue : int {
+  kEpiResidual = 0,   // out = b - t
+  kEpiChebFirstStep,  // d = D^{-1} (b - t) s0; x += d
+  kEpiChebUpdate,     // d = s0 d + s1 D^{-1} (b - t); x += d
+};
+struct EpilogueArgs {
+  int kind;
+  const void *b;
+  void *out;  // residual
+  void *d;    // Chebyshev direction
+  double s0, s1;
+};
+
 struct OperatorData {
   int kind = 0;  // 0 solid (NeoHookOperator), 1 heat (LaplaceOperator)
   int precision = MFG_FP64;
@@ -124,6 +139,8 @@ struct OperatorData {
   void apply(const void *src, void *dst, bool add, hipStream_t on = nullptr) const;
   // dst = A src for callers that order all of the operator's work on its stream
   void apply_ordered(const void *src, void *dst) const;
+  // where gather_ordered(): A x into the epilogue (the Chebyshev ones update x)
+  void apply_epilogue(void *x, const EpilogueArgs &e) const;
   void compute_diagonal();
   size_t memory_consumption() const;
   size_t elem_size() const { return precision == MFG_FP64 ? 8 : 4; }

@@ -57,10 +57,15 @@ struct TransferData {
   int p = 1, nc = 1;
   DeviceBuffer lattice;  // (2p+1)^3 entries per coarse cell (stored order)
   DeviceBuffer E, I;     // embedding (2p+1)x(p+1), interpolation (p+1)x(2p+1)
+  DeviceBuffer contrib;  // restrict_set: the coarse cells' parts
   void build(OperatorData *c, OperatorData *f, const int32_t *children);
   void prolongate_add(void *fine, const void *coarse);
   void restrict_add(void *coarse, const void *fine);
   void interpolate(void *coarse, const void *fine);
+  // coarse = P^T fine for callers that order all of the transfer's work on one
+  // stream (a multigrid hierarchy; prepare_restrict in its setup)
+  void prepare_restrict();
+  void restrict_set(void *coarse, const void *fine);
 
  private:
   void run(int kind, void *fine, const void *coarse_in, void *coarse_out, const void *fine_in);
@@ -69,6 +74,10 @@ struct TransferData {
 struct MGLevel {
   OperatorData *op = nullptr;
   DeviceBuffer sol, def, tmp, d, t, cg_r, cg_p, cg_h, cg_z;
+  // the solution and right-hand side of the running V-cycle: sol and def, or on
+  // the finest level the caller's vectors
+  void *x = nullptr;
+  const void *b = nullptr;
   int degree = 5;
   double theta = 1, delta = 0, lmin = 0, lmax = 0;
   void allocate();
@@ -92,7 +101,9 @@ struct MGData {
   int coarse_iterations = 0;
   void setup();
   void vmult(void *dst, const void *src, int vec_prec);
-  void v_cycle();
+  // the V-cycle on the finest level's vectors x (out) and b
+  void v_cycle(void *x, const void *b);
+  void set_vectors(void *x, const void *b);
   void coarse_solve();
   // Multigrid::level_v_step unrolled: pre-smoothing, residual and restriction
   // from the finest level down to level 1, then (after the coarse solve)

@@ -257,3 +257,34 @@ def test_coarse_cg_results_independent_of_history(cuda):
     assert torch.isfinite(outs[0]).all() and torch.isfinite(outs[1]).all()
     assert torch.equal(outs[0], outs[2]) and torch.equal(outs[0], outs[4]) and torch.equal(outs[0], first)
     assert torch.equal(outs[1], outs[3])
+
+
+@pytest.mark.parametrize("kind,p,n,precision", [
+    ("solid", 1, (4, 6, 2), mfgpu.FP64), ("solid", 2, (6, 4, 4), mfgpu.FP32), ("solid", 4, (4, 4, 2), mfgpu.FP64),
+    ("solid", 5, (2, 4, 2), mfgpu.FP32), ("solid", 6, (4, 2, 2), mfgpu.FP64), ("heat", 1, (8, 6, 4), mfgpu.FP64),
+    ("heat", 2, (6, 6, 2), mfgpu.FP32), ("heat", 3, (4, 4, 4), mfgpu.FP64), ("heat", 6, (4, 2, 2), mfgpu.FP32)])
+def test_vcycle_gather_equals_colours(cuda, kind, p, n, precision):
+    """The V-cycle with the smoother's updates and the residual inside the
+    per-node sums, the restriction in two launches and the caller's vectors as
+    the finest level's is bitwise the one of colour launches, separate vector
+    passes and copies; so it is from another precision, and in place."""
+    print(f"V-cycle gather = colours {kind} p={p} precision={precision}", flush=True)
+    out = {}
+    for sched in (None, mfgpu.CELLS_COLOURS):
+        inst = mfgpu.Instance(kind, n, p, level_precision=precision, seed=3, cell_schedule=sched,
+                              coarse_eig_iterations=40)
+        dt = inst.levels[-1].dtype
+        x = mfgpu.fill_uniform(11, torch.empty(inst.n_dofs, dtype=dt, device="cuda"))
+        y = torch.full_like(x, float("nan"))
+        keep = x.clone()
+        inst.mg.vmult(y, x)
+        other = torch.float32 if dt == torch.float64 else torch.float64
+        z = torch.empty(inst.n_dofs, dtype=other, device="cuda")
+        inst.mg.vmult(z, x.to(other))
+        w = x.clone()  # in place, through the C interface
+        mfgpu.check(mfgpu.lib().mfg_mg_vmult(inst.mg.h, mfgpu._ptr(w), mfgpu._ptr(w),
+                                             mfgpu.FP64 if dt == torch.float64 else mfgpu.FP32))
+        assert torch.equal(x, keep) and torch.isfinite(y).all() and torch.equal(w, y)
+        out[sched] = (y, z)
+    a, b = out[None], out[mfgpu.CELLS_COLOURS]
+    assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
