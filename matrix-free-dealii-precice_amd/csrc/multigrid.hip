@@ -78,8 +78,30 @@ void Reducer::jacobi_dot_dev(int prec, void *z, const void *invD, const void *r,
   epilogue(mode, 0, 0, 0, record, s);
 }
 
-void Reducer::repeat_epilogue(int mode, int slot, hipStream_t s, double tol, double rel, bool record) {
-  epilogue(mode, slot, tol, rel, record, s);
+template <typename T, bool kJacobi>
+static void fixed_iteration_t(Reducer &red, T *x, T *r, T *p, const T *h, const T *invD, int64_t n, bool last,
+                              hipStream_t s) {
+  // workgroups past the end of the vectors would only add zeros to the sums
+  const int grid = (int)std::min<int64_t>(kRedBlocks, (n + kRedThreads - 1) / kRedThreads);
+  double *rr = red.fixed_buf.as<double>(), *other = rr + 2 * kRedBlocks;
+  dot_partial_kernel<T><<<grid, kRedThreads, 0, s>>>(p, h, n, red.partials);
+  cg_step_kernel<T, kJacobi><<<grid, kRedThreads, 0, s>>>(x, r, p, h, invD, red.partials, grid, red.scal, other,
+                                                          red.hist_buf.as<double>(), red.hist_cap, n, rr);
+  cg_direction_kernel<T, kJacobi><<<last ? 1 : grid_for(n), kRedThreads, 0, s>>>(
+      p, r, invD, rr, grid, other, red.scal, red.hist_buf.as<double>(), red.hist_cap, n, last ? 1 : 0);
+  MFG_HIP(hipGetLastError());
+}
+
+void Reducer::fixed_iteration(int prec, void *x, void *r, void *p, const void *h, const void *invD, int64_t n,
+                              bool last, hipStream_t s) {
+  if (!fixed_buf.ptr) fixed_buf.allocate((2 * kRedBlocks + kRedScalars) * sizeof(double));
+  auto run = [&](auto tag) {
+    using T = decltype(tag);
+    if (invD) fixed_iteration_t<T, true>(*this, (T *)x, (T *)r, (T *)p, (const T *)h, (const T *)invD, n, last, s);
+    else fixed_iteration_t<T, false>(*this, (T *)x, (T *)r, (T *)p, (const T *)h, nullptr, n, last, s);
+  };
+  if (prec == MFG_FP64) run(double());
+  else run(float());
 }
 
 void Reducer::read(double *out, hipStream_t s) {
@@ -401,11 +423,8 @@ void MGLevel::estimate_eigenvalues(int n_it, Reducer &red) {
   double sc[kRedScalars];
   for (int it = 0; it < n_it; ++it) {
     level_vmult(A, cg_h.ptr, cg_p.ptr);
-    red.dot_dev(pr, cg_p.ptr, cg_h.ptr, n, kRedAlpha, 0, s, 0, 0, true);
-    red.cg_update_dev(pr, sol.ptr, cg_r.ptr, cg_p.ptr, cg_h.ptr, n, kRedRRStop, s);
+    red.fixed_iteration(pr, sol.ptr, cg_r.ptr, cg_p.ptr, cg_h.ptr, A.inv_diag.ptr, n, it + 1 == n_it, s);
     if (it + 1 == n_it) break;
-    red.jacobi_dot_dev(pr, cg_z.ptr, A.inv_diag.ptr, cg_r.ptr, 1.0, n, kRedBeta, s, true);
-    red.xpby_dev(pr, cg_p.ptr, cg_z.ptr, n, s);
     if (n_it > 32 && (it + 1) % 16 == 0) {
       red.read(sc, s);
       if (sc[kSlotStop] != 0) break;
@@ -793,12 +812,7 @@ double cg_condition_estimate(const OperatorData &A, const void *b, void *x, int 
   red.dot_dev(pr, v.r, v.r, n, kRedRes0, 0, s, tol, 0.0);
   for (int it = 0; it < n_it; ++it) {
     op_vmult(A, v.h, v.p);
-    red.dot_dev(pr, v.p, v.h, n, kRedAlpha, 0, s, 0, 0, true);
-    red.cg_update_dev(pr, x, v.r, v.p, v.h, n, kRedRRStop, s);
-    if (it + 1 == n_it) break;
-    // (r, r) of the new iterate: the update's partial sums again
-    red.repeat_epilogue(kRedBeta, 0, s, 0, 0, true);
-    red.xpby_dev(pr, v.p, v.r, n, s);
+    red.fixed_iteration(pr, x, v.r, v.p, v.h, nullptr, n, it + 1 == n_it, s);
   }
   double sc[kRedScalars];
   red.read(sc, s);

@@ -12,6 +12,7 @@ namespace mfg {
 struct Reducer {
   DeviceBuffer own;            // partials and scalars, when the reducer allocates them
   DeviceBuffer hist_buf;       // step lengths of fixed-count runs (alphas, then betas)
+  DeviceBuffer fixed_buf;      // fixed-count runs: 2 kRedBlocks partials and the other copy of the scalar block
   double *partials = nullptr;  // kRedBlocks
   double *scal = nullptr;      // kRedScalars
   int hist_cap = 0;
@@ -31,9 +32,11 @@ struct Reducer {
   // z = omega D^{-1} r, and r.z through `mode` (one pass over the vectors)
   void jacobi_dot_dev(int prec, void *z, const void *invD, const void *r, double omega, int64_t n, int mode,
                       hipStream_t s, bool record = false);
-  // the partial sums of the last reduction through another epilogue (a second
-  // dot product of the same vectors, without reading them again)
-  void repeat_epilogue(int mode, int slot, hipStream_t s, double tol = 0, double rel = 0, bool record = false);
+  // One iteration of a fixed-count CG after h = A p: step length, updates of x
+  // and r, stop test, and (unless `last`) the next direction p; invD null: no
+  // preconditioner.  The scalar block holds the state before and after.
+  void fixed_iteration(int prec, void *x, void *r, void *p, const void *h, const void *invD, int64_t n, bool last,
+                       hipStream_t s);
   // p = z + beta p (beta from the scalar block)
   void xpby_dev(int prec, void *p, const void *z, int64_t n, hipStream_t s);
   // the scalar block, synchronising the stream

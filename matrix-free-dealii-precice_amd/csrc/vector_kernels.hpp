@@ -289,6 +289,158 @@ __global__ void __launch_bounds__(kRedThreads) jacobi_dot_kernel(T *z, const T *
   block_reduce_store<T>(v, partials);
 }
 
+// ------------------------------------------------ fixed-count CG steps ---
+// The vector work of a CG iteration that runs without the host (eigenvalue and
+// condition estimates) in three launches: the (p, A p) partial sums, then
+// cg_step_kernel, then cg_direction_kernel.  Each workgroup of the last two
+// adds up the partial sums of the launch before by itself, in the order of
+// sum_partials_epilogue_kernel, and derives the step length from the scalar
+// block: the three one-workgroup epilogue launches of an iteration (2.8 us
+// each, more than the vectors of a level of 10^5 unknowns take) and the store
+// and load of z go.  No workgroup may read what another writes in the same
+// launch, so the scalar block has two copies: a kernel reads `in`, and its
+// first workgroup writes all of `out`.
+// Same partial sums, same order, same expressions as the separate kernels:
+// iterates, step lengths and history are theirs bit for bit.
+// Newton step of 32x8x8 Q3 cells with FP32 levels: 26.7 -> 22.6 ms (6651
+// launches before, 1639 of them epilogues).
+
+// the sum of kRedThreads values in the order of sum_partials_epilogue_kernel,
+// on every thread
+template <int K>
+__device__ inline void sum_partials_all(const double *partials, int n, int stride, double (&v)[K]) {
+  __shared__ double s[K][kRedThreads];
+#pragma unroll
+  for (int j = 0; j < K; ++j) {
+    double a = 0;
+    for (int i = threadIdx.x; i < n; i += kRedThreads) a += partials[j * stride + i];
+    s[j][threadIdx.x] = a;
+  }
+  __syncthreads();
+  for (int w = kRedThreads / 2; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w)
+#pragma unroll
+      for (int j = 0; j < K; ++j) s[j][threadIdx.x] += s[j][threadIdx.x + w];
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < K; ++j) v[j] = s[j][0];
+  __syncthreads();
+}
+
+// alpha from the (p, A p) partial sums, x += alpha p, r -= alpha h, and the
+// partial sums of (r, r) and (r, D^{-1} r) (kJacobi; without it the second is
+// the first): red_epilogue's kRedAlpha, cg_update_dev_kernel and the product of
+// jacobi_dot_kernel
+template <typename T, bool kJacobi>
+__global__ void __launch_bounds__(kRedThreads)
+    cg_step_kernel(T *x, T *r, const T *p, const T *h, const T *invD, const double *ph, int n_ph, const double *in,
+                   double *out, double *hist, int hist_cap, int64_t n, double *partials) {
+  double v[1];
+  sum_partials_all<1>(ph, n_ph, 0, v);
+  const bool stopped = in[kSlotStop] != 0, broke = !stopped && !(v[0] > 0);
+  const double alpha = stopped || broke ? 0.0 : in[kSlotGH] / v[0];
+  if (blockIdx.x == 0 && threadIdx.x < kRedScalars) {
+    double o = in[threadIdx.x];
+    const int k = (int)in[kSlotNAlpha];
+    const bool record = !stopped && !broke && k < hist_cap;
+    switch (threadIdx.x) {
+      case kSlotPH: o = v[0]; break;
+      case kSlotAlpha: o = alpha; break;
+      case kSlotActive: o = stopped || broke ? 0 : 1; break;
+      case kSlotStop: o = stopped || broke ? 1 : 0; break;
+      case kSlotBreakdown: o = broke ? 1 : o; break;
+      case kSlotNAlpha:
+        if (record) {
+          hist[k] = alpha;
+          o = k + 1;
+        }
+        break;
+      default: break;
+    }
+    out[threadIdx.x] = o;
+  }
+  double rr = 0, rz = 0;
+  T rv[kRedBatch], xv[kRedBatch], pv[kRedBatch], hv[kRedBatch], dv[kRedBatch];
+  auto products = [&](T ri, T di) {
+    rr += (double)ri * (double)ri;
+    if constexpr (kJacobi) {
+      const T zi = T(1) * di * ri;
+      rz += (double)ri * (double)zi;
+    }
+  };
+  if (alpha != 0)
+    red_batches(
+        n,
+        [&](int64_t i, int u) {
+          rv[u] = r[i];
+          xv[u] = x[i];
+          pv[u] = p[i];
+          hv[u] = h[i];
+          if constexpr (kJacobi) dv[u] = invD[i];
+        },
+        [&](int64_t i, int u) {
+          x[i] = (T)((double)xv[u] + alpha * (double)pv[u]);
+          const T ri = (T)((double)rv[u] - alpha * (double)hv[u]);
+          r[i] = ri;
+          products(ri, kJacobi ? dv[u] : T(0));
+        });
+  else
+    red_batches(
+        n,
+        [&](int64_t i, int u) {
+          rv[u] = r[i];
+          if constexpr (kJacobi) dv[u] = invD[i];
+        },
+        [&](int64_t, int u) { products(rv[u], kJacobi ? dv[u] : T(0)); });
+  block_reduce_store<T>(rr, partials);
+  if constexpr (kJacobi) {
+    __syncthreads();
+    block_reduce_store<T>(rz, partials + gridDim.x);
+  }
+}
+
+// the stop test and beta from the partial sums, p = D^{-1} r + beta p (kJacobi;
+// p = r + beta p without): red_epilogue's kRedRRStop and kRedBeta and
+// xpby_dev_kernel.  `last`: the stop test alone (one workgroup).
+template <typename T, bool kJacobi>
+__global__ void __launch_bounds__(kRedThreads)
+    cg_direction_kernel(T *p, const T *r, const T *invD, const double *partials, int n_part, const double *in,
+                        double *out, double *hist, int hist_cap, int64_t n, int last) {
+  constexpr int K = kJacobi ? 2 : 1;
+  double v[K];
+  sum_partials_all<K>(partials, n_part, n_part, v);
+  const double rr = v[0], rz = v[K - 1];
+  const bool active = in[kSlotActive] != 0;
+  const bool stop =
+      in[kSlotStop] != 0 || (active && sqrt(rr) <= fmax(in[kSlotTol], in[kSlotRel] * in[kSlotRes0]));
+  const bool go = active && !stop;
+  const double beta = go ? rz / in[kSlotGH] : 0.0;
+  if (blockIdx.x == 0 && threadIdx.x < kRedScalars) {
+    double o = in[threadIdx.x];
+    const int k = (int)in[kSlotNBeta];
+    switch (threadIdx.x) {
+      case kSlotRR: o = rr; break;
+      case kSlotStop: o = stop ? 1 : 0; break;
+      case kSlotBeta: o = last ? o : beta; break;
+      case kSlotGH: o = !last && go ? rz : o; break;
+      case kSlotNBeta:
+        if (!last && go && k < hist_cap) {
+          hist[hist_cap + k] = beta;
+          o = k + 1;
+        }
+        break;
+      default: break;
+    }
+    out[threadIdx.x] = o;
+  }
+  if (last) return;
+  MFG_GRID_STRIDE(i, n) {
+    const T z = kJacobi ? T(T(1) * invD[i] * r[i]) : r[i];
+    p[i] = (T)((double)z + beta * (double)p[i]);
+  }
+}
+
 // p = d + beta p with beta = scal[kSlotBeta]
 template <typename T>
 __global__ void xpby_dev_kernel(T *p, const T *d, const double *scal, int64_t n) {

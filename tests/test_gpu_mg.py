@@ -288,3 +288,27 @@ def test_vcycle_gather_equals_colours(cuda, kind, p, n, precision):
         out[sched] = (y, z)
     a, b = out[None], out[mfgpu.CELLS_COLOURS]
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("kind,p,n", [("solid", 1, (1, 1, 1)), ("solid", 1, (6, 2, 3)), ("solid", 2, (2, 1, 2)),
+                                      ("heat", 1, (7, 7, 4)), ("heat", 2, (3, 3, 3))])
+def test_eigenvalue_estimate_small_levels(cuda, kind, p, n):
+    """The fixed-count CG's estimate on levels of one to two workgroups of
+    unknowns, run until it stops by itself (||r|| <= 1e-15 ||r_0||; the remaining
+    iterations change nothing), against the oracle's."""
+    print(f"eigenvalue estimate {kind} p={p} n={n}", flush=True)
+    nc, fm, cm = (3, 1, 7) if kind == "solid" else (1, 63, 1)
+    lo, hi = [0, 0, 0], [1.0, 0.7, 0.5]
+    gm, om = mfgpu.BoxMesh(lo, hi, list(n), p, nc, fm, cm), O.Mesh(lo, hi, list(n), p, nc, fm, cm)
+    if kind == "solid":
+        u = om.u0(amp=1e-2, noise=1e-5)
+        op, oo = mfgpu.NeoHookOperator(gm, O.MU, O.NU, O.RHO, O.ALPHA1), O.Solid(om, caching=1)
+        op.cache(dev(u))
+        oo.cache(u)
+    else:
+        op, oo = mfgpu.LaplaceOperator(gm, 0.1, None), O.Heat(om, dt=0.1, coef=np.ones(om.n_cells * (p + 1) ** 3))
+    mg = mfgpu.Multigrid([op], [], coarse_eig_iterations=gm.n_dofs)
+    mg.setup()
+    # an extreme Lanczos value is stable to rounding until the run stops
+    lmax = O.cheb_eigenvalues(oo, gm.n_dofs)[0]
+    assert abs(mg.level_info(0)[0] - lmax) <= 1e-8 * lmax
