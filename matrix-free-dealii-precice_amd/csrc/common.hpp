@@ -74,6 +74,23 @@ struct DeviceBuffer {
   template <class T> T *as() const { return static_cast<T *>(ptr); }
 };
 
+// Pinned host memory that kernels reach directly (T is plain data): an error
+// flag that a kernel writes only when it has something to report costs no fill
+// and no copy, and a read-back into it needs no staging.
+template <class T>
+struct PinnedHost {
+  T *ptr = nullptr;
+  PinnedHost() = default;
+  PinnedHost(const PinnedHost &) = delete;
+  PinnedHost &operator=(const PinnedHost &) = delete;
+  ~PinnedHost() {
+    if (ptr) (void)hipHostFree(ptr);
+  }
+  void allocate(size_t n = 1) {
+    if (!ptr) MFG_HIP(hipHostMalloc((void **)&ptr, n * sizeof(T), hipHostMallocDefault));
+  }
+};
+
 template <class T>
 inline void upload(DeviceBuffer &buf, const T *host, size_t n, hipStream_t s) {
   buf.allocate(n * sizeof(T));

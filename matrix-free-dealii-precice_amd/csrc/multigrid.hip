@@ -22,6 +22,7 @@ static int grid_for(int64_t n) { return (int)std::min<int64_t>((n + 255) / 256, 
 
 Reducer::Reducer() {
   own.allocate((kRedBlocks + kRedScalars) * sizeof(double));
+  host.allocate(kRedScalars);
   partials = own.as<double>();
   scal = partials + kRedBlocks;
 }
@@ -105,8 +106,10 @@ void Reducer::fixed_iteration(int prec, void *x, void *r, void *p, const void *h
 }
 
 void Reducer::read(double *out, hipStream_t s) {
-  MFG_HIP(hipMemcpyAsync(out, scal, kRedScalars * sizeof(double), hipMemcpyDeviceToHost, s));
+  double *to = host.ptr ? host.ptr : out;
+  MFG_HIP(hipMemcpyAsync(to, scal, kRedScalars * sizeof(double), hipMemcpyDeviceToHost, s));
   MFG_HIP(hipStreamSynchronize(s));
+  if (to != out) std::memcpy(out, to, kRedScalars * sizeof(double));
 }
 
 void Reducer::ensure_hist(int cap) {

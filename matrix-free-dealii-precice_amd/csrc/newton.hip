@@ -15,31 +15,22 @@
 
 namespace mfg {
 
-template <int P>
-struct ResidualCPB {
-  static constexpr int value = P == 1 ? 8 : P == 2 ? 7 : P == 6 ? 1 : 2;
-};
-
-template <int P>
-static void residual_launch(const OperatorData &op, const double *u, const double *acc, const double *body,
-                            double *R) {
-  constexpr int CPB = ResidualCPB<P>::value;
+template <int P, int KIND>
+static void residual_launch_kind(const OperatorData &op, const double *u, const double *acc, const double *body,
+                                 double *R) {
+  constexpr int CPB = DefaultCPB<P, double>::value, NT = block_threads<P, CPB>();
   ResidualArgs<double> a;
   a.cell_nodes = op.cell_nodes.as<uint32_t>();
   a.u = u;
   a.acc = acc;
-  a.R = R;
   a.vertices = op.vertices.as<double>();
   a.shape = op.tab_shape.as<double>();
   a.colloc = op.tab_colloc.as<double>();
   a.points = op.tab_points.as<double>();
   a.weights = op.tab_weights.as<double>();
   for (int d = 0; d < 3; ++d) a.body[d] = body[d];
-  a.formulation = op.sp.formulation;
-  a.error = op.flag.as<int>();
-  // one launch per colour and material (the cell's material,
-  // mf_elasticity.h:1781-1784)
-  op.for_each_range([&](int, int b, int e, int m) {
+  a.error = op.clear_flag();
+  auto cells = [&](int b, int e, int m, auto to_cells) {  // the cell's material, mf_elasticity.h:1781-1784
     const OperatorData::MaterialConstants &M = op.mats[m];
     a.mu = M.mu;
     a.lambda = M.lambda;
@@ -48,21 +39,46 @@ static void residual_launch(const OperatorData &op, const double *u, const doubl
     a.rho = M.rho;
     a.cell_begin = b;
     a.cell_end = e;
-    residual_cells<P, CPB, double><<<blocks_for(e - b, CPB), block_threads<P, CPB>(), 0, op.stream>>>(a);
+    residual_cells<P, CPB, KIND, decltype(to_cells)::value, double><<<blocks_for(e - b, CPB), NT, 0, op.stream>>>(a);
     MFG_HIP(hipGetLastError());
-  });
+  };
+  // as vmult's schedules: all cells and the sums per node, or a launch per
+  // colour (and material).  The contributions have a buffer of their own
+  // (residuals are synchronous, so no two share it).
+  if (op.gather_ordered()) {
+    if (!op.residual_contrib.ptr) op.residual_contrib.allocate((size_t)op.nqp * 3 * sizeof(double));
+    a.R = op.residual_contrib.as<double>();
+    a.slots = op.gather_slots();
+    if (op.has_inclusion()) op.for_each_range([&](int, int b, int e, int m) { cells(b, e, m, std::true_type()); });
+    else cells(0, op.n_cells, 0, std::true_type());
+    GatherTables<double> g = gather_tables<double>(op);
+    g.contrib = op.residual_contrib.as<double>();
+    residual_sums_kernel<double><<<blocks_for(op.n_nodes, kGatherThreads), kGatherThreads, 0, op.stream>>>(g, R,
+                                                                                                          op.n_nodes);
+    MFG_HIP(hipGetLastError());
+    return;
+  }
+  a.R = R;
+  a.slots = nullptr;
+  op.for_each_range([&](int, int b, int e, int m) { cells(b, e, m, std::false_type()); });
+}
+
+template <int P>
+static void residual_launch(const OperatorData &op, const double *u, const double *acc, const double *body,
+                            double *R) {
+  if (op.sp.formulation != 1) residual_launch_kind<P, 2>(op, u, acc, body, R);
+  else if (op.affine_ref) residual_launch_kind<P, 0>(op, u, acc, body, R);
+  else residual_launch_kind<P, 1>(op, u, acc, body, R);
 }
 
 // R = residual(u, acc) (+ the interface traction over n_faces stored face
 // pairs) with constrained entries zero; returns ||R||.  One host round trip:
-// the norm, the det F flag and (sc) the reducer's scalar block come back
-// together.
+// the norm and (sc) the reducer's scalar block come back together, the det F
+// flag is in host memory.
 double solid_residual(const OperatorData &op, const double *u, const double *acc, const double *body, double *R,
                       Reducer &red, int64_t n_faces = 0, const int32_t *faces = nullptr,
                       const double *traction = nullptr, double *sc = nullptr) {
   MFG_REQUIRE(op.kind == 0 && op.precision == MFG_FP64, MFG_ERR_ARGUMENT, "residual needs an FP64 solid operator");
-  vec_fill(MFG_FP64, R, op.n_dofs, 0.0, op.stream);
-  vec_fill(MFG_FP32, op.flag.ptr, 1, 0.0, op.stream);  // int 0 == float 0 bit pattern
   switch (op.p) {
     case 1: residual_launch<1>(op, u, acc, body, R); break;
     case 2: residual_launch<2>(op, u, acc, body, R); break;
@@ -75,12 +91,10 @@ double solid_residual(const OperatorData &op, const double *u, const double *acc
   // mf_elasticity.h:1849-1897, skipping constrained dofs (zero after :1907)
   add_interface_traction(op, n_faces, faces, u, traction, R);
   red.dot_dev(MFG_FP64, R, R, op.n_dofs, kRedSet, kSlotNewton, op.stream);
-  int h = 0;
-  MFG_HIP(hipMemcpyAsync(&h, op.flag.ptr, sizeof(int), hipMemcpyDeviceToHost, op.stream));
   double local[kRedScalars];
   if (!sc) sc = local;
   red.read(sc, op.stream);
-  MFG_REQUIRE(h == 0, MFG_ERR_NUMERIC, "det_F is not positive");
+  MFG_REQUIRE(*op.flag.ptr == 0, MFG_ERR_NUMERIC, "det_F is not positive");
   return std::sqrt(sc[kSlotNewton]);
 }
 

@@ -255,8 +255,8 @@ static void launch_cache(OperatorData &op, const void *u, int u_fp32, void *expo
   a.affine = op.affine_ref ? 1 : 0;
   a.jxw_ref_field = op.affine_ref ? 0 : 1;
   a.t2_gradient = export_gradient ? 2 : op.t2_gradient() ? 1 : 0;
-  a.u_copy = a.t2_gradient == 1 ? op.u_nodal.as<Number>() : nullptr;
-  a.error = op.flag.as<int>();
+  a.u_copy = a.t2_gradient == 1 ? op.u_copy<Number>() : nullptr;
+  a.error = op.flag.ptr;  // cleared by cache()
   auto cells = [&](int b, int e, int m) {
     a.cell_begin = b;
     a.cell_end = e;
@@ -396,7 +396,7 @@ void OperatorData::compute_diagonal() {
     inv_diag.allocate(n_dofs * es);
     ++buffers_version;
   }
-  fill<int>(flag.as<int>(), 1, 0, stream);
+  clear_flag();
   const int threads = 256;
   if (precision == MFG_FP64) {
     fill<double>(diag.as<double>(), n_dofs, 0.0, stream);
@@ -405,7 +405,7 @@ void OperatorData::compute_diagonal() {
       set_entries_kernel<double><<<blocks_for(n_constrained, threads), threads, 0, stream>>>(
           diag.as<double>(), constrained.as<int32_t>(), n_constrained, 1.0);
     invert_kernel<double><<<std::min(blocks_for(n_dofs, threads), 65536), threads, 0, stream>>>(
-        diag.as<double>(), inv_diag.as<double>(), n_dofs, flag.as<int>());
+        diag.as<double>(), inv_diag.as<double>(), n_dofs, flag.ptr);
   } else {
     fill<float>(diag.as<float>(), n_dofs, 0.0f, stream);
     diagonal_t<float>(*this);
@@ -413,29 +413,24 @@ void OperatorData::compute_diagonal() {
       set_entries_kernel<float><<<blocks_for(n_constrained, threads), threads, 0, stream>>>(
           diag.as<float>(), constrained.as<int32_t>(), n_constrained, 1.0f);
     invert_kernel<float><<<std::min(blocks_for(n_dofs, threads), 65536), threads, 0, stream>>>(
-        diag.as<float>(), inv_diag.as<float>(), n_dofs, flag.as<int>());
+        diag.as<float>(), inv_diag.as<float>(), n_dofs, flag.ptr);
   }
   MFG_HIP(hipGetLastError());
-  int h = 0;
-  MFG_HIP(hipMemcpyAsync(&h, flag.ptr, sizeof(int), hipMemcpyDeviceToHost, stream));
   MFG_HIP(hipStreamSynchronize(stream));
-  MFG_REQUIRE(h == 0, MFG_ERR_NUMERIC, "No diagonal entry in a positive definite operator should be zero or negative");
+  MFG_REQUIRE(*flag.ptr == 0, MFG_ERR_NUMERIC, "No diagonal entry in a positive definite operator should be zero or negative");
   has_diagonal = true;
 }
 
 void OperatorData::cache(const void *u, int u_precision) {
   MFG_REQUIRE(kind == 0, MFG_ERR_ARGUMENT, "cache() applies to the solid operator");
   MFG_REQUIRE(u, MFG_ERR_ARGUMENT, "null displacement");
-  fill<int>(flag.as<int>(), 1, 0, stream);
-  const bool scalar_referential = sp.caching == MFG_CACHING_SCALAR_REFERENTIAL;
-  // scalar_referential keeps the displacement itself (mf_nh_operator.h:442-455),
-  // the 10-word storage for export_qp_gradient
-  if ((scalar_referential || t2_gradient()) && u_nodal.bytes != (size_t)n_dofs * elem_size()) {
-    u_nodal.allocate((size_t)n_dofs * elem_size());
-    ++buffers_version;
-  }
-  if (scalar_referential) {
+  clear_flag();
+  if (sp.caching == MFG_CACHING_SCALAR_REFERENTIAL) {  // keeps the displacement itself (mf_nh_operator.h:442-455)
     const int threads = 256, blocks = std::min(blocks_for(n_dofs, threads), 65536);
+    if (u_nodal.bytes != (size_t)n_dofs * elem_size()) {
+      u_nodal.allocate((size_t)n_dofs * elem_size());
+      ++buffers_version;
+    }
     if (precision == MFG_FP64 && u_precision == MFG_FP64)
       convert_kernel<double, double><<<blocks, threads, 0, stream>>>(u_nodal.as<double>(), (const double *)u, n_dofs);
     else if (precision == MFG_FP64)
@@ -448,10 +443,8 @@ void OperatorData::cache(const void *u, int u_precision) {
   }
   if (precision == MFG_FP64) cache_t<double>(*this, u, u_precision == MFG_FP32);
   else cache_t<float>(*this, u, u_precision == MFG_FP32);
-  int h = 0;
-  MFG_HIP(hipMemcpyAsync(&h, flag.ptr, sizeof(int), hipMemcpyDeviceToHost, stream));
   MFG_HIP(hipStreamSynchronize(stream));
-  MFG_REQUIRE(h == 0, MFG_ERR_NUMERIC, "det_F is not positive");
+  MFG_REQUIRE(*flag.ptr == 0, MFG_ERR_NUMERIC, "det_F is not positive");
   ready = true;
   has_diagonal = false;
 }
@@ -462,8 +455,8 @@ void OperatorData::cache(const void *u, int u_precision) {
 // J_cur only.
 void OperatorData::export_qp_gradient(DeviceBuffer &out) {
   out.allocate((size_t)n_fields * nqp * elem_size());
-  if (precision == MFG_FP64) cache_t<double>(*this, u_nodal.ptr, 0, out.ptr);
-  else cache_t<float>(*this, u_nodal.ptr, 1, out.ptr);
+  if (precision == MFG_FP64) cache_t<double>(*this, u_copy<double>(), 0, out.ptr);
+  else cache_t<float>(*this, u_copy<float>(), 1, out.ptr);
 }
 
 template <typename Number>
@@ -662,7 +655,6 @@ void OperatorData::setup_layout(const mfg_level_desc &d) {
   upload(perm_dev, perm.data(), perm.size(), stream);
   host_cell_nodes.assign(d.cell_nodes, d.cell_nodes + nqp);
   host_cmask = std::move(cmask);
-  flag.allocate(sizeof(int));
   const Tables1D t = make_tables(p);
   if (precision == MFG_FP64) upload_tables<double>(*this, t);
   else upload_tables<float>(*this, t);
@@ -800,12 +792,13 @@ void OperatorData::setup_solid() {
                                      : QSolidT2F1<double>::kFields;
   }
   const size_t es = precision == MFG_FP64 ? 8 : 4;
-  qd.allocate((size_t)n_fields * nqp * es);
+  // the 10-word storage keeps the displacement as well (export_qp_gradient)
+  qd.allocate((size_t)n_fields * nqp * es + (t2_gradient() ? (size_t)n_dofs * es : 0));
 }
 
 size_t OperatorData::memory_consumption() const {
   return qd.bytes + cell_nodes.bytes + constrained.bytes + u_nodal.bytes + cell_jxw.bytes + wq3.bytes + cell_geo.bytes + cell_met.bytes +
-         gather_offsets.bytes + gather_places.bytes + gather_cmask.bytes + contrib.bytes;
+         gather_offsets.bytes + gather_places.bytes + gather_cmask.bytes + contrib.bytes + residual_contrib.bytes;
 }
 
 }  // namespace mfg

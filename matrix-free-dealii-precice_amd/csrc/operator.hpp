@@ -66,7 +66,12 @@ struct OperatorData {
   DeviceBuffer tab_shape, tab_colloc, tab_sq, tab_points, tab_weights;
   DeviceBuffer qd;           // quadrature cache, field-major SoA
   DeviceBuffer diag, inv_diag;
-  DeviceBuffer u_nodal;      // the linearisation point (scalar_referential caching and the 10-word storage)
+  DeviceBuffer u_nodal;      // the linearisation point (scalar_referential caching)
+  // the linearisation point of the 10-word storage, after its fields in qd
+  template <class T>
+  T *u_copy() const {
+    return qd.as<T>() + (size_t)n_fields * nqp;
+  }
   // reference-frame JxW per cell: when every cell's trilinear map is affine,
   // JxW_ref = cell_jxw[stored cell] * wq3[point] (tensor2, formulation 1)
   bool affine_ref = false;
@@ -76,7 +81,14 @@ struct OperatorData {
   bool cartesian_ref = false;  // affine, and every cell's J_ref is diagonal
   int t2_storage = MFG_T2_FOLDED;  // tensor2 formulation-1 point storage (MFG_T2_*)
   bool t2_gradient() const { return kind == 0 && sp.caching == MFG_CACHING_TENSOR2 && sp.formulation == 1 && t2_storage == MFG_T2_GRADIENT; }
-  DeviceBuffer flag;         // int error flag
+  // Error flag that the kernels of cache(), compute_diagonal() and the residual
+  // set; these calls clear it, launch, synchronise and look at it.
+  mutable PinnedHost<int> flag;
+  int *clear_flag() const {
+    flag.allocate();
+    *flag.ptr = 0;
+    return flag.ptr;
+  }
   std::vector<int32_t> host_constrained;
   std::vector<int32_t> host_cell_nodes;  // input cell order (used to build transfers)
   std::vector<uint8_t> host_cmask;       // per node: constrained components
@@ -113,6 +125,7 @@ struct OperatorData {
   // cmask: the node's constrained components.
   DeviceBuffer gather_offsets, gather_places, gather_cmask, contrib;
   bool gather_indexed = false;
+  mutable DeviceBuffer residual_contrib;  // the contributions of the Newton residual
   const uint32_t *gather_slots() const { return gather_indexed ? nullptr : gather_places.as<uint32_t>(); }
   void build_gather();
   // The schedule was set through mfg_operator_set_cell_schedule: every

@@ -155,7 +155,7 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) cache_solid(CacheAr
     }
   const Number J = det3(F);
   if (!(J > Number(0))) {
-    atomicOr(a.error, 1);
+    *a.error = 1;
     return;
   }
   const int64_t n = a.nqp;

@@ -13,6 +13,7 @@ struct Reducer {
   DeviceBuffer own;            // partials and scalars, when the reducer allocates them
   DeviceBuffer hist_buf;       // step lengths of fixed-count runs (alphas, then betas)
   DeviceBuffer fixed_buf;      // fixed-count runs: 2 kRedBlocks partials and the other copy of the scalar block
+  PinnedHost<double> host;     // read()'s copy of the scalar block, when the reducer allocates
   double *partials = nullptr;  // kRedBlocks
   double *scal = nullptr;      // kRedScalars
   int hist_cap = 0;

@@ -24,7 +24,7 @@ template <typename T>
 __global__ void invert_kernel(const T *d, T *inv, int64_t n, int *flag) {
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
     const T v = d[i];
-    if (!(v > T(0))) atomicOr(flag, 1);
+    if (!(v > T(0))) *flag = 1;
     inv[i] = T(1) / v;
   }
 }

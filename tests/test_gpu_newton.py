@@ -97,3 +97,30 @@ def test_coupled_steps_with_interface_traction(cuda, level_precision):
         pu, cu = plain.get_state()[0], cleared.get_state()[0]
         assert torch.equal(pu, cu) and pi.newton_iterations == ci.newton_iterations
         assert float((pu - dev(gu)).norm()) > 1e-3 * float(pu.norm())  # the traction moves the solid
+
+
+@pytest.mark.parametrize("p,n", [(1, (3, 3, 2)), (2, (3, 2, 2)), (4, (2, 3, 1)), (6, (2, 1, 1))])
+@pytest.mark.parametrize("amp", [1e-9, 1e-2])
+def test_residual_of_linear_displacement(cuda, p, n, amp):
+    """u = A X: the stress is constant, so the residual's stress term vanishes at
+    every node inside the box to the rounding of the stress itself, for a strain
+    of 1e-9 as well as for one of 1e-2, in both schedules."""
+    print(f"residual of a linear displacement p={p} n={n} amp={amp}", flush=True)
+    lo, hi = [0, 0, 0], [1.0, 0.6, 0.4]
+    gm = mfgpu.BoxMesh(lo, hi, list(n), p, 3, 1, 7)
+    A = amp * np.array([[1.0, 0.3, -0.2], [0.4, -0.7, 0.1], [0.2, 0.5, 0.6]])
+    X = gm.node_coords()
+    u = (X @ A.T).ravel()
+    inside = np.all((X > 1e-9) & (X < np.array(hi) - 1e-9), axis=1)
+    op = mfgpu.NeoHookOperator(gm, O.MU, O.NU, O.RHO, O.ALPHA1)
+    for sched in (mfgpu.CELLS_GATHER, mfgpu.CELLS_COLOURS):
+        op.set_cell_schedule(sched)
+        R, _ = mfgpu.solid_residual(op, dev(u), dev(np.zeros_like(u)), (0.0, 0.0, 0.0))
+        r = R.cpu().numpy().reshape(-1, 3)
+        # |R_a| <= sum over 8 cells of int |P| |Grad phi_a|; the gradient's rows sum to 2 p^2 / h, a face area
+        # times p^2 bounds a cell's integral, and Grad u carries 2 p^2 (p + 1) roundings of |u| / h
+        stress = 10 * O.MU * amp
+        eps = np.finfo(np.float64).eps
+        tol = 8 * 2 * p * p * stress * 0.4 * 4 * (p + 1) * 2 * p * p * eps * 3
+        assert np.abs(r[inside]).max(initial=0.0) <= tol
+        assert np.abs(r).max() > 0
