@@ -46,13 +46,14 @@ static void residual_launch_kind(const OperatorData &op, const double *u, const 
   // colour (and material).  The contributions have a buffer of their own
   // (residuals are synchronous, so no two share it).
   if (op.gather_ordered()) {
-    if (!op.residual_contrib.ptr) op.residual_contrib.allocate((size_t)op.nqp * 3 * sizeof(double));
-    a.R = op.residual_contrib.as<double>();
+    const size_t bytes = (size_t)op.nqp * 3 * sizeof(double);
+    if (op.setup_contrib.bytes < bytes) op.setup_contrib.allocate(bytes);
+    a.R = op.setup_contrib.as<double>();
     a.slots = op.gather_slots();
     if (op.has_inclusion()) op.for_each_range([&](int, int b, int e, int m) { cells(b, e, m, std::true_type()); });
     else cells(0, op.n_cells, 0, std::true_type());
     GatherTables<double> g = gather_tables<double>(op);
-    g.contrib = op.residual_contrib.as<double>();
+    g.contrib = op.setup_contrib.as<double>();
     residual_sums_kernel<double><<<blocks_for(op.n_nodes, kGatherThreads), kGatherThreads, 0, op.stream>>>(g, R,
                                                                                                           op.n_nodes);
     MFG_HIP(hipGetLastError());

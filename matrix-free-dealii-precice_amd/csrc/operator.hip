@@ -137,15 +137,6 @@ static void with_column_qop(const OperatorData &op, int m, F fn) {
     fn(QSolidT2F0<Number>{op.qd.as<Number>(), op.nqp, Number(M.kappa), Number(M.c_1), Number(M.rho_alpha)});
 }
 
-template <typename Number>
-static void fill(Number *x, int64_t n, Number v, hipStream_t s) {
-  if (n <= 0) return;
-  const int threads = 256;
-  const int blocks = (int)std::min<int64_t>((n + threads - 1) / threads, 65536);
-  fill_kernel<Number><<<blocks, threads, 0, s>>>(x, n, v);
-  MFG_HIP(hipGetLastError());
-}
-
 // --------------------------------------------------------- dispatchers ---
 template <int P, typename Number>
 static void launch_apply(const OperatorData &op, const void *src, void *dst, int fix_mode, bool gather,
@@ -269,23 +260,50 @@ static void launch_cache(OperatorData &op, const void *u, int u_fp32, void *expo
   else cells(0, op.n_cells, 0);
 }
 
+// The diagonal's cells and (GATHER, as vmult's schedules) sums, which then
+// cover the constrained rows and the inverse; the contributions share the
+// residual's buffer (both calls are synchronous).
 template <int P, typename Number>
-static void launch_diagonal(OperatorData &op) {
+static void launch_diagonal(OperatorData &op, bool gather) {
+  constexpr int CPB = DefaultCPB<P, Number>::value, NT = block_threads<P, CPB>();
   DiagArgs<Number> a;
   a.cell_nodes = op.cell_nodes.as<uint32_t>();
   a.sq = op.tab_sq.as<Number>();
   a.shape = op.tab_shape.as<Number>();
   a.colloc = op.tab_colloc.as<Number>();
   a.diag = op.diag.as<Number>();
-  constexpr int NT = ((P + 1) * (P + 1) * (P + 1) + 63) / 64 * 64;
-  op.for_each_range([&](int, int b, int e, int m) {
-    with_qop<Number, false>(op, m, [&](auto q) {
-      a.cell_begin = b;
-      a.cell_end = e;
-      diagonal_cells<P, Number, decltype(q)><<<e - b, NT, 0, op.stream>>>(a, q);
+  a.slots = nullptr;
+  auto cells = [&](int b, int e, int m, auto to_cells) {
+    a.cell_begin = b;
+    a.cell_end = e;
+    auto launch = [&](auto q) {
+      diagonal_cells<P, CPB, decltype(to_cells)::value, Number, decltype(q)>
+          <<<blocks_for(e - b, CPB), NT, 0, op.stream>>>(a, q);
       MFG_HIP(hipGetLastError());
-    });
-  });
+    };
+    if (op.t2_gradient() && op.cartesian_ref) launch(t2_gradient_op<Number, false, true>(op, m));
+    else with_qop<Number, false>(op, m, launch);
+  };
+  if (!gather) {
+    op.for_each_range([&](int, int b, int e, int m) { cells(b, e, m, std::false_type()); });
+    return;
+  }
+  const size_t bytes = (size_t)op.nqp * op.nc * op.elem_size();
+  if (op.setup_contrib.bytes < bytes) op.setup_contrib.allocate(bytes);
+  a.diag = op.setup_contrib.as<Number>();
+  a.slots = op.gather_slots();
+  if (op.has_inclusion()) op.for_each_range([&](int, int b, int e, int m) { cells(b, e, m, std::true_type()); });
+  else cells(0, op.n_cells, 0, std::true_type());
+  GatherTables<Number> g = gather_tables<Number>(op);
+  g.contrib = op.setup_contrib.as<Number>();
+  const int blocks = blocks_for(op.n_nodes, kGatherThreads);
+  if (op.nc == 3)
+    diagonal_sums_kernel<Number, 3><<<blocks, kGatherThreads, 0, op.stream>>>(
+        g, op.diag.as<Number>(), op.inv_diag.as<Number>(), op.n_nodes, op.flag.ptr);
+  else
+    diagonal_sums_kernel<Number, 1><<<blocks, kGatherThreads, 0, op.stream>>>(
+        g, op.diag.as<Number>(), op.inv_diag.as<Number>(), op.n_nodes, op.flag.ptr);
+  MFG_HIP(hipGetLastError());
 }
 
 #define MFG_DISPATCH_DEGREE(p, FN, ...)                                                  \
@@ -309,8 +327,8 @@ static void cache_t(OperatorData &op, const void *u, int u_fp32, void *export_gr
   MFG_DISPATCH_DEGREE(op.p, launch_cache, op, u, u_fp32, export_gradient);
 }
 template <typename Number>
-static void diagonal_t(OperatorData &op) {
-  MFG_DISPATCH_DEGREE(op.p, launch_diagonal, op);
+static void diagonal_t(OperatorData &op, bool gather) {
+  MFG_DISPATCH_DEGREE(op.p, launch_diagonal, op, gather);
 }
 
 static void apply_checked(const OperatorData &op, const void *src, void *dst, bool add, bool gather, hipStream_t s) {
@@ -397,24 +415,20 @@ void OperatorData::compute_diagonal() {
     ++buffers_version;
   }
   clear_flag();
-  const int threads = 256;
-  if (precision == MFG_FP64) {
-    fill<double>(diag.as<double>(), n_dofs, 0.0, stream);
-    diagonal_t<double>(*this);
+  const bool gather = gather_ordered();
+  auto run = [&](auto tag) {
+    using Number = decltype(tag);
+    diagonal_t<Number>(*this, gather);
+    if (gather) return;
+    const int threads = 256;
     if (n_constrained)
-      set_entries_kernel<double><<<blocks_for(n_constrained, threads), threads, 0, stream>>>(
-          diag.as<double>(), constrained.as<int32_t>(), n_constrained, 1.0);
-    invert_kernel<double><<<std::min(blocks_for(n_dofs, threads), 65536), threads, 0, stream>>>(
-        diag.as<double>(), inv_diag.as<double>(), n_dofs, flag.ptr);
-  } else {
-    fill<float>(diag.as<float>(), n_dofs, 0.0f, stream);
-    diagonal_t<float>(*this);
-    if (n_constrained)
-      set_entries_kernel<float><<<blocks_for(n_constrained, threads), threads, 0, stream>>>(
-          diag.as<float>(), constrained.as<int32_t>(), n_constrained, 1.0f);
-    invert_kernel<float><<<std::min(blocks_for(n_dofs, threads), 65536), threads, 0, stream>>>(
-        diag.as<float>(), inv_diag.as<float>(), n_dofs, flag.ptr);
-  }
+      set_entries_kernel<Number><<<blocks_for(n_constrained, threads), threads, 0, stream>>>(
+          diag.as<Number>(), constrained.as<int32_t>(), n_constrained, Number(1));
+    invert_kernel<Number><<<std::min(blocks_for(n_dofs, threads), 65536), threads, 0, stream>>>(
+        diag.as<Number>(), inv_diag.as<Number>(), n_dofs, flag.ptr);
+  };
+  if (precision == MFG_FP64) run(double());
+  else run(float());
   MFG_HIP(hipGetLastError());
   MFG_HIP(hipStreamSynchronize(stream));
   MFG_REQUIRE(*flag.ptr == 0, MFG_ERR_NUMERIC, "No diagonal entry in a positive definite operator should be zero or negative");
@@ -798,7 +812,7 @@ void OperatorData::setup_solid() {
 
 size_t OperatorData::memory_consumption() const {
   return qd.bytes + cell_nodes.bytes + constrained.bytes + u_nodal.bytes + cell_jxw.bytes + wq3.bytes + cell_geo.bytes + cell_met.bytes +
-         gather_offsets.bytes + gather_places.bytes + gather_cmask.bytes + contrib.bytes + residual_contrib.bytes;
+         gather_offsets.bytes + gather_places.bytes + gather_cmask.bytes + contrib.bytes + setup_contrib.bytes;
 }
 
 }  // namespace mfg

@@ -125,7 +125,10 @@ struct OperatorData {
   // cmask: the node's constrained components.
   DeviceBuffer gather_offsets, gather_places, gather_cmask, contrib;
   bool gather_indexed = false;
-  mutable DeviceBuffer residual_contrib;  // the contributions of the Newton residual
+  // the contributions of the Newton residual and the diagonal (synchronous
+  // calls: no two share it, and an application in flight on another stream has
+  // its own)
+  mutable DeviceBuffer setup_contrib;
   const uint32_t *gather_slots() const { return gather_indexed ? nullptr : gather_places.as<uint32_t>(); }
   void build_gather();
   // The schedule was set through mfg_operator_set_cell_schedule: every

@@ -29,7 +29,7 @@ struct ResidualArgs {
 // No term cancels down from the size of the identity to that of the strain
 // (mu b - s I does), and b and tau are not formed.
 template <typename Number>
-__device__ inline bool residual_point_affine(const ResidualArgs<Number> &a, const double *X, double wq,
+__device__ inline bool residual_point_affine(const ResidualArgs<Number> &a, ConstantPtr<double> X, double wq,
                                              const Number (&gr)[3][3], const Number (&av)[3], Number (&val)[3],
                                              Number (&grad)[3][3]) {
   double Jr[3][3], R[3][3];
@@ -207,7 +207,8 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) residual_cells(Resi
     gr[c][2] = T.template line<2>(s_colloc, T.k, 6 + c);
   }
   const double wq = a.weights[T.i] * a.weights[T.j] * a.weights[T.k];
-  const double *X = a.vertices + (int64_t)(active ? cell : first_cell) * 24;
+  const int vcell = CPB == 1 ? __builtin_amdgcn_readfirstlane(first_cell) : active ? cell : first_cell;
+  const ConstantPtr<double> X = as_constant(a.vertices) + (int64_t)vcell * 24;
   bool ok;
   if constexpr (KIND == 0) {
     ok = residual_point_affine(a, X, wq, gr, av, val, grad);

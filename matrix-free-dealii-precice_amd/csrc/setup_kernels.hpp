@@ -51,7 +51,8 @@ __device__ inline void inv3(const Number (&A)[3][3], Number (&R)[3][3]) {
 }
 
 // Trilinear Jacobian dX_e/dxi_f at reference point xi from 8 vertices.
-__device__ inline void trilinear_jacobian(const double *v, double x0, double x1, double x2, double (&J)[3][3]) {
+template <class Ptr>
+__device__ inline void trilinear_jacobian(Ptr v, double x0, double x1, double x2, double (&J)[3][3]) {
 #pragma unroll
   for (int e = 0; e < 3; ++e)
 #pragma unroll
@@ -76,7 +77,8 @@ __device__ inline void trilinear_jacobian(const double *v, double x0, double x1,
 // the host forms the per-cell tables from them.  The general sum over the
 // vertices cancels from the size of the coordinates down to that of the cell
 // (1e-14 of the Jacobian on the 32-cell beam, 4 long); the differences do not.
-__device__ inline void affine_jacobian(const double *v, double (&J)[3][3]) {
+template <class Ptr>
+__device__ inline void affine_jacobian(Ptr v, double (&J)[3][3]) {
 #pragma unroll
   for (int e = 0; e < 3; ++e) {
     J[e][0] = v[3 + e] - v[e];
@@ -89,46 +91,57 @@ template <int P, int CPB, typename Number>
 __global__ void __launch_bounds__((block_threads<P, CPB>())) cache_solid(CacheArgs<Number> a) {
   constexpr int N = P + 1, N3 = N * N * N;
   __shared__ Number s_shape[N * N], s_colloc[N * N];
-  __shared__ Number s_tile[CPB * 9 * N3];
+  __shared__ Number s_tile[CPB * 6 * N3];
   const int t = threadIdx.x;
-  if (t < N * N) {
-    s_shape[t] = a.shape[t];
-    s_colloc[t] = a.colloc[t];
-  }
   const int lc_raw = t / N3;
   const bool pad = lc_raw >= CPB;
   const int lc = pad ? CPB - 1 : lc_raw;
   const int pt = pad ? 0 : t - lc_raw * N3;
   Tile<N, Number> T;
-  T.base = s_tile + lc * 9 * N3;
+  T.base = s_tile + lc * 6 * N3;
   T.pt = pt;
   T.i = pt % N;
   T.j = (pt / N) % N;
   T.k = pt / (N * N);
   T.writer = !pad;
-  const int cell = a.cell_begin + blockIdx.x * CPB + lc;
+  const int first_cell = a.cell_begin + xcd_remap(blockIdx.x, gridDim.x) * CPB, cell = first_cell + lc;
   const bool active = !pad && cell < a.cell_end;
-  const int64_t qidx = active ? (int64_t)cell * N3 + pt : 0;
+  const int64_t qidx = (int64_t)first_cell * N3 + (active ? t : 0);
   const uint32_t entry = active ? a.cell_nodes[qidx] : 0u;
+  Number sh = 0, co = 0;
+  if (t < N * N) {
+    sh = a.shape[t];
+    co = a.colloc[t];
+  }
   const int64_t node = (int64_t)(entry & kNodeMaskDev);
   Number u[3];
+  // read_dof_values_plain: constrained entries are read as stored
+  if (a.u_fp32) {
+    const NodeValues<float, 3> x = active ? load_node<float, 3>((const float *)a.u + node * 3) : NodeValues<float, 3>{};
 #pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    // read_dof_values_plain: constrained entries are read as stored
-    if (!active) u[c] = 0;
-    else if (a.u_fp32) u[c] = (Number)((const float *)a.u)[node * 3 + c];
-    else u[c] = (Number)((const double *)a.u)[node * 3 + c];
+    for (int c = 0; c < 3; ++c) u[c] = (Number)x.v[c];
+  } else {
+    const NodeValues<double, 3> x =
+        active ? load_node<double, 3>((const double *)a.u + node * 3) : NodeValues<double, 3>{};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) u[c] = (Number)x.v[c];
   }
   // one (cell, point) of every node carries the first-touch bit
   if (a.u_copy && active && (entry >> 31)) store_node<Number, 3>(a.u_copy + node * 3, u);
-  __syncthreads();
+  if (t < N * N) {  // published by the first barrier of the sweeps
+    s_shape[t] = sh;
+    s_colloc[t] = co;
+  }
   Number gr[3][3];
-  evaluate_g<N, 3, Number>(T, s_shape, s_colloc, u, gr);
+  evaluate_g<N, 3, Number, rolled_components<N, true>()>(T, s_shape, s_colloc, u, gr);
   if (!active) return;
 
   double Jr[3][3], Jri[3][3];
-  if (a.affine) affine_jacobian(a.vertices + (int64_t)cell * 24, Jr);
-  else trilinear_jacobian(a.vertices + (int64_t)cell * 24, a.points[T.i], a.points[T.j], a.points[T.k], Jr);
+  // one cell per workgroup: the vertices come in as scalar loads
+  const int vcell = CPB == 1 ? __builtin_amdgcn_readfirstlane(first_cell) : cell;
+  const ConstantPtr<double> X = as_constant(a.vertices) + (int64_t)vcell * 24;
+  if (a.affine) affine_jacobian(X, Jr);
+  else trilinear_jacobian(X, a.points[T.i], a.points[T.j], a.points[T.k], Jr);
   {
     const double id = 1.0 / (Jr[0][0] * (Jr[1][1] * Jr[2][2] - Jr[1][2] * Jr[2][1]) -
                              Jr[0][1] * (Jr[1][0] * Jr[2][2] - Jr[1][2] * Jr[2][0]) +
@@ -267,119 +280,228 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) cache_solid(CacheAr
 // The diagonal entry of dof (node a, component d) is
 //   sum_q [ m_d(q) phi_a(q)^2 + sum_{f,g} G_d[f][g](q) dphi_a/dxi_f dphi_a/dxi_g ],
 // where m_d and G_d come from applying the quadrature op to unit values and
-// unit reference gradients.  Each of the 7 (m, G_ff, G_fg+G_gf) terms is a
-// tensor-product sum over q with squared 1D matrices (phi^2, phi*phi',
-// phi'^2), evaluated with the same transposed sweeps as integrate.
+// unit reference gradients.  Each of the 7 terms (m; G_xx, G_yy, G_zz; G_xy,
+// G_xz, G_yz with their transposes) is a tensor-product sum over q with squared
+// 1D matrices (phi^2, phi*phi', phi'^2), evaluated with the same transposed
+// sweeps as integrate.  After a direction's sweep the terms whose remaining
+// directions take the same matrices are added: 7 lines along z, 6 along y, 3
+// along x per component instead of 7 each.  Pinning each component's results
+// before the next component's lines takes the FP64 kernel from 198 - 256 VGPRs
+// to 66 - 82 (Q3 - Q6).  compute_diagonal(), against unit vectors through the
+// quadrature op and a launch per colour: Q3 cubes FP64 of 20K, 0.3M and 3M
+// unknowns 93 -> 17, 99 -> 29, 222 -> 160 us; Q6 220 -> 22, 237 -> 35, 690 ->
+// 246; Q1 3M unknowns 1669 -> 268 us (8 cells per workgroup instead of one).
+
+// the 7 terms of every component at a point
+template <class QOp>
+struct DiagonalTerms {
+  template <typename Number>
+  static __device__ void eval(const QOp &qop, const typename QOp::Cell &cd, const typename QOp::Data &qd,
+                              Number (&coef)[7 * QOp::NC]) {
+    constexpr int NC = QOp::NC;
+    const Number m = qop.value_scale(cd, qd);
+#pragma unroll
+    for (int d = 0; d < NC; ++d) {
+      Number G[3][3];
+#pragma unroll
+      for (int h = 0; h < 3; ++h) {
+        Number g[NC][3] = {};
+        g[d][h] = 1;
+        qop.apply_grad(cd, qd, g);
+#pragma unroll
+        for (int f = 0; f < 3; ++f) G[f][h] = g[d][f];
+      }
+      coef[d * 7] = m;
+      coef[d * 7 + 1] = G[0][0];
+      coef[d * 7 + 2] = G[1][1];
+      coef[d * 7 + 3] = G[2][2];
+      coef[d * 7 + 4] = G[0][1] + G[1][0];
+      coef[d * 7 + 5] = G[0][2] + G[2][0];
+      coef[d * 7 + 6] = G[1][2] + G[2][1];
+    }
+  }
+};
+// QSolidT2F1G: G_d = w (mu G + (s + 2 lambda) j_d j_d^T), j_d the column d of Jinv_cur
+template <typename Number, bool kEarlyCell, bool kCartesian>
+struct DiagonalTerms<QSolidT2F1G<Number, kEarlyCell, kCartesian>> {
+  using QOp = QSolidT2F1G<Number, kEarlyCell, kCartesian>;
+  static __device__ void eval(const QOp &qop, const typename QOp::Cell &cd, const typename QOp::Data &qd,
+                              Number (&coef)[21]) {
+    const Number m = qop.value_scale(cd, qd), w = cd.jxw * qd.w, wm = w * qop.mu, ws = w * (qd.s + qop.two_lambda);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const Number j0 = qd.ji[d], j1 = qd.ji[3 + d], j2 = qd.ji[6 + d];
+      const Number s0 = ws * j0, s1 = ws * j1, s2 = ws * j2;
+      coef[d * 7] = m;
+      coef[d * 7 + 1] = wm * cd.g[0] + s0 * j0;
+      coef[d * 7 + 2] = wm * cd.g[1] + s1 * j1;
+      coef[d * 7 + 3] = wm * cd.g[2] + s2 * j2;
+      const Number off[3] = {s0 * j1, s0 * j2, s1 * j2};
+#pragma unroll
+      for (int x = 0; x < 3; ++x) {
+        if constexpr (kCartesian) coef[d * 7 + 4 + x] = Number(2) * off[x];
+        else coef[d * 7 + 4 + x] = Number(2) * (wm * cd.g[3 + x] + off[x]);
+      }
+    }
+  }
+};
+// heat on affine cells: c dt JxW G
+template <typename Number>
+struct DiagonalTerms<QHeat<Number, true>> {
+  using QOp = QHeat<Number, true>;
+  static __device__ void eval(const QOp &qop, const typename QOp::Cell &cd, const typename QOp::Data &qd,
+                              Number (&coef)[7]) {
+    coef[0] = qop.value_scale(cd, qd);
+    const Number s = qd.c * qop.dt * coef[0];
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      coef[1 + x] = s * cd.g[x];
+      coef[4 + x] = Number(2) * (s * cd.g[3 + x]);
+    }
+  }
+};
+
 template <typename Number>
 struct DiagArgs {
   const uint32_t *cell_nodes;
-  int cell_begin, cell_end;  // one colour: cells share no node
+  int cell_begin, cell_end;  // one colour: cells share no node; or (GATHER) all cells
   const Number *sq;  // 3 x N x N: SS, SD, DD
   const Number *shape, *colloc;  // for ops that read a nodal field
-  Number *diag;
+  Number *diag;                  // or (GATHER) the contribution buffer
+  const uint32_t *slots;         // GATHER: places of the contributions
 };
 
-template <int P, typename Number, class QOp>
-__global__ void __launch_bounds__(((P + 1) * (P + 1) * (P + 1) + 63) / 64 * 64) diagonal_cells(DiagArgs<Number> a, QOp qop) {
+// The first colour touching a node stores; constrained components are left.
+template <int P, int CPB, bool kToCells, typename Number, class QOp>
+__global__ void __launch_bounds__((block_threads<P, CPB>())) diagonal_cells(DiagArgs<Number> a, QOp qop) {
   constexpr int N = P + 1, N3 = N * N * N, NC = QOp::NC, NTERM = 7 * NC;
   __shared__ Number s_sq[3 * N * N];
-  __shared__ Number s_tile[NTERM * N3];
+  __shared__ Number s_tile[CPB * NTERM * N3];
   const int t = threadIdx.x;
   for (int x = t; x < 3 * N * N; x += blockDim.x) s_sq[x] = a.sq[x];
-  const bool pad = t >= N3;
-  const int pt = pad ? 0 : t;
+  const int lc_raw = t / N3;
+  const bool pad = lc_raw >= CPB;
+  const int lc = pad ? CPB - 1 : lc_raw;
+  const int pt = pad ? 0 : t - lc_raw * N3;
   Tile<N, Number> T;
-  T.base = s_tile;
+  T.base = s_tile + lc * NTERM * N3;
   T.pt = pt;
   T.i = pt % N;
   T.j = (pt / N) % N;
   T.k = pt / (N * N);
   T.writer = !pad;
-  const int cell = a.cell_begin + blockIdx.x;
+  const int first_cell = a.cell_begin + blockIdx.x * CPB, cell = first_cell + lc;
   const bool active = !pad && cell < a.cell_end;
-  const int64_t qidx = active ? (int64_t)cell * N3 + pt : 0;
+  const int64_t qb = (int64_t)first_cell * N3;
+  const uint32_t lo = active ? (uint32_t)t : 0u;
+  const uint32_t entry = active ? (a.cell_nodes + qb)[lo] : 0u;
+  uint32_t slot = 0;
+  if constexpr (kToCells) slot = a.slots ? (a.slots + qb)[lo] : (uint32_t)(qb + lo);
   Number coef[NTERM];
   {
-    typename QOp::Data qd = qop.load((int64_t)(a.cell_begin + blockIdx.x) * N3, (uint32_t)pt, pt);
-    const typename QOp::Cell cd = qop.load_cell(active ? cell : 0);
+    typename QOp::Data qd = qop.load(qb, lo, CPB > 1 && !active ? 0 : pt);
+    const typename QOp::Cell cd = qop.load_cell(active ? cell : first_cell);
     if constexpr (QOp::kNodalField) {
       __shared__ Number s_shape[N * N], s_colloc[N * N];
       if (t < N * N) {
         s_shape[t] = a.shape[t];
         s_colloc[t] = a.colloc[t];
       }
-      const int64_t node = active ? (int64_t)(a.cell_nodes[qidx] & kNodeMaskDev) : 0;
+      const int64_t node = (int64_t)(entry & kNodeMaskDev);
       Number w[3], wg[3][3];
 #pragma unroll
       for (int c = 0; c < 3; ++c) w[c] = active ? qop.u[node * 3 + c] : Number(0);
       evaluate_g<N, 3, Number>(T, s_shape, s_colloc, w, wg);
       qop.attach(qd, wg);
     }
-    Number v[NC], g[NC][3];
-#pragma unroll
-    for (int c = 0; c < NC; ++c) {
-      v[c] = 1;
-      g[c][0] = g[c][1] = g[c][2] = 0;
-    }
-    apply_qop(qop, cd, qd, v, g);
-#pragma unroll
-    for (int c = 0; c < NC; ++c) coef[c * 7] = v[c];
-    Number G[NC][3][3];
-#pragma unroll
-    for (int d = 0; d < NC; ++d)
-#pragma unroll
-      for (int gg = 0; gg < 3; ++gg) {
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          v[c] = 0;
-          g[c][0] = g[c][1] = g[c][2] = 0;
-        }
-        g[d][gg] = 1;
-        apply_qop(qop, cd, qd, v, g);
-#pragma unroll
-        for (int f = 0; f < 3; ++f) G[d][f][gg] = g[d][f];
-      }
-#pragma unroll
-    for (int d = 0; d < NC; ++d) {
-      coef[d * 7 + 1] = G[d][0][0];
-      coef[d * 7 + 2] = G[d][1][1];
-      coef[d * 7 + 3] = G[d][2][2];
-      coef[d * 7 + 4] = G[d][0][1] + G[d][1][0];
-      coef[d * 7 + 5] = G[d][0][2] + G[d][2][0];
-      coef[d * 7 + 6] = G[d][1][2] + G[d][2][1];
-    }
-    if (!active)
-#pragma unroll
-      for (int x = 0; x < NTERM; ++x) coef[x] = 0;
+    DiagonalTerms<QOp>::eval(qop, cd, qd, coef);
   }
-  // matrix (0 SS, 1 SD, 2 DD) per term and direction
-  constexpr int mat[7][3] = {{0, 0, 0}, {2, 0, 0}, {0, 2, 0}, {0, 0, 2}, {1, 1, 0}, {1, 0, 1}, {0, 1, 1}};
+  if (!active)
+#pragma unroll
+    for (int x = 0; x < NTERM; ++x) coef[x] = 0;
+  const Number *SS = s_sq, *SD = s_sq + N * N, *DD = s_sq + 2 * N * N;
   __syncthreads();
 #pragma unroll
   for (int x = 0; x < NTERM; ++x) T.put(x, coef[x]);
   __syncthreads();
-#pragma unroll
-  for (int x = 0; x < NTERM; ++x) coef[x] = T.template line_t<2>(s_sq + mat[x % 7][2] * N * N, T.k, x);
-  __syncthreads();
-#pragma unroll
-  for (int x = 0; x < NTERM; ++x) T.put(x, coef[x]);
-  __syncthreads();
-#pragma unroll
-  for (int x = 0; x < NTERM; ++x) coef[x] = T.template line_t<1>(s_sq + mat[x % 7][1] * N * N, T.j, x);
-  __syncthreads();
-#pragma unroll
-  for (int x = 0; x < NTERM; ++x) T.put(x, coef[x]);
-  __syncthreads();
-  if (!active) return;
-  const uint32_t entry = a.cell_nodes[qidx];
-  const int64_t node = entry & kNodeMaskDev;
+  // z: m and zz share (SS, SS) afterwards
 #pragma unroll
   for (int d = 0; d < NC; ++d) {
-    Number s = 0;
-#pragma unroll
-    for (int x = 0; x < 7; ++x) s += T.template line_t<0>(s_sq + mat[x][0] * N * N, T.i, d * 7 + x);
-    if (!((entry >> (kConstraintShift + d)) & 1u)) a.diag[node * NC + d] += s;
+    Number *c = coef + 7 * d;
+    c[0] = T.template line_t<2>(SS, T.k, 7 * d) + T.template line_t<2>(DD, T.k, 7 * d + 3);
+    c[1] = T.template line_t<2>(SS, T.k, 7 * d + 1);
+    c[2] = T.template line_t<2>(SS, T.k, 7 * d + 2);
+    c[4] = T.template line_t<2>(SS, T.k, 7 * d + 4);
+    c[5] = T.template line_t<2>(SD, T.k, 7 * d + 5);
+    c[6] = T.template line_t<2>(SD, T.k, 7 * d + 6);
+    // the component is done here: without it all components' lines are in
+    // flight at once
+    if constexpr (NC == 3)
+      asm volatile("" : "+v"(c[0]), "+v"(c[1]), "+v"(c[2]), "+v"(c[4]), "+v"(c[5]), "+v"(c[6]) : : "memory");
   }
+  __syncthreads();
+#pragma unroll
+  for (int d = 0; d < NC; ++d)
+#pragma unroll
+    for (int x = 0; x < 7; ++x)
+      if (x != 3) T.put(7 * d + x, coef[7 * d + x]);
+  __syncthreads();
+  // y: (m + zz), yy and yz share SS afterwards, xy and xz share SD
+#pragma unroll
+  for (int d = 0; d < NC; ++d) {
+    Number *c = coef + 7 * d;
+    c[0] = T.template line_t<1>(SS, T.j, 7 * d) + T.template line_t<1>(DD, T.j, 7 * d + 2) +
+           T.template line_t<1>(SD, T.j, 7 * d + 6);
+    c[1] = T.template line_t<1>(SS, T.j, 7 * d + 1);
+    c[4] = T.template line_t<1>(SD, T.j, 7 * d + 4) + T.template line_t<1>(SS, T.j, 7 * d + 5);
+    if constexpr (NC == 3) asm volatile("" : "+v"(c[0]), "+v"(c[1]), "+v"(c[4]) : : "memory");
+  }
+  __syncthreads();
+#pragma unroll
+  for (int d = 0; d < NC; ++d) {
+    T.put(7 * d, coef[7 * d]);
+    T.put(7 * d + 1, coef[7 * d + 1]);
+    T.put(7 * d + 4, coef[7 * d + 4]);
+  }
+  __syncthreads();
+  if (!active) return;
+  const int64_t node = entry & kNodeMaskDev;
+  Number r[NC];
+#pragma unroll
+  for (int d = 0; d < NC; ++d)
+    r[d] = T.template line_t<0>(SS, T.i, 7 * d) + T.template line_t<0>(DD, T.i, 7 * d + 1) +
+           T.template line_t<0>(SD, T.i, 7 * d + 4);
+  if constexpr (kToCells) {
+    store_node<Number, NC>(a.diag + (int64_t)slot * NC, r);
+  } else {
+#pragma unroll
+    for (int d = 0; d < NC; ++d)
+      if (!((entry >> (kConstraintShift + d)) & 1u)) {
+        Number *out = a.diag + node * NC + d;
+        *out = (entry >> 31) ? r[d] : *out + r[d];
+      }
+  }
+}
+
+// GATHER: the nodes' sums in colour order, 1 on constrained components, and the
+// inverse; flags entries that are not positive
+template <typename Number, int NC>
+__global__ void __launch_bounds__(kGatherThreads)
+    diagonal_sums_kernel(GatherTables<Number> g, Number *__restrict__ diag, Number *__restrict__ inv, int64_t n_nodes,
+                         int *flag) {
+  const int64_t node = (int64_t)blockIdx.x * kGatherThreads + threadIdx.x;
+  if (node >= n_nodes) return;
+  const unsigned m = g.cmask[node];
+  Number t[NC] = {}, r[NC];
+  add_contributions<Number, NC>(g.contrib, g.index, g.offsets[node], g.offsets[node + 1], t);
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    if ((m >> c) & 1u) t[c] = Number(1);
+    if (!(t[c] > Number(0))) *flag = 1;
+    r[c] = Number(1) / t[c];
+  }
+  store_node<Number, NC>(diag + node * NC, t);
+  store_node<Number, NC>(inv + node * NC, r);
 }
 
 }  // namespace mfg

@@ -606,3 +606,34 @@ def test_column_kernels(cuda, kind, p, precision, n):
         go.vmult_add(z, x)
         out.append((y, z))
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("kind", ["solid", "solid_folded", "solid_f0", "heat"])
+@pytest.mark.parametrize("p,precision", [(1, mfgpu.FP64), (2, mfgpu.FP64), (3, mfgpu.FP32), (5, mfgpu.FP64), (6, mfgpu.FP32)])
+def test_diagonal_gather_equals_colours(cuda, kind, p, precision):
+    """The diagonal and its inverse from one launch over all cells and the sums
+    per node are bitwise those of the colour launches, and the oracle's; 5 cells
+    leave the last workgroup of Q1 and Q2 partly empty."""
+    print(f"diagonal {kind} p={p} precision={precision}", flush=True)
+    lo, hi, n = [0, 0, 0], [1.0, 0.6, 0.4], [5, 1, 3]
+    nc, fm, cm = (1, 63, 1) if kind == "heat" else (3, 1, 7)
+    om, gm = O.Mesh(lo, hi, n, p, nc, fm, cm), mfgpu.BoxMesh(lo, hi, n, p, nc, fm, cm)
+    if kind == "heat":
+        coef = np.random.default_rng(p).uniform(0.5, 2.0, om.n_cells * (p + 1) ** 3)
+        oo, go = O.Heat(om, dt=0.1, coef=coef), mfgpu.LaplaceOperator(gm, 0.1, coef, precision=precision)
+    else:
+        form = 0 if kind == "solid_f0" else 1
+        u = om.u0(amp=1e-2, noise=1e-5)
+        oo = O.Solid(om, formulation=form, caching=1)
+        oo.cache(u)
+        go = mfgpu.NeoHookOperator(gm, O.MU, O.NU, O.RHO, O.ALPHA1, formulation=form, precision=precision)
+        if kind == "solid_folded":
+            go.set_point_storage(mfgpu.T2_FOLDED)
+        go.cache(dev(u, go.dtype))
+    out = []
+    for sched in (mfgpu.CELLS_GATHER, mfgpu.CELLS_COLOURS):
+        go.set_cell_schedule(sched)
+        go.compute_diagonal()
+        out.append((go.diagonal(), go.get_matrix_diagonal_inverse()))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+    assert rel(out[0][0].double(), oo.diagonal()) < (TOL64 if precision == mfgpu.FP64 else TOL32)
