@@ -23,7 +23,7 @@
 //
 // Measured, point per thread -> column per thread (vmult, colour launches,
 // cubes of about 20M unknowns): heat Q4 FP64 606 -> 452 us, FP32 350 -> 277;
-// Q5 640 -> 524, 424 -> 290; Q6 745 -> 431, 436 -> 267; Q2 FP32 545 -> 454;
+// Q5 640 -> 524, 424 -> 290; Q6 745 -> 431, 436 -> 267 (before the pins below); Q2 FP32 545 -> 454;
 // solid (10 words) Q6 FP64 881 -> 577, FP32 341 -> 281; Q5 560 -> 518,
 // 345 -> 313.  Solid Q4 and below are bound by the gather and scatter of the
 // colour launches either way (Q4 FP64 480 and 481 us, FP32 264 and 288).
@@ -58,6 +58,23 @@ constexpr int column_lds() {
 __device__ inline void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
+}
+
+// Completes x here and keeps the LDS loads that follow after it; no instruction.
+template <typename Number>
+__device__ inline void pin(Number &x) {
+  asm volatile("" : "+v"(x) : : "memory");
+}
+// Whether each line's sum is completed before the loads of the next one.  The
+// compiler otherwise gathers the loads of many lines first.  For the long lines
+// of one component that costs waves (heat FP64 Q5 129 -> 121 VGPRs, 3 -> 4
+// waves per SIMD: 650 -> 576 us at 24.6M unknowns, FP32 354 -> 336; Q6 546 ->
+// 536, 344 -> 316); with three components, whose points have work enough
+// between the loads, the loads in flight are worth more (solid Q6 FP64 727 us,
+// pinned 861), and lines of 5 and less measured the same or 2% slower pinned.
+template <int P, int NC>
+constexpr bool pin_lines() {
+  return NC == 1 && P >= 5;
 }
 
 // The cells [cell_begin, min(cell_begin + column_cells<P>(), cell_end)) on one
@@ -123,6 +140,7 @@ __device__ inline void cell_columns(const QOp &qop, const uint32_t *__restrict__
       Number r = 0;
 #pragma unroll
       for (int a = 0; a < N; ++a) r += ri[a] * xl[(c * N + k) * NL + a];
+      if constexpr (pin_lines<P, NC>()) pin(r);
       v[c][k] = r;
     }
   wave_lds_fence();
@@ -134,6 +152,7 @@ __device__ inline void cell_columns(const QOp &qop, const uint32_t *__restrict__
       Number r = 0;
 #pragma unroll
       for (int a = 0; a < N; ++a) r += rj[a] * yl[(c * N + k) * NL + a * N];
+      if constexpr (pin_lines<P, NC>()) pin(r);
       v[c][k] = r;
     }
   wave_lds_fence();
@@ -182,6 +201,8 @@ __device__ inline void cell_columns(const QOp &qop, const uint32_t *__restrict__
       grad[c][0] = gx;
       grad[c][1] = gy;
       grad[c][2] = gz;
+      if constexpr (pin_lines<P, NC>())
+        asm volatile("" : "+v"(grad[c][0]), "+v"(grad[c][1]), "+v"(grad[c][2]) : : "memory");
     }
     wave_lds_fence();
     qop.apply_grad(cd, qd, grad);
@@ -213,6 +234,7 @@ __device__ inline void cell_columns(const QOp &qop, const uint32_t *__restrict__
       for (int a = 0; a < N; ++a) ry += rj[a] * yl[B + (c * N + k) * NL + a * N];
       const Number s = scale[k] * v[c][k];
       v[c][k] = s + rx + ry + z[c][k];
+      if constexpr (pin_lines<P, NC>()) pin(v[c][k]);
     }
   wave_lds_fence();
   // back to the nodes: z in registers, y, x through LDS
@@ -260,6 +282,7 @@ __device__ inline void cell_columns(const QOp &qop, const uint32_t *__restrict__
       Number r = 0;
 #pragma unroll
       for (int a = 0; a < N; ++a) r += rj[a] * yl[(c * N + k) * NL + a * N];
+      if constexpr (pin_lines<P, NC>()) pin(r);
       v[c][k] = r;
     }
   wave_lds_fence();
