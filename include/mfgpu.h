@@ -542,8 +542,8 @@ int64_t mfg_session_n_dofs(const mfg_session_spec *spec);
  * that small instances overlap, or MFG_SCHEDULE_GATHER (batched vmult only):
  * the instances of one (kind, degree) packed into units of similar work, each
  * unit one launch over the cells of all its instances into their
- * contribution buffers and one launch of the ordered per-node sums, units
- * spread over several streams (each instance's GATHER tables and buffer are
+ * contribution buffers (large batches: on two streams), then one launch per
+ * component count of all instances' ordered per-node sums (each instance's GATHER tables and buffer are
  * its operator's: a batch and a GATHER application of one of its operators on
  * another stream must not overlap).  The tuner times them and the cells per task of every
  * (kind, degree) present, and keeps the fastest.  For the batched solver,

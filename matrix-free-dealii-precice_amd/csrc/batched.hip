@@ -606,10 +606,9 @@ struct TransferGroup {
 // ------------------------------------------------ batch GATHER schedule ---
 // The instances of one (kind, degree) are packed into units of about equal
 // work (a large instance alone, small ones together); a unit is one cells
-// launch over all its instances' cells (batched_cells_kernel) followed, on the
-// same stream, by one segmented per-node sum over its instances
-// (batched_gather_kernel).  Units are spread over streams by work, so the sums
-// of one unit overlap the cells of others.  Each instance's GATHER tables and
+// launch over all its instances' cells (batched_cells_kernel).  After all of
+// them, one launch per component count sums the nodes of the whole batch
+// (batched_gather_kernel).  Each instance's GATHER tables and
 // contribution buffer are its operator's own (built on first use, as
 // mfg_operator_set_cell_schedule builds them): a batch and a GATHER
 // application of one of its operators on another stream must not overlap.
@@ -617,14 +616,33 @@ struct BatchGather {
   struct Unit {
     int code = 0;  // kind * 8 + degree
     std::vector<int> inst;
-    DeviceBuffer tasks, segs, gather_blocks;
+    DeviceBuffer tasks;
     int n_tasks = 0;
-    int64_t blocks = 0;
     double work = 0;
+  };
+  // the launch of per-node sums over all instances of one component count
+  struct Sums {
+    int nc = 0;
+    std::vector<int> inst;
+    DeviceBuffer segs, gather_blocks;
+    int64_t blocks = 0;
   };
   std::vector<OperatorData *> ops;
   int prec = MFG_FP64;
   std::vector<Unit> units;
+  std::vector<Sums> sums;
+  // Streams of the cells launches.  The host, not the GPU, sets a small batch's
+  // time: a launch costs it 3 to 5 us, a stream's fork and join 15.  Two
+  // streams overlap one unit's drain with the next one's fill; below
+  // kOneStreamWork that gains less than the fork and everything stays on the
+  // caller's stream.  Measured, us per application of FP64 batches of 8 to 40
+  // instances, 8 streams with a sums launch per unit / two streams / one:
+  // 0.5M work 145 / 75 / 34; 4.9M 225 / 117 / 75; 9.5M 208 / 97 / 89; 14M
+  // 225 / 121 / 119; 16M 232 / 123 / 125; 131M 622 / 587 / 637; 366M 1503 /
+  // 1488 / 1573.  Four streams with merged sums took 140 at 14M, 1535 at 366M.
+  static constexpr int kStreams = 2;
+  static constexpr double kOneStreamWork = 1.5e7;
+  bool one_stream = false;
   StreamPool pool;
   DeviceBuffer vecs;
   std::vector<const void *> last_src;
@@ -649,6 +667,8 @@ struct BatchGather {
     // unit per (kind, degree), where launches rather than work set the time
     const double cap = std::max(total / (2.0 * kBatchStreams), 5.0e6);
     units.clear();
+    sums.clear();
+    one_stream = total < kOneStreamWork;
     for (auto &kv : by_code) {
       std::vector<int> v = kv.second;
       std::stable_sort(v.begin(), v.end(), [&](int a, int b) { return apply_work(*ops[a]) > apply_work(*ops[b]); });
@@ -681,16 +701,26 @@ struct BatchGather {
       }
       u.n_tasks = (int)tv.size();
       upload_vec(u.tasks, tv, s);
+      work.push_back(u.work);
+      const int nc = ops[u.inst[0]]->nc;
+      int k = 0;
+      while (k < (int)sums.size() && sums[k].nc != nc) ++k;
+      if (k == (int)sums.size()) {
+        sums.emplace_back();
+        sums[k].nc = nc;
+      }
+      sums[k].inst.insert(sums[k].inst.end(), u.inst.begin(), u.inst.end());
+    }
+    for (Sums &x : sums) {
       std::vector<GatherBlock> gb;
-      for (size_t k = 0; k < u.inst.size(); ++k)
-        for (int64_t v = 0; v < ops[u.inst[k]]->n_nodes; v += kGatherThreads)
+      for (size_t k = 0; k < x.inst.size(); ++k)
+        for (int64_t v = 0; v < ops[x.inst[k]]->n_nodes; v += kGatherThreads)
           gb.push_back(GatherBlock{(int32_t)k, (int32_t)v});
       MFG_REQUIRE(gb.size() < (size_t)INT32_MAX, MFG_ERR_ARGUMENT, "batch unit too large for one gather launch");
-      u.blocks = (int64_t)gb.size();
-      upload_vec(u.gather_blocks, gb, s);
-      work.push_back(u.work);
+      x.blocks = (int64_t)gb.size();
+      upload_vec(x.gather_blocks, gb, s);
     }
-    pool.build(work, kBatchStreams);
+    if (!one_stream) pool.build(work, kStreams);
   }
 
   BatchGather(const std::vector<OperatorData *> &o, hipStream_t s) : ops(o) {
@@ -714,9 +744,9 @@ struct BatchGather {
       v[i].slots = ops[i]->gather_slots();
     }
     upload_vec(vecs, v, s);
-    for (Unit &u : units) {
+    for (Sums &x : sums) {
       std::vector<GatherSeg<Number>> g;
-      for (int i : u.inst) {
+      for (int i : x.inst) {
         const OperatorData &op = *ops[i];
         GatherSeg<Number> e;
         e.tables = gather_tables<Number>(op);
@@ -725,7 +755,7 @@ struct BatchGather {
         e.n_nodes = op.n_nodes;
         g.push_back(e);
       }
-      upload_vec(u.segs, g, s);
+      upload_vec(x.segs, g, s);
     }
     last_src = sv;
     last_dst = dv;
@@ -756,26 +786,34 @@ struct BatchGather {
   }
 
   template <typename Number>
+  void launch_sums(const Sums &x, int fix, hipStream_t s) const {
+    if (x.nc == 1)
+      batched_gather_kernel<Number, 1><<<(unsigned)x.blocks, kGatherThreads, 0, s>>>(
+          x.segs.as<GatherSeg<Number>>(), x.gather_blocks.as<GatherBlock>(), fix);
+    else
+      batched_gather_kernel<Number, 3><<<(unsigned)x.blocks, kGatherThreads, 0, s>>>(
+          x.segs.as<GatherSeg<Number>>(), x.gather_blocks.as<GatherBlock>(), fix);
+    MFG_HIP(hipGetLastError());
+  }
+
+  template <typename Number>
   void apply_t(const void *inst_table, const void *const *src, void *const *dst, bool add, hipStream_t s) {
     set_vectors<Number>(src, dst, s);
     const int fix = add ? 2 : 1;
-    pool.run(s, [&](int ui, hipStream_t us) {
+    auto cells = [&](int ui, hipStream_t us) {
       const Unit &u = units[ui];
-      const int kind = u.code >> 3;
-      switch (kind) {
+      switch (u.code >> 3) {
         case kSolidF1: launch_kind<kSolidF1, Number>(u, inst_table, us); break;
         case kSolidF1G: launch_kind<kSolidF1G, Number>(u, inst_table, us); break;
         case kSolidF0: launch_kind<kSolidF0, Number>(u, inst_table, us); break;
         default: launch_kind<kHeat, Number>(u, inst_table, us); break;
       }
-      if (kind == kHeat)
-        batched_gather_kernel<Number, 1><<<(unsigned)u.blocks, kGatherThreads, 0, us>>>(
-            u.segs.as<GatherSeg<Number>>(), u.gather_blocks.as<GatherBlock>(), fix);
-      else
-        batched_gather_kernel<Number, 3><<<(unsigned)u.blocks, kGatherThreads, 0, us>>>(
-            u.segs.as<GatherSeg<Number>>(), u.gather_blocks.as<GatherBlock>(), fix);
-      MFG_HIP(hipGetLastError());
-    });
+    };
+    if (one_stream)
+      for (int ui = 0; ui < (int)units.size(); ++ui) cells(ui, s);
+    else
+      pool.run(s, cells);
+    for (const Sums &x : sums) launch_sums<Number>(x, fix, s);
   }
 
   void apply(const void *inst_table, const void *const *src, void *const *dst, bool add, hipStream_t s) {

@@ -207,8 +207,8 @@ __global__ void __launch_bounds__(kBatchThreads, WAVES) batched_apply_kernel(Bat
 }
 
 // ------------------------------------------------------ GATHER schedule ---
-// One launch per (kind, degree) present: every cell of every instance of that
-// kind and degree, a workgroup per task (DefaultCPB cells of one instance),
+// A launch covers every cell of some instances of one kind and degree, a
+// workgroup per task (DefaultCPB cells of one instance),
 // with the register allocation and the cell arithmetic of the single-operator
 // kernels.  Each point stores its contribution into its instance's
 // contribution buffer: no colours and no waits between workgroups.  Then

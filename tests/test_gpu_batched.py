@@ -74,6 +74,30 @@ def test_batched_vmult_equals_per_instance(cuda, precision, storage, schedule):
         assert err < (1e-6 if precision == mfgpu.FP32 else 1e-14), (i, err)
 
 
+# GATHER batches whose cells run on the caller's stream (work below 15M words)
+# and over two streams (above); two units of one (kind, degree) in the latter
+@pytest.mark.parametrize("precision", [mfgpu.FP64, mfgpu.FP32])
+@pytest.mark.parametrize("specs", [[("solid", [1, 1, 1], 1, 1)],
+                                   [("heat", [9, 8, 7], 3, 1), ("solid", [9, 7, 6], 2, 1), ("heat", [7, 7, 5], 3, 1)],
+                                   [("solid", [18, 17, 16], 3, 1), ("heat", [13, 12, 11], 5, 1),
+                                    ("solid", [19, 16, 17], 3, 1), ("solid", [15, 14, 13], 2, 0)]])
+def test_batched_gather_streams(cuda, specs, precision):
+    print(f"batched gather {len(specs)} instances precision={precision}", flush=True)
+    ops, meshes = make_ops(specs, precision, mfgpu.T2_GRADIENT)
+    srcs = [mfgpu.fill_uniform(100 + i, torch.empty(m.n_dofs, dtype=ops[0].dtype, device="cuda"))
+            for i, m in enumerate(meshes)]
+    ref = [torch.empty_like(s) for s in srcs]
+    for op, s, r in zip(ops, srcs, ref):
+        op.vmult(r, s)
+    b = mfgpu.Batch(ops)
+    b.set_schedule(mfgpu.SCHEDULE_GATHER)
+    for _ in range(3):
+        out = [torch.full_like(s, float("nan")) for s in srcs]
+        b.vmult(out, srcs)
+        b.synchronize()
+        assert all(torch.equal(o, r) for o, r in zip(out, ref))
+
+
 def test_batched_cells_per_task_and_tuner(cuda):
     ops, meshes = make_ops(SPECS, mfgpu.FP32)
     srcs = [mfgpu.fill_uniform(200 + i, torch.empty(m.n_dofs, dtype=torch.float32, device="cuda"))
