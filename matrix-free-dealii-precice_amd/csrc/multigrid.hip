@@ -155,15 +155,6 @@ void vec_convert(int prec_dst, void *dst, int prec_src, const void *src, int64_t
     MFG_HIP(hipGetLastError());                                                                \
   } while (0)
 
-template <typename T>
-static void xpby_t(void *p, const void *d, double beta, int64_t n, hipStream_t s) {
-  xpby_kernel<T><<<grid_for(n), 256, 0, s>>>((T *)p, (const T *)d, beta, n);
-}
-void vec_xpby(int prec, void *p, const void *d, double beta, int64_t n, hipStream_t s) {
-  if (prec == MFG_FP64) xpby_t<double>(p, d, beta, n, s);
-  else xpby_t<float>(p, d, beta, n, s);
-  MFG_HIP(hipGetLastError());
-}
 void Reducer::xpby_dev(int prec, void *p, const void *z, int64_t n, hipStream_t s) {
   if (prec == MFG_FP64) xpby_dev_kernel<double><<<grid_for(n), 256, 0, s>>>((double *)p, (const double *)z, scal, n);
   else xpby_dev_kernel<float><<<grid_for(n), 256, 0, s>>>((float *)p, (const float *)z, scal, n);

@@ -52,7 +52,6 @@ struct Reducer {
 
 void vec_fill(int prec, void *x, int64_t n, double v, hipStream_t s);
 void vec_convert(int prec_dst, void *dst, int prec_src, const void *src, int64_t n, hipStream_t s);
-void vec_xpby(int prec, void *p, const void *d, double beta, int64_t n, hipStream_t s);
 void vec_residual(int prec, void *t, const void *b, int64_t n, hipStream_t s);
 void vec_add_scaled(int prec, void *y, const void *a, double sc, const void *b, int64_t n, hipStream_t s);
 

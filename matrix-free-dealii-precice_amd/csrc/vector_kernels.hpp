@@ -107,19 +107,6 @@ __global__ void __launch_bounds__(kRedThreads) dot_partial_kernel(const T *a, co
   block_reduce_store<T>(v, partials);
 }
 
-static __global__ void __launch_bounds__(kRedThreads) sum_partials_kernel(const double *partials, int n, double *out) {
-  __shared__ double s[kRedThreads];
-  double v = 0;
-  for (int i = threadIdx.x; i < n; i += kRedThreads) v += partials[i];
-  s[threadIdx.x] = v;
-  __syncthreads();
-  for (int w = kRedThreads / 2; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) s[threadIdx.x] += s[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) *out = s[0];
-}
-
 // ------------------------------------------ device-resident CG scalars ---
 // A block of scalars that the reduction epilogues and the update kernels read
 // and write, so that a CG iteration computes its step lengths on the device
@@ -445,26 +432,6 @@ __global__ void __launch_bounds__(kRedThreads)
 template <typename T>
 __global__ void xpby_dev_kernel(T *p, const T *d, const double *scal, int64_t n) {
   const double beta = scal[kSlotBeta];
-  MFG_GRID_STRIDE(i, n) p[i] = (T)((double)d[i] + beta * (double)p[i]);
-}
-
-// x += alpha p ; r -= alpha h ; partial r.r
-template <typename T>
-__global__ void __launch_bounds__(kRedThreads) cg_update_kernel(T *x, T *r, const T *p, const T *h, double alpha,
-                                                                 int64_t n, double *partials) {
-  double v = 0;
-  MFG_GRID_STRIDE(i, n) {
-    x[i] = (T)((double)x[i] + alpha * (double)p[i]);
-    const T ri = (T)((double)r[i] - alpha * (double)h[i]);
-    r[i] = ri;
-    v += (double)ri * (double)ri;
-  }
-  block_reduce_store<T>(v, partials);
-}
-
-// p = d + beta p
-template <typename T>
-__global__ void xpby_kernel(T *p, const T *d, double beta, int64_t n) {
   MFG_GRID_STRIDE(i, n) p[i] = (T)((double)d[i] + beta * (double)p[i]);
 }
 
