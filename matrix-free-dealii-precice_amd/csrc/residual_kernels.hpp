@@ -130,7 +130,7 @@ __device__ inline bool residual_point(const ResidualArgs<Number> &a, int formula
 // Jacobian, b and tau: Q4 64x16x16 cells 212 -> 162 us, Q3 cubes of 20K, 0.3M
 // and 3M unknowns 117 -> 28, 124 -> 40, 224 -> 149 us; Q6 155 -> 33, 159 -> 46,
 // 272 -> 236.  Bounding the registers to 4 waves per SIMD instead of 3 (12 to
-// 30 spilled) is not faster at any degree.
+// 30 spilled) was not faster at any degree.
 template <int P, int CPB, int KIND, bool kToCells, typename Number>
 __global__ void __launch_bounds__((block_threads<P, CPB>())) residual_cells(ResidualArgs<Number> a) {
   constexpr int N = P + 1, N3 = N * N * N, NL = N * N;
@@ -226,12 +226,21 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) residual_cells(Resi
 #pragma unroll
     for (int f = 0; f < 3; ++f) T.put(g_slot(3 * c + f), grad[c][f]);
   __syncthreads();
+  // Colour launches: each component's sum is completed before the loads of the
+  // next one.  Without it the loads of all 9 lines come first, at 138 (Q4) and
+  // 156 VGPRs (Q6), 3 waves per SIMD; with it 104 each, 4 waves.  3M
+  // unknowns: Q4 164 -> 159 us, Q5 168 -> 169, Q6 241 -> 221.  Below Q4 and in
+  // the GATHER form the loads in flight are worth more (Q3 147 -> 153, Q2 198
+  // -> 204; GATHER 1% slower), as they are in the forward lines of any degree.
+  constexpr bool kPin = P >= 4 && !kToCells;
   Number r[3];
 #pragma unroll
-  for (int c = 0; c < 3; ++c)
+  for (int c = 0; c < 3; ++c) {
     r[c] = val[c] + T.template line_t<0>(s_colloc, T.i, g_slot(3 * c + 0)) +
            T.template line_t<1>(s_colloc, T.j, g_slot(3 * c + 1)) +
            T.template line_t<2>(s_colloc, T.k, g_slot(3 * c + 2));
+    if constexpr (kPin) asm volatile("" : "+v"(r[c]) : : "memory");
+  }
 #pragma unroll
   for (int c = 0; c < 3; ++c) T.put(6 + c, r[c]);
   __syncthreads();
