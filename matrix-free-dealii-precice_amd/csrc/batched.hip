@@ -618,6 +618,7 @@ struct BatchGather {
     std::vector<int> inst;
     DeviceBuffer tasks;
     int n_tasks = 0;
+    bool columns = false;  // cells by batched_columns_kernel
     double work = 0;
   };
   // the launch of per-node sums over all instances of one component count
@@ -647,6 +648,32 @@ struct BatchGather {
   DeviceBuffer vecs;
   std::vector<const void *> last_src;
   std::vector<void *> last_dst;
+
+  // The rule of the single operators, from a full round of the GPU (1024 waves
+  // at one wave per SIMD) on: below, other units run beside this one and the
+  // point kernels leave them more of the chip (40 operators of 16M work with one
+  // Q6 solid unit of 704 cells: 123 us, with columns 127).
+  template <typename Number>
+  bool unit_columns(const Unit &u) const {
+    const int kind = u.code >> 3, p = u.code & 7, cc = 64 / ((p + 1) * (p + 1));
+    int64_t cells = 0, waves = 0;
+    for (int i : u.inst) {
+      if (kind == kHeat && !ops[i]->affine_ref) return false;
+      cells += ops[i]->n_cells;
+      waves += (ops[i]->n_cells + cc - 1) / cc;
+    }
+    const int nc = (int)std::min<int64_t>(cells, INT32_MAX), w = (int)std::min<int64_t>(waves, INT32_MAX);
+    if (w < 1024) return false;
+    const bool heat = kind == kHeat, f1 = kind != kSolidF0;
+    switch (p) {
+      case 1: return columns_pay<1, Number>(heat, f1, nc, w);
+      case 2: return columns_pay<2, Number>(heat, f1, nc, w);
+      case 3: return columns_pay<3, Number>(heat, f1, nc, w);
+      case 4: return columns_pay<4, Number>(heat, f1, nc, w);
+      case 5: return columns_pay<5, Number>(heat, f1, nc, w);
+      default: return columns_pay<6, Number>(heat, f1, nc, w);
+    }
+  }
 
   template <typename Number>
   void build_t(hipStream_t s) {
@@ -687,10 +714,14 @@ struct BatchGather {
     std::vector<double> work;
     for (Unit &u : units) {
       std::vector<BatchTask> tv;
+      const int p = u.code & 7;
+      u.columns = unit_columns<Number>(u);
+      const int cpb = u.columns ? 64 / ((p + 1) * (p + 1))
+                      : p == 1  ? DefaultCPB<1, Number>::value
+                      : p == 2  ? DefaultCPB<2, Number>::value
+                                : 1;
       for (int i : u.inst) {
         const OperatorData &op = *ops[i];
-        const int p = op.p;
-        const int cpb = p == 1 ? DefaultCPB<1, Number>::value : p == 2 ? DefaultCPB<2, Number>::value : 1;
         for (int c = 0; c < op.n_cells; c += cpb) {
           BatchTask t{};
           t.inst = i;
@@ -768,6 +799,13 @@ struct BatchGather {
     a.inst = (const BatchInst<Number> *)inst_table;
     a.tasks = u.tasks.as<BatchTask>();
     a.vecs = vecs.as<GatherVecs<Number>>();
+    if constexpr (KIND == kHeat ? has_heat_columns<P, Number>() : has_solid_columns<P, Number>(KIND != kSolidF0)) {
+      if (u.columns) {
+        batched_columns_kernel<P, KIND, Number><<<u.n_tasks, 64, 0, s>>>(a);
+        MFG_HIP(hipGetLastError());
+        return;
+      }
+    }
     batched_cells_kernel<P, CPB, KIND, Number><<<u.n_tasks, block_threads<P, CPB>(), 0, s>>>(a);
     MFG_HIP(hipGetLastError());
   }

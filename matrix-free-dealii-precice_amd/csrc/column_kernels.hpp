@@ -39,6 +39,43 @@ constexpr int column_cells() {
   return 64 / ((P + 1) * (P + 1));
 }
 
+// whether there is a column kernel for the heat operator
+template <int P, typename Number>
+constexpr bool has_heat_columns() {
+  return P >= 2 || sizeof(Number) == 4;
+}
+// whether there is a column kernel for the solid operators of a formulation
+template <int P, typename Number>
+constexpr bool has_solid_columns(bool formulation1) {
+  return (P == 6 && sizeof(Number) == 8) || (P >= 5 && formulation1);
+}
+// Whether a launch of the heat operator on affine cells or of a tensor2 solid
+// operator over n_cells cells (waves: workgroups of the column kernel) takes the
+// column kernels; the results are the same bit for bit.  They hold 64 / (p+1)^2
+// cells per wave at 1 to 4 waves per SIMD, so they need that many waves to fill
+// the 1024 SIMDs; with fewer, the point-per-thread kernels spread the same
+// cells over more waves.
+// Measured over cubes of 2e4 to 2e7 unknowns, in one launch (GATHER) and in 8
+// colours, times as point -> column in us:
+//  - heat on affine cells: equal at about 600 waves (Q4 7.8 -> 9.2 at 172, Q2
+//    8.4 -> 8.4 at 392), 7 to 50 % faster from 1000 (Q4 16.6 -> 14.8 at 1688,
+//    Q6 16.8 -> 15.0 at 1000).  FP64 Q1 to Q3 is bound by its vector traffic
+//    once that leaves the caches: Q2 151 -> 143 at 46,656 cells a launch but
+//    906 -> 943 at 314,432, Q3 108 -> 103 at 13,824 but 583 -> 608 at 91,125;
+//    Q1 gains nothing at any size.
+//  - solid Q6 FP64: 175 -> 146 at 614 waves, 881 -> 577 at 3724 (formulation 0
+//    213 -> 176 and 1027 -> 743).
+//  - solid Q5 and Q6 FP32, Q5 FP64, formulation 1: slower at 614 to 1000 waves
+//    (Q6 FP32 91 -> 118, Q5 FP64 113.6 -> 114), faster at 1728 and above (Q6
+//    FP32 36.6 -> 30.7, Q5 FP64 48.5 -> 45.9 at 2744).
+//  - solid up to Q4: not faster at the large sizes.
+template <int P, typename Number>
+inline bool columns_pay(bool heat, bool formulation1, int n_cells, int waves) {
+  constexpr bool fp64 = sizeof(Number) == 8;
+  if (heat) return has_heat_columns<P, Number>() && waves >= 768 && !(fp64 && P <= 3 && n_cells > 65536);
+  return has_solid_columns<P, Number>(formulation1) && waves >= (fp64 && P == 6 ? 512 : 1536);
+}
+
 // LDS values of one cell: 2 NC N^3 (the point values or x gradients, and the y
 // gradients), padded so that the lines which the cells of a wave read together
 // start in different banks: the stride is 5, 9 and 17 modulo 32 values for

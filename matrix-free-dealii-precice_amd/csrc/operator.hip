@@ -78,37 +78,12 @@ static void with_qop(const OperatorData &op, int m, F fn) {
   }
 }
 
-// Whether a launch over n_cells cells takes the column kernels (the results
-// are the same bit for bit).  They hold 64 / (p+1)^2 cells per wave at 1 to 4
-// waves per SIMD, so they need that many waves to fill the 1024 SIMDs; with
-// fewer, the point-per-thread kernels spread the same cells over more waves.
-// Measured over cubes of 2e4 to 2e7 unknowns, in one launch (GATHER) and in 8
-// colours, times as point -> column in us:
-//  - heat on affine cells: equal at about 600 waves (Q4 7.8 -> 9.2 at 172, Q2
-//    8.4 -> 8.4 at 392), 7 to 50 % faster from 1000 (Q4 16.6 -> 14.8 at 1688,
-//    Q6 16.8 -> 15.0 at 1000).  FP64 Q1 to Q3 is bound by its vector traffic
-//    once that leaves the caches: Q2 151 -> 143 at 46,656 cells a launch but
-//    906 -> 943 at 314,432, Q3 108 -> 103 at 13,824 but 583 -> 608 at 91,125;
-//    Q1 gains nothing at any size.
-//  - solid Q6 FP64: 175 -> 146 at 614 waves, 881 -> 577 at 3724 (formulation 0
-//    213 -> 176 and 1027 -> 743).
-//  - solid Q5 and Q6 FP32, Q5 FP64, formulation 1: slower at 614 to 1000 waves
-//    (Q6 FP32 91 -> 118, Q5 FP64 113.6 -> 114), faster at 1728 and above (Q6
-//    FP32 36.6 -> 30.7, Q5 FP64 48.5 -> 45.9 at 2744).
-//  - solid up to Q4: not faster at the large sizes.
-template <int P, typename Number>
-constexpr bool has_heat_columns() {
-  return P >= 2 || sizeof(Number) == 4;
-}
+// Whether a launch over n_cells cells of op takes the column kernels
 template <int P, typename Number>
 static bool use_columns(const OperatorData &op, int n_cells) {
-  constexpr bool fp64 = sizeof(Number) == 8;
-  const int waves = blocks_for(n_cells, column_cells<P>());
-  if (op.kind == 1)
-    return has_heat_columns<P, Number>() && op.affine_ref && waves >= 768 && !(fp64 && P <= 3 && n_cells > 65536);
-  if (P < 5 || op.sp.caching != MFG_CACHING_TENSOR2) return false;
-  if (fp64 && P == 6) return waves >= 512;
-  return op.sp.formulation == 1 && waves >= 1536;
+  if (op.kind == 1 ? !op.affine_ref : op.sp.caching != MFG_CACHING_TENSOR2) return false;
+  return columns_pay<P, Number>(op.kind == 1, op.sp.formulation == 1, n_cells,
+                                blocks_for(n_cells, column_cells<P>()));
 }
 // fn(q) with the quadrature op of the column kernels, where use_columns holds
 template <int P, typename Number, class F>

@@ -98,6 +98,33 @@ def test_batched_gather_streams(cuda, specs, precision):
         assert all(torch.equal(o, r) for o, r in zip(out, ref))
 
 
+# GATHER units with enough cells for a thread per z column (1024 waves, 1536 of
+# the Q5 and FP32 Q6 solids) beside ones without
+@pytest.mark.parametrize("precision", [mfgpu.FP64, mfgpu.FP32])
+@pytest.mark.parametrize("specs", [[("solid", [11, 10, 10], 6, 1), ("solid", [2, 3, 2], 6, 0),
+                                    ("heat", [13, 13, 13], 4, 1)],
+                                   [("solid", [11, 11, 9], 6, 0), ("solid", [3, 2, 2], 6, 0),
+                                    ("heat", [9, 9, 13], 5, 1)],
+                                   [("solid", [13, 11, 11], 5, 1), ("heat", [11, 10, 10], 6, 1),
+                                    ("heat", [20, 19, 20], 2, 1)]])
+@pytest.mark.parametrize("storage", [mfgpu.T2_GRADIENT, mfgpu.T2_FOLDED])
+def test_batched_gather_columns(cuda, specs, precision, storage):
+    print(f"batched gather columns {specs} precision={precision} storage={storage}", flush=True)
+    ops, meshes = make_ops(specs, precision, storage)
+    srcs = [mfgpu.fill_uniform(100 + i, torch.empty(m.n_dofs, dtype=ops[0].dtype, device="cuda"))
+            for i, m in enumerate(meshes)]
+    ref = [torch.empty_like(s) for s in srcs]
+    for op, s, r in zip(ops, srcs, ref):
+        op.vmult(r, s)
+    b = mfgpu.Batch(ops)
+    b.set_schedule(mfgpu.SCHEDULE_GATHER)
+    for _ in range(2):
+        out = [torch.full_like(s, float("nan")) for s in srcs]
+        b.vmult(out, srcs)
+        b.synchronize()
+        assert all(torch.equal(o, r) for o, r in zip(out, ref))
+
+
 def test_batched_cells_per_task_and_tuner(cuda):
     ops, meshes = make_ops(SPECS, mfgpu.FP32)
     srcs = [mfgpu.fill_uniform(200 + i, torch.empty(m.n_dofs, dtype=torch.float32, device="cuda"))
