@@ -545,7 +545,9 @@ int64_t mfg_session_n_dofs(const mfg_session_spec *spec);
  * contribution buffers (large batches: on two streams), then one launch per
  * component count of all instances' ordered per-node sums (each instance's GATHER tables and buffer are
  * its operator's: a batch and a GATHER application of one of its operators on
- * another stream must not overlap).  The tuner times them and the cells per task of every
+ * another stream must not overlap).  An operator may appear several times in
+ * a batch, with other vectors (the GATHER schedule then holds a contribution
+ * buffer more for each repetition).  The tuner times them and the cells per task of every
  * (kind, degree) present, and keeps the fastest.  For the batched solver,
  * STREAMS runs every instance's own mfg_cg_solve / mfg_mg_vmult on worker
  * threads with a stream each. */

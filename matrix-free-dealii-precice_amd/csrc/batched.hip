@@ -612,6 +612,8 @@ struct TransferGroup {
 // contribution buffer are its operator's own (built on first use, as
 // mfg_operator_set_cell_schedule builds them): a batch and a GATHER
 // application of one of its operators on another stream must not overlap.
+// An operator may appear several times (several right-hand sides): all cells
+// run before the sums, so each further appearance has a buffer of the batch's.
 struct BatchGather {
   struct Unit {
     int code = 0;  // kind * 8 + degree
@@ -630,6 +632,8 @@ struct BatchGather {
   };
   std::vector<OperatorData *> ops;
   int prec = MFG_FP64;
+  std::vector<DeviceBuffer> repeats;  // contributions of an operator's second and later appearances
+  std::vector<void *> contrib;        // per instance
   std::vector<Unit> units;
   std::vector<Sums> sums;
   // Streams of the cells launches.  The host, not the GPU, sets a small batch's
@@ -688,6 +692,11 @@ struct BatchGather {
       }
       by_code[code_of(op)].push_back(i);
       total += apply_work(op);
+      contrib.push_back(op.contrib.ptr);
+      if (std::find(ops.begin(), ops.begin() + i, &op) != ops.begin() + i) {
+        repeats.emplace_back(op.contrib.bytes);
+        contrib.back() = repeats.back().ptr;
+      }
     }
     // units of at most cap work (one instance at least), largest first; the
     // floor (about 2^18 solid quadrature points) keeps small batches at one
@@ -771,7 +780,7 @@ struct BatchGather {
       MFG_REQUIRE(src[i] && dst[i], MFG_ERR_ARGUMENT, "null vector");
       MFG_REQUIRE(src[i] != dst[i], MFG_ERR_ARGUMENT, "vmult needs distinct source and destination");
       v[i].src = (const Number *)src[i];
-      v[i].contrib = ops[i]->contrib.as<Number>();
+      v[i].contrib = (Number *)contrib[i];
       v[i].slots = ops[i]->gather_slots();
     }
     upload_vec(vecs, v, s);
@@ -781,6 +790,7 @@ struct BatchGather {
         const OperatorData &op = *ops[i];
         GatherSeg<Number> e;
         e.tables = gather_tables<Number>(op);
+        e.tables.contrib = (const Number *)contrib[i];
         e.src = (const Number *)src[i];
         e.dst = (Number *)dst[i];
         e.n_nodes = op.n_nodes;
@@ -911,6 +921,7 @@ struct BatchVmult {
     g->build(tu, stream);
     group = std::move(g);
     gather.reset();
+    pool.assign.clear();  // the chains follow the operators' schedules
     last_src.clear();
     last_dst.clear();
     record_versions();
@@ -925,8 +936,11 @@ struct BatchVmult {
     last_dst = d;
   }
   StreamPool pool;
+  std::vector<std::vector<int>> chains;  // instances that follow each other on one of the pool's streams
   // STREAMS: every instance's own apply (its default cell schedule) on the
-  // pool's streams; bitwise the per-instance result
+  // pool's streams; bitwise the per-instance result.  The appearances of one
+  // operator with the GATHER schedule share its contribution buffer and stay on
+  // one stream.
   void apply_streams(const void *const *src, void *const *dst, bool add) {
     const size_t n = group->ops.size();
     for (size_t i = 0; i < n; ++i) {
@@ -935,10 +949,26 @@ struct BatchVmult {
     }
     if (pool.assign.empty()) {
       std::vector<double> w;
-      for (const OperatorData *op : group->ops) w.push_back(apply_work(*op));
+      std::map<const OperatorData *, size_t> chain_of;
+      chains.clear();
+      for (size_t i = 0; i < n; ++i) {
+        const OperatorData *op = group->ops[i];
+        const bool shared = op->cell_schedule == MFG_CELLS_GATHER;
+        const auto at = chain_of.find(op);
+        if (shared && at != chain_of.end()) {
+          chains[at->second].push_back((int)i);
+          w[at->second] += apply_work(*op);
+          continue;
+        }
+        if (shared) chain_of[op] = chains.size();
+        chains.push_back({(int)i});
+        w.push_back(apply_work(*op));
+      }
       pool.build(w, kBatchStreams);
     }
-    pool.run(stream, [&](int i, hipStream_t s) { group->ops[i]->apply(src[i], dst[i], add, s); });
+    pool.run(stream, [&](int c, hipStream_t s) {
+      for (int i : chains[c]) group->ops[i]->apply(src[i], dst[i], add, s);
+    });
   }
   void apply_gather(const void *const *src, void *const *dst, bool add) {
     if (!gather) {

@@ -125,6 +125,42 @@ def test_batched_gather_columns(cuda, specs, precision, storage):
         assert all(torch.equal(o, r) for o, r in zip(out, ref))
 
 
+@pytest.mark.parametrize("schedule", [mfgpu.SCHEDULE_COLOUR, mfgpu.SCHEDULE_QUEUE, mfgpu.SCHEDULE_STREAMS,
+                                      mfgpu.SCHEDULE_GATHER])
+@pytest.mark.parametrize("cells", [mfgpu.CELLS_GATHER, mfgpu.CELLS_COLOURS])
+@pytest.mark.parametrize("big", [False, True])
+def test_batch_of_repeated_operators(cuda, schedule, cells, big):
+    """An operator with several right-hand sides in one batch: every appearance
+    gives its own result, in one unit (the cells of one kind and degree), beside
+    other units, and (big: above 15M words of work) over two streams."""
+    print(f"repeated operators schedule={schedule} cells={cells} big={big}", flush=True)
+    specs = [("solid", [18, 17, 16] if big else [4, 3, 3], 3, 1), ("heat", [5, 4, 3], 2, 1), ("heat", [9, 8, 9], 4, 1)]
+    ops, meshes = make_ops(specs, mfgpu.FP64, mfgpu.T2_GRADIENT)
+    for op in ops:
+        op.set_cell_schedule(cells)
+    order = [0, 1, 0, 2, 1, 0, 0]
+    rep = [ops[k] for k in order]
+    srcs = [mfgpu.fill_uniform(300 + i, torch.empty(meshes[k].n_dofs, dtype=torch.float64, device="cuda"))
+            for i, k in enumerate(order)]
+    ref = [torch.empty_like(s) for s in srcs]
+    for op, s, r in zip(rep, srcs, ref):
+        op.vmult(r, s)
+    b = mfgpu.Batch(rep)
+    b.set_schedule(schedule)
+    for _ in range(2):
+        out = [torch.full_like(s, float("nan")) for s in srcs]
+        b.vmult(out, srcs)
+        b.synchronize()
+        assert all(torch.equal(o, r) for o, r in zip(out, ref))
+    acc = [mfgpu.fill_uniform(400 + i, torch.empty_like(s)) for i, s in enumerate(srcs)]
+    want = [a.clone() for a in acc]
+    for op, s, w in zip(rep, srcs, want):
+        op.vmult_add(w, s)
+    b.vmult_add(acc, srcs)
+    b.synchronize()
+    assert all(torch.equal(o, r) for o, r in zip(acc, want))
+
+
 def test_batched_cells_per_task_and_tuner(cuda):
     ops, meshes = make_ops(SPECS, mfgpu.FP32)
     srcs = [mfgpu.fill_uniform(200 + i, torch.empty(m.n_dofs, dtype=torch.float32, device="cuda"))
