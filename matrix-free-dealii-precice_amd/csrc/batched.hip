@@ -1517,19 +1517,51 @@ struct BatchSolver {
     check_error();
   }
 
+  // Spreads the instances over the workers.  Instances that share an operator
+  // (one system with several right-hand sides, say) share its stream, its
+  // contribution buffer and its transfers' scratch: they follow each other on
+  // one worker.
+  void ensure_pool() {
+    if (!pool.assign.empty()) return;
+    std::vector<int> root(n);  // disjoint sets of instances, by their first one
+    std::map<const void *, int> seen;
+    auto find = [&](int i) {
+      while (root[i] != i) i = root[i];
+      return i;
+    };
+    for (int i = 0; i < n; ++i) {
+      root[i] = i;
+      std::vector<const void *> used{fine[i], mg[i]};
+      for (const MGLevel &L : mg[i]->levels) used.push_back(L.op);
+      for (const void *o : used) {
+        const int a = find(i), b = find(seen.emplace(o, i).first->second);
+        root[std::max(a, b)] = std::min(a, b);
+      }
+    }
+    std::vector<std::vector<int>> sets;
+    std::vector<int> set_of(n, -1);
+    std::vector<double> w;
+    for (int i = 0; i < n; ++i) {
+      const int r = find(i);
+      if (set_of[r] < 0) {
+        set_of[r] = (int)sets.size();
+        sets.emplace_back();
+        w.push_back(0);
+      }
+      sets[set_of[r]].push_back(i);
+      w[set_of[r]] += apply_work(*fine[i]);
+      for (MGLevel &L : mg[i]->levels) w[set_of[r]] += 11.0 * apply_work(*L.op);  // operator applications per cycle
+    }
+    pool.build(w, kBatchStreams);
+    for (std::vector<int> &v : pool.assign) {
+      std::vector<int> ins;
+      for (int k : v) ins.insert(ins.end(), sets[k].begin(), sets[k].end());
+      v = ins;
+    }
+  }
   // Runs f(i) for every instance on the pool's worker threads, instance i's
   // operators (fine and levels) switched to its worker's stream meanwhile.
   // Errors of one instance go to status[i] (when given) and stop nothing else.
-  void ensure_pool() {
-    if (!pool.assign.empty()) return;
-    std::vector<double> w;
-    for (int i = 0; i < n; ++i) {
-      double x = apply_work(*fine[i]);
-      for (MGLevel &L : mg[i]->levels) x += 11.0 * apply_work(*L.op);  // operator applications per cycle
-      w.push_back(x);
-    }
-    pool.build(w, kBatchStreams);
-  }
   template <class F>
   void run_concurrent(F &&f, int32_t *status, std::string &first_error) {
     ensure_pool();

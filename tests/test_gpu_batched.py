@@ -265,6 +265,41 @@ def test_batched_cg_equals_per_instance(cuda, schedule):
     assert all(s == 0 for s in status2) and all(i.iterations == 0 for i in infos2)
 
 
+@pytest.mark.parametrize("schedule", [mfgpu.SCHEDULE_COLOUR, mfgpu.SCHEDULE_STREAMS])
+def test_batched_solver_of_shared_operators(cuda, schedule):
+    """Several right-hand sides of one system (a hierarchy object each over the
+    same operators and transfers), beside other systems."""
+    print(f"batched solver of shared operators schedule={schedule}", flush=True)
+    inst = instances(ISPECS[:4])
+    order, fine, mgs = [0, 1, 0, 2, 0, 3, 1], [], []
+    for k in order:
+        i, extra = inst[k], (20.0, 30) if ISPECS[k][0] == "solid" else (15.0, 10)
+        mgs.append(mfgpu.Multigrid(i.levels, i.transfers, smoothing_range=extra[0], eig_cg_iterations=extra[1],
+                                   coarse_eig_iterations=40))
+        mgs[-1].setup()
+        fine.append(i.fine)
+    srcs = [mfgpu.fill_uniform(500 + j, torch.empty(inst[k].n_dofs, dtype=torch.float64, device="cuda"))
+            for j, k in enumerate(order)]
+    for s, k in zip(srcs, order):
+        s[torch.from_numpy(inst[k].constrained).long().cuda()] = 0.0
+    pre, sol = [torch.empty_like(s) for s in srcs], [torch.zeros_like(s) for s in srcs]
+    ref_info = []
+    for f, m, s, z, x in zip(fine, mgs, srcs, pre, sol):
+        m.vmult(z, s)
+        ref_info.append(mfgpu.cg_solve(f, s, x, mfgpu.PRECOND_MG, m, tol_rel=1e-8))
+    solver = mfgpu.BatchSolver(fine, mgs)
+    solver.set_schedule(schedule)
+    for _ in range(2):
+        out = [torch.full_like(s, float("nan")) for s in srcs]
+        solver.precondition(out, srcs)
+        assert all(torch.equal(o, z) for o, z in zip(out, pre))
+        xs = [torch.zeros_like(s) for s in srcs]
+        infos, status = solver.solve(srcs, xs, tol_rel=1e-8)
+        assert all(st == 0 for st in status)
+        assert [i.iterations for i in infos] == [i.iterations for i in ref_info]
+        assert all(torch.equal(x, y) for x, y in zip(xs, sol))
+
+
 def test_batched_errors(cuda):
     inst = instances(ISPECS[:2])
     with pytest.raises(mfgpu.MfgError):  # fine operators of different precisions
