@@ -698,14 +698,18 @@ void MGData::v_cycle(void *x, const void *b) {
 
 // PreconditionMG::vmult: copy_to_mg, V-cycle, copy_from_mg.  The copies are
 // left out where the caller's vectors can stand for the finest level's own: of
-// its precision, distinct, and not held by a captured graph.
+// its precision, without a byte in common (src is read until the end of the
+// cycle, dst written from its start), and not held by a captured graph.
 void MGData::vmult(void *dst, const void *src, int vec_prec) {
   MFG_REQUIRE(ready, MFG_ERR_STATE, "mfg_mg_setup() not called");
   MGLevel &F = levels.back();
   const int64_t n = F.op->n_dofs;
   hipStream_t caller = F.op->stream;
   const bool graphed = graphs_allowed() && ++graph_calls >= 2;
-  if (!graphed && vec_prec == F.op->precision && dst != src) {
+  const uintptr_t d = (uintptr_t)dst, r = (uintptr_t)src;
+  const size_t bytes = (size_t)n * F.op->elem_size();
+  const bool apart = d < r ? r - d >= bytes : d - r >= bytes;
+  if (!graphed && vec_prec == F.op->precision && apart) {
     v_cycle(dst, src);
     return;
   }

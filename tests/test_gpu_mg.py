@@ -290,6 +290,28 @@ def test_vcycle_gather_equals_colours(cuda, kind, p, n, precision):
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
 
 
+@pytest.mark.parametrize("kind,p,n,precision", [("solid", 2, (4, 4, 2), mfgpu.FP64), ("heat", 3, (4, 2, 4), mfgpu.FP32),
+                                                ("heat", 2, (3, 3, 3), mfgpu.FP64)])
+@pytest.mark.parametrize("graph", [False, True])
+def test_vcycle_overlapping_vectors(cuda, kind, p, n, precision, graph):
+    """src and dst may be views that share a part of their memory: the V-cycle is
+    the one of separate vectors, whichever of them comes first.  The third case
+    has one level."""
+    print(f"V-cycle of overlapping vectors {kind} p={p} precision={precision} graph={graph}", flush=True)
+    inst = mfgpu.Instance(kind, n, p, level_precision=precision, seed=3, coarse_eig_iterations=40)
+    inst.mg.use_graph(graph)
+    m, dt = inst.n_dofs, inst.levels[-1].dtype
+    x = mfgpu.fill_uniform(11, torch.empty(m, dtype=dt, device="cuda"))
+    y = torch.empty_like(x)
+    inst.mg.vmult(y, x)
+    for src_at, dst_at in ((0, 1), (1, 0), (0, m // 2), (m - 1, 0), (0, m), (m, 0)):
+        buf = torch.full((2 * m,), float("nan"), dtype=dt, device="cuda")
+        src, dst = buf[src_at:src_at + m], buf[dst_at:dst_at + m]
+        src.copy_(x)
+        mfgpu.check(mfgpu.lib().mfg_mg_vmult(inst.mg.h, mfgpu._ptr(dst), mfgpu._ptr(src), precision))
+        assert torch.equal(dst, y), (src_at, dst_at)
+
+
 @pytest.mark.parametrize("kind,p,n", [("solid", 1, (1, 1, 1)), ("solid", 1, (6, 2, 3)), ("solid", 2, (2, 1, 2)),
                                       ("heat", 1, (7, 7, 4)), ("heat", 2, (3, 3, 3))])
 def test_eigenvalue_estimate_small_levels(cuda, kind, p, n):
