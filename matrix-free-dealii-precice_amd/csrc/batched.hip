@@ -686,10 +686,8 @@ struct BatchGather {
     std::map<int, std::vector<int>> by_code;
     for (int i = 0; i < n; ++i) {
       OperatorData &op = *ops[i];
-      if (!op.contrib.ptr) {
-        op.build_gather();
-        ++op.buffers_version;
-      }
+      // new buffers beside those that apply() reads: buffers_version stays
+      if (!op.contrib.ptr) op.build_gather();
       by_code[code_of(op)].push_back(i);
       total += apply_work(op);
       contrib.push_back(op.contrib.ptr);
@@ -971,10 +969,7 @@ struct BatchVmult {
     });
   }
   void apply_gather(const void *const *src, void *const *dst, bool add) {
-    if (!gather) {
-      gather.reset(new BatchGather(mops, stream));
-      record_versions();  // building the operators' GATHER tables counts as a change of their buffers
-    }
+    if (!gather) gather.reset(new BatchGather(mops, stream));
     gather->apply(group->inst.ptr, src, dst, add, stream);
   }
   void apply(const void *const *src, void *const *dst, bool add) {

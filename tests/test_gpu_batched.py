@@ -350,6 +350,42 @@ def test_batched_vmult_follows_operator_changes(cuda, schedule):
             assert torch.equal(o, r), (rep, i, SPECS[i])
 
 
+@pytest.mark.parametrize("tune", [False, True])
+def test_batched_solver_before_a_gather_batch(cuda, tune):
+    """A solver and a batch made before GATHER tables are built for their
+    operators (by a batch's GATHER schedule or tuner; the operators are above
+    the size that builds them by itself) go on working, with the results they
+    gave before."""
+    print(f"batched solver before a GATHER batch tune={tune}", flush=True)
+    inst = [mfgpu.Instance("heat", [44, 44, 34], 3, coarse_eig_iterations=20, conductivity=0.7)]
+    assert inst[0].meshes[-1].n_cells * 4 ** 3 > 4 * 2 ** 20
+    fine, mgs = [i.fine for i in inst], [i.mg for i in inst]
+    assert fine[0].cell_schedule() == mfgpu.CELLS_COLOURS
+    solver, other, b = mfgpu.BatchSolver(fine, mgs), mfgpu.Batch(fine), mfgpu.Batch(fine)
+    src = [mfgpu.fill_uniform(7, torch.empty(inst[0].n_dofs, dtype=torch.float64, device="cuda"))]
+    src[0][torch.from_numpy(inst[0].constrained).long().cuda()] = 0.0
+
+    def results():
+        x, y, z = ([torch.zeros_like(src[0])] for _ in range(3))
+        infos, status = solver.solve(src, x, tol_rel=1e-8)
+        assert status[0] == 0
+        solver.precondition(y, src)
+        other.vmult(z, src)
+        other.synchronize()
+        return x[0], y[0], z[0], infos[0].iterations
+    before = results()
+    out = [torch.empty_like(src[0])]
+    if tune:
+        b.tune(src, out, repetitions=2)
+    else:
+        b.set_schedule(mfgpu.SCHEDULE_GATHER)
+        b.vmult(out, src)
+    b.synchronize()
+    after = results()
+    assert before[3] == after[3] and all(torch.equal(p, q) for p, q in zip(before[:3], after[:3]))
+    assert torch.equal(out[0], before[2])
+
+
 def test_batched_solver_refuses_changed_operators(cuda):
     inst = instances(ISPECS[:3])
     solver = mfgpu.BatchSolver([i.fine for i in inst], [i.mg for i in inst])
