@@ -150,7 +150,7 @@ struct OperatorData {
   void setup_solid();
   void setup_heat(const mfg_level_desc &d, const double *coef);
   void cache(const void *u, int u_precision);
-  void export_qp_gradient(DeviceBuffer &out);
+  void export_qp_gradient(void *out);
   // dst (+)= A src on `on` (the operator's stream when null)
   void apply(const void *src, void *dst, bool add, hipStream_t on = nullptr) const;
   // dst = A src for callers that order all of the operator's work on its stream

@@ -25,10 +25,11 @@ struct CacheArgs {
   int jxw_ref_field;  // tensor2 formulation 1: store JxW_ref as field 16 (not supplied per cell)
   // tensor2 formulation 1, MFG_T2_GRADIENT: 1 stores the operator's 10 fields
   // (Jinv_cur, s), and the displacement itself to u_copy; 2 stores Grad_xi u
-  // and s (what mfg_operator_qp_data exports)
+  // and s (what mfg_operator_qp_data exports) field by field in input cell order
   int t2_gradient;
-  Number *u_copy;  // 3 per node, with t2_gradient 1
-  int *error;   // set to 1 if det F <= 0 anywhere
+  Number *u_copy;       // 3 per node, with t2_gradient 1
+  const int32_t *perm;  // with t2_gradient 2: input index of every stored cell
+  int *error;   // set to 1 if det F <= 0 anywhere (not with t2_gradient 2)
 };
 
 template <typename Number>
@@ -167,23 +168,25 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) cache_solid(CacheAr
       Jc[d][e] = (Number)Jr[d][e] + gr[d][e];
     }
   const Number J = det3(F);
+  const int64_t n = a.nqp;
+  if (a.t2_gradient == 2) {
+    const int64_t at = (int64_t)a.perm[cell] * N3 + pt;
+#pragma unroll
+    for (int f = 0; f < 9; ++f) a.qd[f * n + at] = gr[f / 3][f % 3];
+    a.qd[9 * n + at] = a.mu - Number(2) * a.lambda * log(J);
+    return;
+  }
   if (!(J > Number(0))) {
     *a.error = 1;
     return;
   }
-  const int64_t n = a.nqp;
   const double wq = a.weights[T.i] * a.weights[T.j] * a.weights[T.k];
   const Number scalar = a.mu - Number(2) * a.lambda * log(J);
   if (a.t2_gradient) {  // 9 words and s, in pairs of fields
     Number f10[10];
-    if (a.t2_gradient == 1) {
-      inv3(Jc, Jci);
+    inv3(Jc, Jci);
 #pragma unroll
-      for (int f = 0; f < 9; ++f) f10[f] = Jci[f / 3][f % 3];
-    } else {
-#pragma unroll
-      for (int f = 0; f < 9; ++f) f10[f] = gr[f / 3][f % 3];
-    }
+    for (int f = 0; f < 9; ++f) f10[f] = Jci[f / 3][f % 3];
     f10[9] = scalar;
     typedef Number Pair __attribute__((ext_vector_type(2)));
     Pair *qp = reinterpret_cast<Pair *>(a.qd);

@@ -548,6 +548,47 @@ def test_gradient_point_storage_export(cuda, p, precision, amp):
     assert np.abs(g[9] - s).max() <= 2 * lam * (16 * eps + 9 * tol / 0.2) + 4 * eps * O.MU
 
 
+@pytest.mark.parametrize("kind", ["gradient", "inclusion", "folded", "heat"])
+@pytest.mark.parametrize("p,precision", [(1, mfgpu.FP64), (2, mfgpu.FP32), (4, mfgpu.FP64)])
+def test_qp_data_is_stream_ordered(cuda, kind, p, precision):
+    """mfg_operator_qp_data only launches: it can be captured on the operator's
+    stream (no allocation, no wait), and replays give the data of the cache that
+    is current then."""
+    print(f"qp_data captured {kind} p={p} precision={precision}", flush=True)
+    nc, fm, cm = (1, 63, 1) if kind == "heat" else (3, 1, 7)
+    gm = mfgpu.BoxMesh([0, 0, 0], [1.0, 0.6, 0.4], [3, 5, 2], p, nc, fm, cm)
+    if kind == "heat":
+        go = mfgpu.LaplaceOperator(gm, 0.1, np.random.default_rng(p).uniform(0.5, 2.0, gm.n_cells * (p + 1) ** 3),
+                                   precision=precision)
+    else:
+        if kind == "inclusion":
+            gm.set_material_ids(np.arange(gm.n_cells) % 3 // 2)
+        go = mfgpu.NeoHookOperator(gm, O.MU, O.NU, O.RHO, O.ALPHA1, precision=precision,
+                                   inclusion=(100 * O.MU, O.NU, O.RHO) if kind == "inclusion" else None)
+        if kind == "folded":
+            go.set_point_storage(mfgpu.T2_FOLDED)
+        us = [dev(gm.u0(amp=1e-2, noise=1e-4, seed=k), go.dtype) for k in range(3)]
+        go.cache(us[0])
+    want = go.qp_data()
+    out = torch.full_like(want, float("nan"))
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    go.set_stream(stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        mfgpu.check(mfgpu.lib().mfg_operator_qp_data(go.h, mfgpu._ptr(out), None))
+    for k in range(3):
+        if kind != "heat":
+            torch.cuda.synchronize()
+            go.cache(us[k])
+            want = go.qp_data()
+        torch.cuda.synchronize()
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+
+
 # (kind, degree, precision, cells): one launch over all cells (GATHER) takes the
 # column-per-thread kernels, the eighth of them in a colour launch the
 # point-per-thread ones.  Cell counts: the first the column kernels serve (768
