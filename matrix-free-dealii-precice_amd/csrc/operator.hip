@@ -218,7 +218,6 @@ static void launch_cache(OperatorData &op, const void *u, int u_fp32, void *expo
   a.nqp = op.nqp;
   a.formulation = op.sp.formulation;
   a.caching = op.sp.caching;
-  a.affine = op.affine_ref ? 1 : 0;
   a.jxw_ref_field = op.affine_ref ? 0 : 1;
   a.t2_gradient = export_gradient ? 2 : op.t2_gradient() ? 1 : 0;
   a.u_copy = a.t2_gradient == 1 ? op.u_copy<Number>() : nullptr;
@@ -229,7 +228,9 @@ static void launch_cache(OperatorData &op, const void *u, int u_fp32, void *expo
     a.cell_end = e;
     a.mu = Number(op.mats[m].mu);
     a.lambda = Number(op.mats[m].lambda);
-    cache_solid<P, CPB, Number><<<blocks_for(e - b, CPB), block_threads<P, CPB>(), 0, op.stream>>>(a);
+    const int blocks = blocks_for(e - b, CPB);
+    if (op.affine_ref) cache_solid<P, CPB, Number, true><<<blocks, block_threads<P, CPB>(), 0, op.stream>>>(a);
+    else cache_solid<P, CPB, Number, false><<<blocks, block_threads<P, CPB>(), 0, op.stream>>>(a);
     MFG_HIP(hipGetLastError());
   };
   if (op.has_inclusion()) op.for_each_range([&](int, int b, int e, int m) { cells(b, e, m); });

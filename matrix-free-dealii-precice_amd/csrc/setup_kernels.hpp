@@ -21,7 +21,6 @@ struct CacheArgs {
   Number mu, lambda;
   int formulation;
   int caching;  // MFG_CACHING_*
-  int affine;          // every cell's trilinear map is affine
   int jxw_ref_field;  // tensor2 formulation 1: store JxW_ref as field 16 (not supplied per cell)
   // tensor2 formulation 1, MFG_T2_GRADIENT: 1 stores the operator's 10 fields
   // (Jinv_cur, s), and the displacement itself to u_copy; 2 stores Grad_xi u
@@ -88,8 +87,14 @@ __device__ inline void affine_jacobian(Ptr v, double (&J)[3][3]) {
   }
 }
 
-template <int P, int CPB, typename Number>
-__global__ void __launch_bounds__((block_threads<P, CPB>())) cache_solid(CacheArgs<Number> a) {
+// kAffine: every cell's trilinear map is affine.  Both Jacobians in one kernel
+// take Q1 and Q2 FP64 from 4 waves per SIMD to 3: 1.2M unknowns Q1 non-affine 206
+// against 181 us (178 from the Jacobian of the vertices in point order alone),
+// 1.5M Q2 105 against 95.  Q2 FP64 is 2 registers above 4 waves' share by itself;
+// bounded to it, 3 spill.
+template <int P, int CPB, typename Number, bool kAffine>
+__global__ void __launch_bounds__((block_threads<P, CPB>()), (P == 2 && sizeof(Number) == 8 ? 4 : 1))
+    cache_solid(CacheArgs<Number> a) {
   constexpr int N = P + 1, N3 = N * N * N;
   __shared__ Number s_shape[N * N], s_colloc[N * N];
   __shared__ Number s_tile[CPB * 6 * N3];
@@ -138,11 +143,15 @@ __global__ void __launch_bounds__((block_threads<P, CPB>())) cache_solid(CacheAr
   if (!active) return;
 
   double Jr[3][3], Jri[3][3];
+  auto jacobian = [&](auto X) {
+    if constexpr (kAffine) affine_jacobian(X, Jr);
+    else trilinear_jacobian(X, a.points[T.i], a.points[T.j], a.points[T.k], Jr);
+  };
   // one cell per workgroup: the vertices come in as scalar loads
-  const int vcell = CPB == 1 ? __builtin_amdgcn_readfirstlane(first_cell) : cell;
-  const ConstantPtr<double> X = as_constant(a.vertices) + (int64_t)vcell * 24;
-  if (a.affine) affine_jacobian(X, Jr);
-  else trilinear_jacobian(X, a.points[T.i], a.points[T.j], a.points[T.k], Jr);
+  if constexpr (CPB == 1)
+    jacobian(as_constant(a.vertices) + (int64_t)__builtin_amdgcn_readfirstlane(first_cell) * 24);
+  else
+    jacobian(a.vertices + (int64_t)cell * 24);
   {
     const double id = 1.0 / (Jr[0][0] * (Jr[1][1] * Jr[2][2] - Jr[1][2] * Jr[2][1]) -
                              Jr[0][1] * (Jr[1][0] * Jr[2][2] - Jr[1][2] * Jr[2][0]) +
