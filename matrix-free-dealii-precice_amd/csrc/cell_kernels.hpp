@@ -117,11 +117,15 @@ struct Tile {
 // the 10-word point operation takes 106 VGPRs unrolled, 126 rolled: 487 -> 480
 // us at 20M unknowns FP64, 39.7 -> 37.5 us at 0.2M (FP32 266 -> 264, 35.4 ->
 // 33.1); the other point operations gain as well (formulation 0 649 -> 624,
-// the folded words 544 -> 526).  scalar_referential evaluates two fields (194
-// VGPRs unrolled) and stays rolled.
-template <int N, bool kTwoFields = false>
+// the folded words 544 -> 526; 3M unknowns: tensor4 209 -> 196, the folded words
+// on non-affine cells 119 -> 110).  Two stay rolled: scalar_referential, which
+// evaluates two fields (194 VGPRs unrolled), and the colour launches of
+// tensor4_ns in FP64, whose 91 words per point keep the memory busy by
+// themselves (3M unknowns 303 us unrolled, 272 rolled, 12M 1312 and 1195; its
+// GATHER launch 22.3 and 25.1 at 0.2M, 102.5 and 98.0 at 1M).
+template <int N, bool kRollN5 = false>
 constexpr bool rolled_components() {
-  return N >= (kTwoFields ? 5 : 6);
+  return N >= (kRollN5 ? 5 : 6);
 }
 
 // Evaluate values and reference-coordinate gradients at the quadrature points
@@ -867,7 +871,8 @@ __device__ inline void cell_group(const QOp &qop, const uint32_t *__restrict__ c
                                   const Number *__restrict__ g_colloc, Number *s_shape, Number *s_colloc,
                                   Number *s_tile, const uint32_t *__restrict__ slots = nullptr) {
   constexpr int N = P + 1, N3 = N * N * N, NC = QOp::NC;
-  constexpr bool kRolled = rolled_components<N, QOp::kNodalField>();
+  constexpr bool kRollN5 = QOp::kNodalField || (!kToCells && std::is_same<QOp, QSolidT4NS<double>>::value);
+  constexpr bool kRolled = rolled_components<N, kRollN5>();
   const int t = threadIdx.x;
   const int lc_raw = t / N3;
   const bool pad = lc_raw >= cpb;

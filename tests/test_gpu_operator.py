@@ -315,6 +315,27 @@ def test_solid_other_cachings(cuda, caching, p):
     assert rel(y32.double(), ref) < TOL32
 
 
+@pytest.mark.parametrize("caching", ["scalar_referential", "tensor4", "tensor4_ns"])
+@pytest.mark.parametrize("p,precision", [(1, mfgpu.FP64), (4, mfgpu.FP64), (4, mfgpu.FP32), (5, mfgpu.FP64)])
+def test_cell_schedules_of_other_cachings(cuda, caching, p, precision):
+    """GATHER and colour launches of the other cachings, whose kernels unroll
+    differently at p = 4 (tensor4_ns FP64), give the same bits."""
+    print(f"schedules caching {caching} p={p} precision={precision}", flush=True)
+    gm = mfgpu.BoxMesh([0, 0, 0], [1.0, 0.6, 0.4], [5, 3, 3], p, 3, 1, 7)
+    go = mfgpu.NeoHookOperator(gm, O.MU, O.NU, O.RHO, O.ALPHA1, caching=caching, precision=precision)
+    go.cache(dev(gm.u0(amp=5e-2, noise=1e-3), go.dtype))
+    x, y0 = (dev(O.fill_uniform(k, gm.n_dofs), go.dtype) for k in (3, 4))
+    out = []
+    for sched in (mfgpu.CELLS_COLOURS, mfgpu.CELLS_GATHER):
+        go.set_cell_schedule(sched)
+        y, z = torch.full_like(x, float("nan")), y0.clone()
+        go.vmult(y, x)
+        go.vmult_add(z, x)
+        out.append((y, z))
+    assert torch.isfinite(out[0][0]).all()
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
 @pytest.mark.parametrize("p,n", [(1, [4, 3, 2]), (2, [5, 2, 3]), (3, [3, 3, 3]), (4, [4, 2, 2])])
 def test_cell_schedules(cuda, p, n):
     """The GATHER schedule against the colour schedule (bitwise) and the
