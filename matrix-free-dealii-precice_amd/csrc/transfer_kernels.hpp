@@ -45,12 +45,25 @@ constexpr int transfer_lds() {
   constexpr int N = P + 1, M = 2 * P + 1;
   return M * N + KC * (M * M * M + M * M * N + M * N * N);
 }
+// LDS doubles of the prolongation alone
+template <int P, int KC>
+constexpr int prolongate_lds() {
+  constexpr int N = P + 1, M = 2 * P + 1;
+  return M * N + KC * (N * N * N + M * N * N + M * M * N);
+}
 // components at a time of the single-operator kernels: all of them where the
 // scratch stays within 64 KB (4 barriers per cell instead of 4 per component,
-// the lattice read once)
+// the lattice read once).  The prolongation needs less: 33 KB for the three
+// components of Q5, 52 KB for Q6.  Prolongation to 32x32x24 cells FP32, one
+// component at a time, three in the restriction's LDS, three in its own: Q5 58,
+// 62 and 42 us, Q6 98, (too large) and 80; FP64 Q5 101 -> 49, Q6 173 -> 87.
 template <int P, int NC>
 constexpr int transfer_components() {
   return transfer_lds<P, NC>() * 8 <= 65536 ? NC : 1;
+}
+template <int P, int NC>
+constexpr int prolongate_components() {
+  return prolongate_lds<P, NC>() * 8 <= 65536 ? NC : 1;
 }
 
 // KC components from `c` on of a node
@@ -215,8 +228,8 @@ __device__ inline void interpolate_cell(const TransferArgs<CN, FN> &a, int cell,
 // One workgroup of 256 threads per coarse cell of [cell_begin, cell_end).
 template <int P, int NC, typename CN, typename FN>
 __global__ void __launch_bounds__(256) prolongate_add_kernel(TransferArgs<CN, FN> a) {
-  constexpr int KC = transfer_components<P, NC>();
-  __shared__ double lds[transfer_lds<P, KC>()];
+  constexpr int KC = prolongate_components<P, NC>();
+  __shared__ double lds[prolongate_lds<P, KC>()];
   const int cell = a.cell_begin + blockIdx.x;
   if (cell < a.cell_end) prolongate_cell<P, NC, CN, FN, KC>(a, cell, lds);
 }

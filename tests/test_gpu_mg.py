@@ -80,6 +80,31 @@ def test_transfer_parity(cuda, p, nc):
     assert rel(ci, O.interpolate(cm, fm, f)) < 1e-13
 
 
+@pytest.mark.parametrize("precisions", [(mfgpu.FP64, mfgpu.FP64), (mfgpu.FP64, mfgpu.FP32), (mfgpu.FP32, mfgpu.FP32)])
+@pytest.mark.parametrize("p,nc", [(1, 1), (3, 3), (5, 3), (6, 3), (5, 1), (6, 1)])
+def test_transfers_by_degree(cuda, p, nc, precisions):
+    """The degrees whose kernels take one or all components at a time, in every
+    pair of level precisions."""
+    print(f"transfers p={p} nc={nc} precisions={precisions}", flush=True)
+    cmask = 7 if nc == 3 else 1
+    gms = [mfgpu.BoxMesh([0, 0, 0], [2.0, 1.0, 1.0], n, p, nc, 1 | 16, cmask) for n in ([3, 1, 2], [6, 2, 4])]
+    cm, fm = O.box_levels([0, 0, 0], [2.0, 1.0, 1.0], [3, 1, 2], 2, p, nc, 1 | 16, cmask)
+    ops = [mfgpu.NeoHookOperator(m, O.MU, O.NU, O.RHO, O.ALPHA1, precision=q) if nc == 3
+           else mfgpu.LaplaceOperator(m, 0.1, None, precision=q) for m, q in zip(gms, precisions)]
+    t = mfgpu.Transfer(ops[0], ops[1], mfgpu.box_children(gms[0], gms[1]))
+    c, f = O.fill_uniform(11, cm.n_dofs), O.fill_uniform(12, fm.n_dofs)
+    c, f = (v.astype(np.float32).astype(np.float64) for v in (c, f))  # exact in every precision
+    fo, co = f.copy(), c.copy()
+    O.prolongate_add(cm, fm, c, fo)
+    O.restrict_add(cm, fm, f, co)
+    fg, cg = dev(f, ops[1].dtype), dev(c, ops[0].dtype)
+    t.prolongate_add(fg, dev(c, ops[0].dtype))
+    t.restrict_add(cg, dev(f, ops[1].dtype))
+    # sums in 64 bits, stored once (prolongation) or after each of up to 8 cells
+    eps = [1e-13 if q == mfgpu.FP64 else 8 * 2.0 ** -24 for q in precisions]
+    assert rel(fg, fo) < eps[1] and rel(cg, co) < eps[0]
+
+
 def test_vcycle_and_eigenvalues_small_config(cuda):
     """8^3 Q2 cube, 3 levels, Chebyshev degree 4 (FP64 levels)."""
     gms, oms, gops, oops, trs = hierarchy("solid", [0, 0, 0], [1, 1, 1], [2, 2, 2], 3, 2)
