@@ -58,6 +58,15 @@ def build(jobs=8, verbose=True):
         r = subprocess.run(cmd, capture_output=True, text=True)
         if r.returncode != 0:
             raise RuntimeError(f"drop-in test build failed\n{r.stdout}\n{r.stderr}")
+    # host-only program on the library's own objects where there is no device
+    src = os.path.join(HERE, "..", "tests", "cpp", "no_device_memory.cpp")
+    if os.path.exists(src):
+        exe = os.path.join(BUILD, "no_device_memory_test")
+        cmd = [HIPCC, "-O2", "-std=c++17", "--offload-arch=gfx950", "-Wno-unused-result", "-I",
+               os.path.join(HERE, "..", "include"), src, "-L", HERE, "-lmfgpu", "-Wl,-rpath,$ORIGIN/..", "-o", exe]
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"device memory test build failed\n{r.stdout}\n{r.stderr}")
     if verbose:
         print(f"built {OUT}")
     return OUT

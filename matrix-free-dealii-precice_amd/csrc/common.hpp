@@ -66,6 +66,18 @@ struct DeviceBuffer {
     MFG_HIP(hipMalloc(&ptr, b));
     bytes = b;
   }
+  // false, without an error left behind, where the device has no memory for it
+  bool try_allocate(size_t b) {
+    release();
+    if (b == 0) return true;
+    if (hipMalloc(&ptr, b) != hipSuccess) {
+      ptr = nullptr;
+      (void)hipGetLastError();
+      return false;
+    }
+    bytes = b;
+    return true;
+  }
   void release() {
     if (ptr) (void)hipFree(ptr);
     ptr = nullptr;

@@ -262,8 +262,10 @@ void TransferData::prolongate_add(void *fine, const void *coarse) { run(0, fine,
 void TransferData::restrict_add(void *coarse, const void *fine) { run(1, nullptr, nullptr, coarse, fine); }
 void TransferData::interpolate(void *coarse, const void *fine) { run(2, nullptr, nullptr, coarse, fine); }
 void TransferData::prepare_restrict() {
-  // where the coarse operator has the tables of its nodes' points
-  if (coarse->gather_places.ptr && !contrib.ptr) contrib.allocate((size_t)coarse->nqp * nc * sizeof(double));
+  // where the coarse operator has the tables of its nodes' points; without
+  // memory for it restrict_set goes by colours
+  if (coarse->gather_places.ptr && !contrib.ptr)
+    (void)contrib.try_allocate((size_t)coarse->nqp * nc * sizeof(double));
 }
 void TransferData::restrict_set(void *out, const void *fine_in) {
   if (contrib.ptr) {

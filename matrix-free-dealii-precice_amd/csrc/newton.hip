@@ -45,9 +45,7 @@ static void residual_launch_kind(const OperatorData &op, const double *u, const 
   // as vmult's schedules: all cells and the sums per node, or a launch per
   // colour (and material).  The contributions have a buffer of their own
   // (residuals are synchronous, so no two share it).
-  if (op.gather_ordered()) {
-    const size_t bytes = (size_t)op.nqp * 3 * sizeof(double);
-    if (op.setup_contrib.bytes < bytes) op.setup_contrib.allocate(bytes);
+  if (op.gather_ordered() && op.reserve_setup_contrib()) {
     a.R = op.setup_contrib.as<double>();
     a.slots = op.gather_slots();
     if (op.has_inclusion()) op.for_each_range([&](int, int b, int e, int m) { cells(b, e, m, std::true_type()); });

@@ -265,8 +265,6 @@ static void launch_diagonal(OperatorData &op, bool gather) {
     op.for_each_range([&](int, int b, int e, int m) { cells(b, e, m, std::false_type()); });
     return;
   }
-  const size_t bytes = (size_t)op.nqp * op.nc * op.elem_size();
-  if (op.setup_contrib.bytes < bytes) op.setup_contrib.allocate(bytes);
   a.diag = op.setup_contrib.as<Number>();
   a.slots = op.gather_slots();
   if (op.has_inclusion()) op.for_each_range([&](int, int b, int e, int m) { cells(b, e, m, std::true_type()); });
@@ -338,8 +336,7 @@ void OperatorData::apply_epilogue(void *x, const EpilogueArgs &e) const {
 
 void OperatorData::prepare_gather() {
   if (schedule_set || nqp > gather_max_points(p)) return;
-  if (!contrib.ptr) build_gather();
-  gather_ready = true;
+  gather_ready = contrib.ptr || build_gather(true);
 }
 
 // Event pairs are reused; at most kMaxEvents launches are kept between
@@ -392,7 +389,7 @@ void OperatorData::compute_diagonal() {
     ++buffers_version;
   }
   clear_flag();
-  const bool gather = gather_ordered();
+  const bool gather = gather_ordered() && reserve_setup_contrib();
   auto run = [&](auto tag) {
     using Number = decltype(tag);
     diagonal_t<Number>(*this, gather);
@@ -525,8 +522,17 @@ void OperatorData::colour_cells(const mfg_level_desc &d, int N3) {
   for (int c = 0; c < n_cells; ++c) perm[ids[c] == 0 ? fillp[colour[c]]++ : fill1[colour[c]]++] = c;
 }
 
-void OperatorData::build_gather() {
+bool OperatorData::build_gather(bool optional) {
   MFG_REQUIRE(nqp < ((int64_t)1 << 31), MFG_ERR_ARGUMENT, "too many quadrature points for the GATHER tables");
+  auto drop = [&] {
+    for (DeviceBuffer *b : {&gather_offsets, &gather_places, &gather_cmask, &contrib}) b->release();
+  };
+  if (!gather_offsets.try_allocate((size_t)(n_nodes + 1) * 4) || !gather_places.try_allocate((size_t)nqp * 4) ||
+      !gather_cmask.try_allocate((size_t)n_nodes) || !contrib.try_allocate((size_t)nqp * nc * elem_size())) {
+    drop();
+    MFG_REQUIRE(optional, MFG_ERR_HIP, "no device memory for the GATHER schedule");
+    return false;
+  }
   const int N3 = (p + 1) * (p + 1) * (p + 1);
   std::vector<int32_t> offsets((size_t)n_nodes + 1, 0);
   std::vector<uint32_t> places((size_t)nqp);
@@ -544,10 +550,16 @@ void OperatorData::build_gather() {
       if (gather_indexed) places[at] = q;
       else places[q] = at;
     }
-  upload(gather_offsets, offsets.data(), offsets.size(), stream);
-  upload(gather_places, places.data(), places.size(), stream);
-  upload(gather_cmask, host_cmask.data(), host_cmask.size(), stream);
-  contrib.allocate((size_t)nqp * nc * elem_size());
+  try {
+    MFG_HIP(hipMemcpyAsync(gather_offsets.ptr, offsets.data(), gather_offsets.bytes, hipMemcpyHostToDevice, stream));
+    MFG_HIP(hipMemcpyAsync(gather_places.ptr, places.data(), gather_places.bytes, hipMemcpyHostToDevice, stream));
+    MFG_HIP(hipMemcpyAsync(gather_cmask.ptr, host_cmask.data(), gather_cmask.bytes, hipMemcpyHostToDevice, stream));
+    MFG_HIP(hipStreamSynchronize(stream));  // the host arrays end here
+  } catch (...) {
+    drop();
+    throw;
+  }
+  return true;
 }
 
 void OperatorData::setup_layout(const mfg_level_desc &d) {

@@ -127,16 +127,24 @@ struct OperatorData {
   bool gather_indexed = false;
   // the contributions of the Newton residual and the diagonal (synchronous
   // calls: no two share it, and an application in flight on another stream has
-  // its own)
+  // its own), made by the first of them; false: no memory for it, and the call
+  // takes the colour launches, which need none
   mutable DeviceBuffer setup_contrib;
+  bool reserve_setup_contrib() const {
+    const size_t need = (size_t)nqp * nc * elem_size();
+    return setup_contrib.bytes >= need || setup_contrib.try_allocate(need);
+  }
   const uint32_t *gather_slots() const { return gather_indexed ? nullptr : gather_places.as<uint32_t>(); }
-  void build_gather();
+  // All of the tables and the contribution buffer, or none of them.  Without
+  // memory for them: MFG_ERR_HIP, or (optional) false.
+  bool build_gather(bool optional = false);
   // The schedule was set through mfg_operator_set_cell_schedule: every
   // application keeps it.
   bool schedule_set = false;
   // Up to gather_max_points() a multigrid hierarchy (whose work, like its level
   // vectors, is ordered on one stream) applies its level operators with GATHER
   // whatever their default: prepare_gather() in its setup, apply_ordered() then.
+  // Without memory for it they keep their default.
   void prepare_gather();
   bool gather_ordered() const { return cell_schedule == MFG_CELLS_GATHER || (!schedule_set && gather_ready); }
   bool gather_ready = false;
