@@ -224,35 +224,51 @@ void SolidProblem::step(mfg_step_info &info) {
 size_t SolidProblem::memory() const {
   size_t b = u.bytes + du.bytes + delta_u.bytes + v.bytes + a.bytes + v_old.bytes + a_old.bytes + R.bytes +
              iface_faces.bytes;
-  for (auto &o : levels) b += o->memory_consumption() + o->diag.bytes + o->inv_diag.bytes + o->vertices.bytes;
+  for (auto &o : levels)
+    b += o->memory_consumption() + o->diag.bytes + o->inv_diag.bytes + o->vertices.bytes + o->perm_dev.bytes;
   for (auto &L : mg->levels)
     for (const DeviceBuffer *x : {&L.sol, &L.def, &L.tmp, &L.d, &L.t, &L.cg_r, &L.cg_p, &L.cg_h, &L.cg_z}) b += x->bytes;
-  if (fine64) b += fine64->memory_consumption() + fine64->vertices.bytes;
-  for (auto &t : transfers) b += t->lattice.bytes;
+  if (fine64)
+    b += fine64->memory_consumption() + fine64->diag.bytes + fine64->inv_diag.bytes + fine64->vertices.bytes +
+         fine64->perm_dev.bytes;
+  for (auto &t : transfers) b += t->lattice.bytes + t->contrib.bytes;
   for (auto &x : u_lev) b += x.bytes;
   b += ws.r.bytes + ws.z.bytes + ws.p.bytes + ws.h.bytes + cond_b.bytes + cond_x.bytes;
   return b;
 }
 
-size_t estimate_solid_problem_bytes(int n_levels, const mfg_level_desc *levels, int level_precision) {
-  size_t b = 0;
+// What SolidProblem::memory() reaches once the problem has stepped.
+size_t estimate_solid_problem_bytes(int n_levels, const mfg_level_desc *levels, const mfg_solid_params &material,
+                                    int level_precision) {
+  size_t total = 0;
   for (int l = 0; l < n_levels; ++l) {
     const mfg_level_desc &d = levels[l];
-    const int64_t n3 = (int64_t)(d.degree + 1) * (d.degree + 1) * (d.degree + 1);
-    const int64_t nqp = (int64_t)d.n_cells * n3, ndof = d.n_nodes * d.n_components;
+    const int64_t n3 = (int64_t)(d.degree + 1) * (d.degree + 1) * (d.degree + 1), nqp = (int64_t)d.n_cells * n3,
+                  ndof = d.n_nodes * d.n_components;
+    const bool gather = nqp <= gather_max_points(d.degree);
+    bool affine = true;
+    for (int c = 0; c < d.n_cells && affine; ++c) affine = affine_cell(d.cell_vertices + (size_t)c * 24);
+    const bool t2 = material.formulation == 1 && material.caching == MFG_CACHING_TENSOR2;
+    // the cache, the kept displacement (10-word storage, scalar_referential), map and lists, geometry, and the
+    // GATHER tables with the contributions of the operator and of its diagonal or residual
+    auto op_bytes = [&](size_t es) {
+      size_t b = (size_t)nqp * (OperatorData::solid_fields(material, t2 && affine, affine) * es + 4);
+      if ((t2 && affine) || material.caching == MFG_CACHING_SCALAR_REFERENTIAL) b += ndof * es;
+      b += (size_t)d.n_constrained * 4 + (size_t)d.n_cells * (24 * 8 + 4);
+      if (affine) b += (size_t)d.n_cells * 7 * es + n3 * es;
+      if (gather) b += gather_bytes(nqp, d.n_nodes, d.n_components, es) + (size_t)nqp * d.n_components * es;
+      return b;
+    };
     const size_t es = (l == 0 || level_precision == MFG_FP64) ? 8 : 4;
-    b += nqp * (18 * es + 4) + (size_t)d.n_cells * 24 * 8 + 11 * ndof * es;  // caches, map, vertices, diag + MG vectors
-    if (nqp <= gather_max_points(d.degree)) b += gather_bytes(nqp, d.n_nodes, d.n_components, es);
-    if (l > 0) b += (size_t)levels[l - 1].n_cells * (2 * d.degree + 1) * (2 * d.degree + 1) * (2 * d.degree + 1) * 4;
+    total += op_bytes(es) + 12 * ndof * es;  // diagonal and inverse, MG vectors, displacement of the level
+    if (l > 0) total += (size_t)levels[l - 1].n_cells * (2 * d.degree + 1) * (2 * d.degree + 1) * (2 * d.degree + 1) * 4;
+    if (l < n_levels - 1 && gather) total += (size_t)nqp * d.n_components * 8;  // restriction to this level
     if (l == n_levels - 1) {
-      b += 12 * ndof * 8;  // state, residual, CG workspace
-      if (level_precision == MFG_FP32 && n_levels > 1) {
-        b += nqp * (18 * 8 + 4) + (size_t)d.n_cells * 24 * 8 + 2 * ndof * 4;  // + FP32 condition-estimate vectors
-        if (nqp <= gather_max_points(d.degree)) b += gather_bytes(nqp, d.n_nodes, d.n_components, 8);
-      }
+      total += 12 * ndof * 8;  // state, residual, CG workspace
+      if (level_precision == MFG_FP32 && n_levels > 1) total += op_bytes(8) + 2 * ndof * 4;  // + condition estimate
     }
   }
-  return b;
+  return total;
 }
 
 std::unique_ptr<SolidProblem> make_solid_problem(int n_levels, const mfg_level_desc *levels,

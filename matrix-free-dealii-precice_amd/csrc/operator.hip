@@ -617,18 +617,13 @@ void OperatorData::setup_layout(const mfg_level_desc &d) {
   for (int c = 0; c < n_cells; ++c) {
     const double *X = &vert[(size_t)c * 24];
     auto V = [&](int v, int e) { return X[v * 3 + e]; };
-    double J[3][3], h = 0, mixed = 0;
+    double J[3][3];
     for (int e = 0; e < 3; ++e) {
       J[e][0] = V(1, e) - V(0, e);
       J[e][1] = V(2, e) - V(0, e);
       J[e][2] = V(4, e) - V(0, e);
-      for (int f = 0; f < 3; ++f) h = std::max(h, std::fabs(J[e][f]));
-      mixed = std::max({mixed, std::fabs(V(3, e) - V(2, e) - V(1, e) + V(0, e)),
-                        std::fabs(V(5, e) - V(4, e) - V(1, e) + V(0, e)),
-                        std::fabs(V(6, e) - V(4, e) - V(2, e) + V(0, e)),
-                        std::fabs(V(7, e) - V(6, e) - V(5, e) + V(4, e) - V(3, e) + V(2, e) + V(1, e) - V(0, e))});
     }
-    if (mixed > 1e-12 * h) affine_ref = false;
+    if (!affine_cell(X)) affine_ref = false;
     const double det = J[0][0] * (J[1][1] * J[2][2] - J[1][2] * J[2][1]) -
                        J[0][1] * (J[1][0] * J[2][2] - J[1][2] * J[2][0]) + J[0][2] * (J[1][0] * J[2][1] - J[1][1] * J[2][0]);
     det_ref[c] = std::fabs(det);
@@ -784,19 +779,23 @@ void OperatorData::setup_solid() {
   c_1 = mats[0].c_1;
   lambda = mats[0].lambda;
   rho_alpha = mats[0].rho_alpha;
-  switch (sp.caching) {
-    case MFG_CACHING_SCALAR_REFERENTIAL: n_fields = QSolidSR<double>::kFields; break;
-    case MFG_CACHING_TENSOR4: n_fields = QSolidT4<double>::kFields; break;
-    case MFG_CACHING_TENSOR4_NS: n_fields = QSolidT4NS<double>::kFields; break;
-    default:
-      n_fields = sp.formulation == 0 ? QSolidT2F0<double>::kFields
-                 : t2_gradient()     ? QSolidT2F1G<double>::kFields
-                 : affine_ref        ? QSolidT2F1<double>::kFields - 1
-                                     : QSolidT2F1<double>::kFields;
-  }
+  n_fields = solid_fields(sp, t2_gradient(), affine_ref);
   const size_t es = precision == MFG_FP64 ? 8 : 4;
   // the 10-word storage keeps the displacement as well (export_qp_gradient)
   qd.allocate((size_t)n_fields * nqp * es + (t2_gradient() ? (size_t)n_dofs * es : 0));
+}
+
+int OperatorData::solid_fields(const mfg_solid_params &sp, bool t2_gradient, bool affine) {
+  switch (sp.caching) {
+    case MFG_CACHING_SCALAR_REFERENTIAL: return QSolidSR<double>::kFields;
+    case MFG_CACHING_TENSOR4: return QSolidT4<double>::kFields;
+    case MFG_CACHING_TENSOR4_NS: return QSolidT4NS<double>::kFields;
+    default:
+      return sp.formulation == 0 ? QSolidT2F0<double>::kFields
+             : t2_gradient       ? QSolidT2F1G<double>::kFields
+             : affine            ? QSolidT2F1<double>::kFields - 1
+                                 : QSolidT2F1<double>::kFields;
+  }
 }
 
 size_t OperatorData::memory_consumption() const {

@@ -1,5 +1,8 @@
 // Device operator object shared by the operator, multigrid and solver code.
 #pragma once
+#include <algorithm>
+#include <cmath>
+
 #include "common.hpp"
 
 namespace mfg {
@@ -26,6 +29,21 @@ constexpr int64_t gather_max_points(int p) {
 // device bytes of the GATHER schedule's tables and contribution buffer
 inline size_t gather_bytes(int64_t nqp, int64_t n_nodes, int nc, size_t es) {
   return (size_t)nqp * (nc * es + 4) + (size_t)(n_nodes + 1) * 4 + (size_t)n_nodes;
+}
+
+// Whether the trilinear map of a cell (8 vertices, vertex v at (v & 1, v >> 1 & 1,
+// v >> 2 & 1)) is affine: its mixed terms vanish.
+inline bool affine_cell(const double *X) {
+  auto V = [&](int v, int e) { return X[v * 3 + e]; };
+  double h = 0, mixed = 0;
+  for (int e = 0; e < 3; ++e) {
+    for (int v : {1, 2, 4}) h = std::max(h, std::fabs(V(v, e) - V(0, e)));
+    mixed = std::max({mixed, std::fabs(V(3, e) - V(2, e) - V(1, e) + V(0, e)),
+                      std::fabs(V(5, e) - V(4, e) - V(1, e) + V(0, e)),
+                      std::fabs(V(6, e) - V(4, e) - V(2, e) + V(0, e)),
+                      std::fabs(V(7, e) - V(6, e) - V(5, e) + V(4, e) - V(3, e) + V(2, e) + V(1, e) - V(0, e))});
+  }
+  return mixed <= 1e-12 * h;
 }
 
 // What the per-node sums of a GATHER application do with a row t of A x
@@ -167,6 +185,8 @@ struct OperatorData {
   void apply_epilogue(void *x, const EpilogueArgs &e) const;
   void compute_diagonal();
   size_t memory_consumption() const;
+  // words per point of the quadrature cache of a solid operator
+  static int solid_fields(const mfg_solid_params &sp, bool t2_gradient, bool affine);
   size_t elem_size() const { return precision == MFG_FP64 ? 8 : 4; }
   void timing_begin(hipStream_t s) const;
   void timing_end(hipStream_t s) const;

@@ -50,7 +50,8 @@ std::unique_ptr<SolidProblem> make_solid_problem(int n_levels, const mfg_level_d
                                                  const mfg_newmark_params &newmark, const mfg_mg_params &mgp,
                                                  int level_precision, hipStream_t stream);
 // Device bytes a problem of these levels will allocate (admission control).
-size_t estimate_solid_problem_bytes(int n_levels, const mfg_level_desc *levels, int level_precision);
+size_t estimate_solid_problem_bytes(int n_levels, const mfg_level_desc *levels, const mfg_solid_params &material,
+                                    int level_precision);
 
 }  // namespace mfg
 

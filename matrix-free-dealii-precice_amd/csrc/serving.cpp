@@ -63,7 +63,7 @@ struct Session {
       child_ptrs.push_back(children[l - 1].data());
     }
     n_dofs = descs.back().n_nodes * 3;
-    bytes = estimate_solid_problem_bytes(levels, descs.data(), spec.level_precision);
+    bytes = estimate_solid_problem_bytes(levels, descs.data(), spec.material, spec.level_precision);
     hu.assign(n_dofs, 0.0);
     hv.assign(n_dofs, 0.0);
     ha.assign(n_dofs, 0.0);

@@ -3,6 +3,7 @@ sessions.  Each session's results must be identical alone (sequential) and in
 the concurrent mix, also when HBM-budget admission forces evictions."""
 import numpy as np
 import pytest
+import torch
 
 import mfgpu
 import oracle as O
@@ -61,6 +62,34 @@ def test_hbm_budget_forces_evictions(cuda):
                (b.newton_iterations, b.linear_iterations, b.residual_final)
     for x, y in zip(fin_ref, fin):
         assert np.array_equal(x, y)
+
+
+@pytest.mark.parametrize("level_precision", [mfgpu.FP64, mfgpu.FP32])
+@pytest.mark.parametrize("formulation,caching", [(1, "tensor2"), (0, "tensor2"), (1, "scalar_referential"),
+                                                 (1, "tensor4"), (1, "tensor4_ns")])
+@pytest.mark.parametrize("n,p", [([16, 4, 4], 3), ([4, 2, 2], 2), ([3, 3, 3], 1), ([24, 8, 8], 4)])
+def test_admission_covers_the_memory_held(cuda, level_precision, formulation, caching, n, p):
+    """The bytes a session is admitted with are not fewer than its problem holds
+    after a step (contribution buffers of the residual, the diagonal and the
+    restriction among them), and not a quarter more."""
+    print(f"admission n={n} p={p} precision={level_precision} formulation={formulation} {caching}", flush=True)
+    s = mfgpu.session_spec([0, 0, 0], [4.0, 1.0, 1.0], n, p, O.MU, O.NU, O.RHO, body=(0.0, 0.0, -9.81),
+                           level_precision=level_precision)
+    s.material.formulation, s.material.caching = formulation, mfgpu.CACHING[caching]
+    _, st, _ = mfgpu.serve([s], [(0, 0.0)], max_concurrent=1, real_time=False)
+    meshes, c = [], list(n)
+    while True:
+        meshes.insert(0, mfgpu.BoxMesh([0, 0, 0], [4.0, 1.0, 1.0], c, p, 3, 1, 7, numbering="cellwise"))
+        if any(v % 2 for v in c):
+            break
+        c = [v // 2 for v in c]
+    prob = mfgpu.SolidProblem(meshes, O.MU, O.NU, O.RHO, formulation=formulation, caching=caching,
+                              level_precision=level_precision, body=(0.0, 0.0, -9.81))
+    u = torch.from_numpy(meshes[-1].u0(amp=1e-3, noise=1e-5)).cuda()
+    prob.set_state(u, torch.zeros_like(u), torch.zeros_like(u))
+    prob.step()
+    print(f"admitted {st.peak_bytes} held {prob.memory()}")
+    assert prob.memory() <= st.peak_bytes <= 1.25 * prob.memory()
 
 
 def test_session_larger_than_budget_is_rejected(cuda):
