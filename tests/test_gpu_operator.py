@@ -670,6 +670,55 @@ def test_column_kernels(cuda, kind, p, precision, n):
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
 
 
+# (kind, degree, precision, cells): every colour has enough cells for the column
+# kernels (768 waves of 64 // (p+1)^2 heat cells, 512 solid cells of FP64 Q6, 1536
+# of the others); in some colours the last wave is partly filled
+COLUMN_COLOUR_CASES = [
+    ("heat", 1, mfgpu.FP32, (47, 48, 47)), ("heat", 2, mfgpu.FP32, (37, 36, 35)), ("heat", 2, mfgpu.FP64, (35, 37, 36)),
+    ("heat", 3, mfgpu.FP32, (31, 31, 29)), ("heat", 3, mfgpu.FP64, (29, 31, 31)), ("heat", 4, mfgpu.FP64, (25, 25, 23)),
+    ("heat", 4, mfgpu.FP32, (23, 25, 25)), ("heat", 5, mfgpu.FP32, (20, 19, 19)), ("heat", 6, mfgpu.FP64, (19, 19, 20)),
+    ("solid", 5, mfgpu.FP64, (25, 24, 24)), ("solid", 5, mfgpu.FP32, (24, 24, 25)), ("solid", 6, mfgpu.FP64, (17, 16, 17)),
+    ("solid", 6, mfgpu.FP32, (24, 25, 24)), ("solid_f0", 6, mfgpu.FP64, (16, 17, 17)),
+    ("solid_folded", 6, mfgpu.FP64, (16, 16, 16)), ("solid_folded", 5, mfgpu.FP32, (25, 24, 24))]
+
+
+@pytest.mark.parametrize("kind,p,precision,n", COLUMN_COLOUR_CASES)
+def test_column_kernels_in_colour_launches(cuda, kind, p, precision, n):
+    """vmult and vmult_add of the column kernels' colour launches (stores by the
+    first colour, read-modify-write, identity rows) are bitwise those of the
+    batch's colour launches, which take a thread per point."""
+    print(f"columns in colours {kind} p={p} precision={precision} n={n}", flush=True)
+    nc, fm, cm = (1, 63, 1) if kind == "heat" else (3, 1 | 16, 7)
+    cells = 64 // (p + 1) ** 2
+    waves = -(-(n[0] // 2) * (n[1] // 2) * (n[2] // 2) // cells)  # of the smallest colour
+    assert waves >= (768 if kind == "heat" else 512 if p == 6 and precision == mfgpu.FP64 else 1536)
+    gm = mfgpu.BoxMesh([0, 0, 0], [1.0, 0.6, 0.4], list(n), p, nc, fm, cm)
+    if kind == "heat":
+        coef = np.random.default_rng(p).uniform(0.5, 2.0, gm.n_cells * (p + 1) ** 3)
+        go = mfgpu.LaplaceOperator(gm, 0.1, coef, precision=precision)
+    else:
+        go = mfgpu.NeoHookOperator(gm, O.MU, O.NU, O.RHO, O.ALPHA1, formulation=0 if kind == "solid_f0" else 1,
+                                   precision=precision)
+        if kind == "solid_folded":
+            go.set_point_storage(mfgpu.T2_FOLDED)
+        go.cache(dev(gm.u0(amp=1e-2, noise=1e-5), go.dtype))
+    go.set_cell_schedule(mfgpu.CELLS_COLOURS)
+    assert go.n_colours() == 8
+    x, y0 = (mfgpu.fill_uniform(k, torch.empty(gm.n_dofs, dtype=go.dtype, device="cuda")) for k in (5, 6))
+    b = mfgpu.Batch([go])
+    b.set_schedule(mfgpu.SCHEDULE_COLOUR)
+    ref, ref_add = torch.full_like(x, float("nan")), y0.clone()
+    b.vmult([ref], [x])
+    b.vmult_add([ref_add], [x])
+    b.synchronize()
+    assert torch.isfinite(ref).all()
+    for _ in range(2):
+        y, z = torch.full_like(x, float("nan")), y0.clone()
+        go.vmult(y, x)
+        go.vmult_add(z, x)
+        assert torch.equal(y, ref) and torch.equal(z, ref_add)
+
+
 @pytest.mark.parametrize("kind", ["solid", "solid_folded", "solid_f0", "heat"])
 @pytest.mark.parametrize("p,precision", [(1, mfgpu.FP64), (2, mfgpu.FP64), (3, mfgpu.FP32), (5, mfgpu.FP64), (6, mfgpu.FP32)])
 def test_diagonal_gather_equals_colours(cuda, kind, p, precision):
