@@ -315,6 +315,36 @@ def test_vcycle_gather_equals_colours(cuda, kind, p, n, precision):
     assert torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
 
 
+@pytest.mark.parametrize("kind,p,n,precision", [
+    ("solid", 2, (36, 36, 34), mfgpu.FP64), ("solid", 4, (22, 22, 20), mfgpu.FP32), ("heat", 2, (36, 36, 34), mfgpu.FP32),
+    ("heat", 4, (22, 22, 20), mfgpu.FP64)])
+def test_vcycle_gather_inside_a_hierarchy(cuda, kind, p, n, precision):
+    """Above 2^20 points an operator applies itself by colours and a hierarchy
+    applies it with GATHER: estimates, diagonals and V-cycles are bitwise those of
+    a hierarchy whose operators were set to COLOURS, before and after the schedule
+    is set on a hierarchy in use, and the operator's own vmult stays as it was."""
+    print(f"GATHER inside a hierarchy {kind} p={p} precision={precision}", flush=True)
+    assert 2 ** 20 < n[0] * n[1] * n[2] * (p + 1) ** 3 <= 3 * 2 ** 20
+    out = []
+    for sched in (None, mfgpu.CELLS_COLOURS):
+        inst = mfgpu.Instance(kind, n, p, level_precision=precision, seed=3, cell_schedule=sched, coarse_eig_iterations=20)
+        top = inst.levels[-1]
+        assert top.cell_schedule() == mfgpu.CELLS_COLOURS
+        x = mfgpu.fill_uniform(11, torch.empty(inst.n_dofs, dtype=top.dtype, device="cuda"))
+        y, z, w = (torch.full_like(x, float("nan")) for _ in range(3))
+        inst.mg.vmult(y, x)
+        top.vmult(z, x)
+        info = [inst.mg.level_info(l) for l in range(len(inst.levels))]
+        top.compute_diagonal()
+        out.append((y, z, top.diagonal(), info))
+        if sched is None:
+            top.set_cell_schedule(mfgpu.CELLS_COLOURS)
+            inst.mg.vmult(w, x)
+            assert torch.equal(w, y)
+    assert torch.isfinite(out[0][0]).all() and out[0][3] == out[1][3]
+    assert all(torch.equal(a, b) for a, b in zip(out[0][:3], out[1][:3]))
+
+
 @pytest.mark.parametrize("kind,p,n,precision", [("solid", 2, (4, 4, 2), mfgpu.FP64), ("heat", 3, (4, 2, 4), mfgpu.FP32),
                                                 ("heat", 2, (3, 3, 3), mfgpu.FP64)])
 @pytest.mark.parametrize("graph", [False, True])
