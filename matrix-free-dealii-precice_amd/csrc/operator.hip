@@ -224,6 +224,12 @@ static void launch_cache(OperatorData &op, const void *u, int u_fp32, void *expo
   a.jxw_ref_field = op.affine_ref ? 0 : 1;
   a.t2_gradient = export_gradient ? 2 : op.t2_gradient() ? 1 : 0;
   a.u_copy = a.t2_gradient == 1 ? op.u_copy<Number>() : nullptr;
+  // fields that do not stay in the L2s (8 of 4 MB) leave them to the
+  // displacement and the map.  Cache, plain / streamed: Q2 3M unknowns 153 / 105
+  // us, 15M 676 / 555; Q5 15M 347 / 294 (without the displacement's copy 316);
+  // FP32 Q4 15M 203 / 142.  Below, the next application reads them from there:
+  // cache and two vmults of 0.1M Q1 unknowns (21 MB) 53 / 59.
+  a.stream_stores = (size_t)op.n_fields * op.nqp * sizeof(Number) > ((size_t)32 << 20);
   a.perm = op.perm_dev.as<int32_t>();
   a.error = op.flag.ptr;  // cleared by cache()
   auto cells = [&](int b, int e, int m) {

@@ -27,6 +27,7 @@ struct CacheArgs {
   // and s (what mfg_operator_qp_data exports) field by field in input cell order
   int t2_gradient;
   Number *u_copy;       // 3 per node, with t2_gradient 1
+  int stream_stores;    // with t2_gradient 1: store the fields past the caches
   const int32_t *perm;  // with t2_gradient 2: input index of every stored cell
   int *error;   // set to 1 if det F <= 0 anywhere (not with t2_gradient 2)
 };
@@ -87,15 +88,21 @@ __device__ inline void affine_jacobian(Ptr v, double (&J)[3][3]) {
   }
 }
 
+// Workgroups: where N^3 is no multiple of 8, the fields of neighbouring cells
+// share cache lines, and an XCD takes contiguous cells so that they meet in one
+// L2; otherwise all XCDs walk the fields together.  15M unknowns FP64, contiguous
+// / together: tensor2 words non-affine Q1 2001 / 1810 us, Q4 479 / 538, Q6 460 /
+// 475; formulation 0 Q3 615 / 538; tensor4 (5M) Q4 406 / 447.
 // kAffine: every cell's trilinear map is affine.  Both Jacobians in one kernel
 // take Q1 and Q2 FP64 from 4 waves per SIMD to 3: 1.2M unknowns Q1 non-affine 206
 // against 181 us (178 from the Jacobian of the vertices in point order alone),
-// 1.5M Q2 105 against 95.  Q2 FP64 is 2 registers above 4 waves' share by itself;
-// bounded to it, 3 spill.
+// 1.5M Q2 105 against 95.  Q1 and Q2 FP64 are 2 registers above 4 waves' share;
+// bounded to it, 3 spill (Q2).
 template <int P, int CPB, typename Number, bool kAffine>
-__global__ void __launch_bounds__((block_threads<P, CPB>()), (P == 2 && sizeof(Number) == 8 ? 4 : 1))
+__global__ void __launch_bounds__((block_threads<P, CPB>()), (P <= 2 && sizeof(Number) == 8 ? 4 : 1))
     cache_solid(CacheArgs<Number> a) {
   constexpr int N = P + 1, N3 = N * N * N;
+  constexpr bool kNeighboursShareLines = N3 % 8 != 0;
   __shared__ Number s_shape[N * N], s_colloc[N * N];
   __shared__ Number s_tile[CPB * 6 * N3];
   const int t = threadIdx.x;
@@ -110,7 +117,8 @@ __global__ void __launch_bounds__((block_threads<P, CPB>()), (P == 2 && sizeof(N
   T.j = (pt / N) % N;
   T.k = pt / (N * N);
   T.writer = !pad;
-  const int first_cell = a.cell_begin + xcd_remap(blockIdx.x, gridDim.x) * CPB, cell = first_cell + lc;
+  const int block = kNeighboursShareLines ? xcd_remap(blockIdx.x, gridDim.x) : (int)blockIdx.x;
+  const int first_cell = a.cell_begin + block * CPB, cell = first_cell + lc;
   const bool active = !pad && cell < a.cell_end;
   const int64_t qidx = (int64_t)first_cell * N3 + (active ? t : 0);
   const uint32_t entry = active ? a.cell_nodes[qidx] : 0u;
@@ -200,7 +208,11 @@ __global__ void __launch_bounds__((block_threads<P, CPB>()), (P == 2 && sizeof(N
     typedef Number Pair __attribute__((ext_vector_type(2)));
     Pair *qp = reinterpret_cast<Pair *>(a.qd);
 #pragma unroll
-    for (int k = 0; k < 5; ++k) qp[k * n + qidx] = Pair{f10[2 * k], f10[2 * k + 1]};
+    for (int k = 0; k < 5; ++k) {
+      const Pair x{f10[2 * k], f10[2 * k + 1]};
+      if (a.stream_stores) __builtin_nontemporal_store(x, qp + k * n + qidx);
+      else qp[k * n + qidx] = x;
+    }
     return;
   }
   if (a.caching == MFG_CACHING_SCALAR_REFERENTIAL || a.caching == MFG_CACHING_TENSOR4_NS) {
