@@ -60,9 +60,10 @@ constexpr bool has_solid_columns(bool formulation1) {
 //  - heat on affine cells: equal at about 600 waves (Q4 7.8 -> 9.2 at 172, Q2
 //    8.4 -> 8.4 at 392), 7 to 50 % faster from 1000 (Q4 16.6 -> 14.8 at 1688,
 //    Q6 16.8 -> 15.0 at 1000).  FP64 Q1 to Q3 is bound by its vector traffic
-//    once that leaves the caches: Q2 151 -> 143 at 46,656 cells a launch but
-//    906 -> 943 at 314,432, Q3 108 -> 103 at 13,824 but 583 -> 608 at 91,125;
-//    Q1 gains nothing at any size.
+//    once that leaves the caches, from about 2^19 nodes a colour launch on: Q2
+//    197 -> 185 at 64,000 cells a launch but 906 -> 943 at 314,432, Q3 133 ->
+//    131 at 17,576 but 158 -> 169 at 21,952 and 293 -> 315 at 46,656 (one launch
+//    over as many: 25.9 -> 28.8 and 46.5 -> 50.7); Q1 gains nothing at any size.
 //  - solid Q6 FP64: 175 -> 146 at 614 waves, 881 -> 577 at 3724 (formulation 0
 //    213 -> 176 and 1027 -> 743).
 //  - solid Q5 and Q6 FP32, Q5 FP64, formulation 1: slower at 614 to 1000 waves
@@ -72,7 +73,8 @@ constexpr bool has_solid_columns(bool formulation1) {
 template <int P, typename Number>
 inline bool columns_pay(bool heat, bool formulation1, int n_cells, int waves) {
   constexpr bool fp64 = sizeof(Number) == 8;
-  if (heat) return has_heat_columns<P, Number>() && waves >= 768 && !(fp64 && P <= 3 && n_cells > 65536);
+  if (heat)
+    return has_heat_columns<P, Number>() && waves >= 768 && !(fp64 && P <= 3 && n_cells > (1 << 19) / (P * P * P));
   return has_solid_columns<P, Number>(formulation1) && waves >= (fp64 && P == 6 ? 512 : 1536);
 }
 
