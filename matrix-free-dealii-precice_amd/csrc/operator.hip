@@ -224,12 +224,12 @@ static void launch_cache(OperatorData &op, const void *u, int u_fp32, void *expo
   a.jxw_ref_field = op.affine_ref ? 0 : 1;
   a.t2_gradient = export_gradient ? 2 : op.t2_gradient() ? 1 : 0;
   a.u_copy = a.t2_gradient == 1 ? op.u_copy<Number>() : nullptr;
-  // fields that do not stay in the L2s (8 of 4 MB) leave them to the
+  // 10-word fields that do not stay in the L2s (8 of 4 MB) leave them to the
   // displacement and the map.  Cache, plain / streamed: Q2 3M unknowns 153 / 105
   // us, 15M 676 / 555; Q5 15M 347 / 294 (without the displacement's copy 316);
   // FP32 Q4 15M 203 / 142.  Below, the next application reads them from there:
   // cache and two vmults of 0.1M Q1 unknowns (21 MB) 53 / 59.
-  a.stream_stores = (size_t)op.n_fields * op.nqp * sizeof(Number) > ((size_t)32 << 20);
+  const bool stream = a.t2_gradient == 1 && (size_t)op.n_fields * op.nqp * sizeof(Number) > ((size_t)32 << 20);
   a.perm = op.perm_dev.as<int32_t>();
   a.error = op.flag.ptr;  // cleared by cache()
   auto cells = [&](int b, int e, int m) {
@@ -238,8 +238,10 @@ static void launch_cache(OperatorData &op, const void *u, int u_fp32, void *expo
     a.mu = Number(op.mats[m].mu);
     a.lambda = Number(op.mats[m].lambda);
     const int blocks = blocks_for(e - b, CPB);
-    if (op.affine_ref) cache_solid<P, CPB, Number, true><<<blocks, block_threads<P, CPB>(), 0, op.stream>>>(a);
-    else cache_solid<P, CPB, Number, false><<<blocks, block_threads<P, CPB>(), 0, op.stream>>>(a);
+    constexpr int NT = block_threads<P, CPB>();
+    if (stream) cache_solid<P, CPB, Number, true, true><<<blocks, NT, 0, op.stream>>>(a);
+    else if (op.affine_ref) cache_solid<P, CPB, Number, true><<<blocks, NT, 0, op.stream>>>(a);
+    else cache_solid<P, CPB, Number, false><<<blocks, NT, 0, op.stream>>>(a);
     MFG_HIP(hipGetLastError());
   };
   if (op.has_inclusion()) op.for_each_range([&](int, int b, int e, int m) { cells(b, e, m); });

@@ -27,7 +27,6 @@ struct CacheArgs {
   // and s (what mfg_operator_qp_data exports) field by field in input cell order
   int t2_gradient;
   Number *u_copy;       // 3 per node, with t2_gradient 1
-  int stream_stores;    // with t2_gradient 1: store the fields past the caches
   const int32_t *perm;  // with t2_gradient 2: input index of every stored cell
   int *error;   // set to 1 if det F <= 0 anywhere (not with t2_gradient 2)
 };
@@ -98,7 +97,9 @@ __device__ inline void affine_jacobian(Ptr v, double (&J)[3][3]) {
 // against 181 us (178 from the Jacobian of the vertices in point order alone),
 // 1.5M Q2 105 against 95.  Q1 and Q2 FP64 are 2 registers above 4 waves' share;
 // bounded to it, 3 spill (Q2).
-template <int P, int CPB, typename Number, bool kAffine>
+// kStream: with t2_gradient 1, the fields are stored past the caches (a run-time
+// choice is no use: the compiler merges the two stores into a plain one).
+template <int P, int CPB, typename Number, bool kAffine, bool kStream = false>
 __global__ void __launch_bounds__((block_threads<P, CPB>()), (P <= 2 && sizeof(Number) == 8 ? 4 : 1))
     cache_solid(CacheArgs<Number> a) {
   constexpr int N = P + 1, N3 = N * N * N;
@@ -210,7 +211,7 @@ __global__ void __launch_bounds__((block_threads<P, CPB>()), (P <= 2 && sizeof(N
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       const Pair x{f10[2 * k], f10[2 * k + 1]};
-      if (a.stream_stores) __builtin_nontemporal_store(x, qp + k * n + qidx);
+      if constexpr (kStream) __builtin_nontemporal_store(x, qp + k * n + qidx);
       else qp[k * n + qidx] = x;
     }
     return;
