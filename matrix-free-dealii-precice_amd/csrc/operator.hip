@@ -7,8 +7,6 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
-#include <system_error>
-#include <thread>
 
 #include "column_kernels.hpp"
 #include "common.hpp"
@@ -533,28 +531,11 @@ void OperatorData::colour_cells(const mfg_level_desc &d, int N3) {
   for (int c = 0; c < n_cells; ++c) perm[ids[c] == 0 ? fillp[colour[c]]++ : fill1[colour[c]]++] = c;
 }
 
-// f(first, end) over pieces of the stored cells [b, e) on up to n_threads
-// threads, the caller's among them; returns when all are done.
-template <class F>
-static void split_cells(int b, int e, int n_threads, F f) {
-  const int64_t n = e - b;
-  std::vector<std::thread> others;
-  others.reserve(n_threads);
-  int t = 1;
-  try {
-    for (; t < n_threads; ++t) others.emplace_back(f, b + (int)(n * t / n_threads), b + (int)(n * (t + 1) / n_threads));
-  } catch (const std::system_error &) {  // no more threads: the rest here
-  }
-  f(b, b + (int)(n / n_threads));
-  if (t < n_threads) f(b + (int)(n * t / n_threads), e);
-  for (std::thread &x : others) x.join();
-}
-
-// Cells of one colour share no node, so their points' ranks at their nodes are
-// counted without order between them: a colour's cells on several threads, the
-// colours one after the other (the order of the colour launches, in which the
-// sums add).  5.1M points (32x32x40 Q4 cells) on 8 cores: 33 ms counting and
-// placing point by point on one thread, 17 like this on one, 8 on four.
+// A node's rank per point is counted in the stored (colour-major) order, the
+// order of the colour launches in which the sums add, straight into the array
+// that becomes the places: 32x32x40 Q4 cells (5.1M points) 18 -> 11 ms against a
+// count, a copy of the offsets and a second pass that counts again.  Several
+// threads over the cells of a colour, which share no node, were not faster (12 ms).
 bool OperatorData::build_gather(bool optional) {
   MFG_REQUIRE(nqp < ((int64_t)1 << 31), MFG_ERR_ARGUMENT, "too many quadrature points for the GATHER tables");
   auto drop = [&] {
@@ -567,7 +548,6 @@ bool OperatorData::build_gather(bool optional) {
     return false;
   }
   const int N3 = (p + 1) * (p + 1) * (p + 1);
-  const int n_threads = (int)std::min<int64_t>(4, 1 + nqp / (1 << 19));
   std::vector<int32_t> offsets((size_t)n_nodes + 1, 0);
   std::unique_ptr<uint32_t[]> ranks(new uint32_t[nqp]), index;  // not cleared: every entry is written
   // heat Q1 and Q2: reading through an index is the faster form (1M unknowns
@@ -575,25 +555,20 @@ bool OperatorData::build_gather(bool optional) {
   // against 34)
   gather_indexed = nc == 1 && p <= 2;
   if (gather_indexed) index.reset(new uint32_t[nqp]);
-  for (size_t k = 0; k + 1 < colour_start.size(); ++k)
-    split_cells(colour_start[k], colour_start[k + 1], n_threads, [&](int first, int end) {
-      for (int c = first; c < end; ++c) {
-        const int32_t *node = &host_cell_nodes[(int64_t)perm[c] * N3];
-        uint32_t *r = &ranks[(int64_t)c * N3];
-        for (int pt = 0; pt < N3; ++pt) r[pt] = (uint32_t)offsets[node[pt] + 1]++;
-      }
-    });
+  for (int c = 0; c < n_cells; ++c) {
+    const int32_t *node = &host_cell_nodes[(int64_t)perm[c] * N3];
+    uint32_t *r = &ranks[(int64_t)c * N3];
+    for (int pt = 0; pt < N3; ++pt) r[pt] = (uint32_t)offsets[node[pt] + 1]++;
+  }
   for (int64_t v = 0; v < n_nodes; ++v) offsets[v + 1] += offsets[v];
-  split_cells(0, n_cells, n_threads, [&](int first, int end) {
-    for (int c = first; c < end; ++c) {
-      const int32_t *node = &host_cell_nodes[(int64_t)perm[c] * N3];
-      uint32_t *r = &ranks[(int64_t)c * N3];
-      for (int pt = 0; pt < N3; ++pt) {
-        r[pt] += (uint32_t)offsets[node[pt]];
-        if (index) index[r[pt]] = (uint32_t)c * N3 + pt;
-      }
+  for (int c = 0; c < n_cells; ++c) {
+    const int32_t *node = &host_cell_nodes[(int64_t)perm[c] * N3];
+    uint32_t *r = &ranks[(int64_t)c * N3];
+    for (int pt = 0; pt < N3; ++pt) {
+      r[pt] += (uint32_t)offsets[node[pt]];
+      if (index) index[r[pt]] = (uint32_t)c * N3 + pt;
     }
-  });
+  }
   const uint32_t *places = index ? index.get() : ranks.get();
   try {
     MFG_HIP(hipMemcpyAsync(gather_offsets.ptr, offsets.data(), gather_offsets.bytes, hipMemcpyHostToDevice, stream));
