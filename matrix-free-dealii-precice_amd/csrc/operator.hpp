@@ -21,7 +21,8 @@ constexpr int64_t kGatherMaxPoints = 1 << 20;
 // Q3 1.47 at 0.9M, 1.07 at 2.3M, 0.94 at 4.7M; Q4 1.55 at 0.6M, 1.07 at 3.7M,
 // 0.88 at 8M (FP32 1.00); Q5 1.10 at 3.4M; Q6 1.39 at 3.2M, 1.15 at 6M; heat
 // Q2 0.96 at 3.4M (FP32 1.40), Q3 1.22 at 2.3M, Q4 1.04 at 5.8M, Q6 1.31 at
-// 4.7M.
+// 4.7M.  One limit per degree for both kinds and precisions: about where the
+// first of them stops gaining, and leaves what others would gain above it.
 constexpr int64_t gather_max_points(int p) {
   return p == 1 ? kGatherMaxPoints : p <= 3 ? 3 * kGatherMaxPoints : 5 * kGatherMaxPoints;
 }
