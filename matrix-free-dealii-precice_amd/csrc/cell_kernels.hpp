@@ -277,7 +277,13 @@ constexpr int kSymI[6] = {0, 1, 2, 0, 0, 1}, kSymJ[6] = {0, 1, 2, 1, 2, 2};
 //                 weights (wq).
 // 16 words per point instead of the reference's 18, and no JxW products in
 // the point operation.
-template <typename Number>
+// kStreamLast: field 16 is loaded past the caches.  It stays in the 256 MB MALL
+// from one application to the next where it is a good part smaller; above, it
+// only drives the vectors out.  Non-affine Q1 FP64, streamed / cached: 5M
+// unknowns (a field of 107 MB) 432 / 414 us, 10M (213 MB) 824 / 836, 15M 1269 /
+// 1373; Q4 2M (10 MB) 97 / 89.  A type of its own: with cell_jxw decided at run
+// time the compiler merges the two loads into a plain one.
+template <typename Number, bool kStreamLast = false>
 struct QSolidT2F1 {
   static constexpr int NC = 3;
   static constexpr int kFields = 17;  // 16 with cell_jxw
@@ -293,7 +299,9 @@ struct QSolidT2F1 {
   struct Data {
     Number ji[9], s, T[6], w;  // w: the point's quadrature weight (with cell_jxw) or JxW_ref
   };
-  __device__ Cell load_cell(int cell) const { return Cell{cell_jxw ? as_constant(cell_jxw)[cell] : Number(1)}; }
+  __device__ Cell load_cell(int cell) const {
+    return Cell{!kStreamLast && cell_jxw ? as_constant(cell_jxw)[cell] : Number(1)};
+  }
   __device__ Number jxw(const Cell &cd, const Data &d) const { return cd.jxw * d.w; }
   // fields 0..15 are stored in pairs, qd[((f / 2) nqp + q) 2 + f % 2], field
   // 16 plainly after them: 8 16-byte (FP64) loads bring a point's 16 words
@@ -313,7 +321,8 @@ struct QSolidT2F1 {
     d.s = f16[9];
 #pragma unroll
     for (int f = 0; f < 6; ++f) d.T[f] = f16[10 + f];
-    d.w = cell_jxw ? wq[pt] : stream_load(qd + 16 * nqp + qb + lo);
+    if constexpr (kStreamLast) d.w = stream_load(qd + 16 * nqp + qb + lo);
+    else d.w = cell_jxw ? wq[pt] : qd[16 * nqp + qb + lo];
     return d;
   }
   __device__ Number value_scale(const Cell &cd, const Data &d) const { return rho_alpha * jxw(cd, d); }

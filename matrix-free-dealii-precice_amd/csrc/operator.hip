@@ -72,8 +72,12 @@ static void with_qop(const OperatorData &op, int m, F fn) {
     }
     fn(t2_gradient_op<Number, kEarlyCell>(op, m));
   } else if (op.sp.formulation == 1) {
-    fn(QSolidT2F1<Number>{op.qd.as<Number>(), op.nqp, Number(2.0 * M.lambda), ra, t2_cell_jxw<Number>(op),
-                          op.wq3.as<Number>()});
+    auto words = [&](auto q) {
+      fn(decltype(q){op.qd.as<Number>(), op.nqp, Number(2.0 * M.lambda), ra, t2_cell_jxw<Number>(op),
+                     op.wq3.as<Number>()});
+    };
+    if (!op.affine_ref && op.nqp * (int64_t)sizeof(Number) > ((int64_t)160 << 20)) words(QSolidT2F1<Number, true>());
+    else words(QSolidT2F1<Number>());
   } else {
     fn(QSolidT2F0<Number>{op.qd.as<Number>(), op.nqp, Number(M.kappa), Number(M.c_1), ra});
   }

@@ -670,6 +670,28 @@ def test_column_kernels(cuda, kind, p, precision, n):
     assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
 
 
+def test_streamed_last_field(cuda):
+    """Non-affine solids whose 17th point field exceeds 160 MB load it past the
+    caches: bitwise the batch's colour launches, which do not."""
+    n, p = (93, 94, 93), 2
+    print(f"streamed last field n={n} p={p}", flush=True)
+    assert n[0] * n[1] * n[2] * (p + 1) ** 3 * 8 > 160 * 2 ** 20
+    base = mfgpu.BoxMesh([0, 0, 0], [1.0, 0.6, 0.4], list(n), p, 3, 1, 7)
+    go = mfgpu.NeoHookOperator(DistortedMesh(base, distort(base.cell_vertices())), O.MU, O.NU, O.RHO, O.ALPHA1)
+    assert go.n_fields() == 17
+    go.cache(dev(base.u0(amp=1e-3, noise=1e-6)))
+    x, y0 = (mfgpu.fill_uniform(k, torch.empty(base.n_dofs, dtype=torch.float64, device="cuda")) for k in (5, 6))
+    ref, ref_add, y, z = torch.full_like(x, float("nan")), y0.clone(), torch.full_like(x, float("nan")), y0.clone()
+    b = mfgpu.Batch([go])
+    b.set_schedule(mfgpu.SCHEDULE_COLOUR)
+    b.vmult([ref], [x])
+    b.vmult_add([ref_add], [x])
+    b.synchronize()
+    go.vmult(y, x)
+    go.vmult_add(z, x)
+    assert torch.isfinite(ref).all() and torch.equal(y, ref) and torch.equal(z, ref_add)
+
+
 # (kind, degree, precision, cells): every colour has enough cells for the column
 # kernels (768 waves of 64 // (p+1)^2 heat cells, 512 solid cells of FP64 Q6, 1536
 # of the others); in some colours the last wave is partly filled
